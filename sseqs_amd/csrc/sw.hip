@@ -505,26 +505,29 @@ template <bool AFFINE, class Src>
 static int launch_sw(const Src& src, const uint8_t* q, int Lq, int64_t n, int p1, int p2,
                      int32_t* out, hipStream_t stream) {
     const Blosum bl = blosum62();
-    if constexpr (std::is_same<Src, SrcPacked>::value) {
-        if (sw16_ok(Lq, AFFINE, p1, p2)) {
-            const int64_t quads = ceil_div(n, 4 * SW16_WAVES);
-            const unsigned grid16 = (unsigned)(quads < 8192 ? quads : 8192);
-            switch ((Lq + 31) >> 5) {
+    // Both sources take the packed kernel wherever it is exact (sw16_ok): VALU
+    // issue bounds both kernels, and it advances two cells per instruction.
+    // ASCII targets, affine, 40 000 of mean length 284 at 350 residues: 636 us
+    // (6.3 T cells/s) against 1183 us on k_sw; 32 targets at 120 residues, a
+    // latency chain of rows: 129 against 154 us for the whole call.
+    if (sw16_ok(Lq, AFFINE, p1, p2)) {
+        const int64_t quads = ceil_div(n, 4 * SW16_WAVES);
+        const unsigned grid16 = (unsigned)(quads < 8192 ? quads : 8192);
+        switch ((Lq + 31) >> 5) {
 #define SW16_CASE(T)                                                                            \
     case T:                                                                                     \
         hipLaunchKernelGGL((k_sw16<T, AFFINE, Src>), dim3(grid16), dim3(64 * SW16_WAVES), 0,   \
                            stream, src, q, Lq, n, p1, p2, out, bl);                             \
         break;
-                SW16_CASE(1) SW16_CASE(2) SW16_CASE(3) SW16_CASE(4) SW16_CASE(5) SW16_CASE(6)
-                SW16_CASE(7) SW16_CASE(8) SW16_CASE(9) SW16_CASE(10) SW16_CASE(11) SW16_CASE(12)
-                SW16_CASE(13) SW16_CASE(14) SW16_CASE(15) SW16_CASE(16) SW16_CASE(17)
-                SW16_CASE(18) SW16_CASE(19) SW16_CASE(20) SW16_CASE(21) SW16_CASE(22)
-                SW16_CASE(23) SW16_CASE(24) SW16_CASE(25) SW16_CASE(26) SW16_CASE(27)
-                SW16_CASE(28) SW16_CASE(29) SW16_CASE(30) SW16_CASE(31) SW16_CASE(32)
+            SW16_CASE(1) SW16_CASE(2) SW16_CASE(3) SW16_CASE(4) SW16_CASE(5) SW16_CASE(6)
+            SW16_CASE(7) SW16_CASE(8) SW16_CASE(9) SW16_CASE(10) SW16_CASE(11) SW16_CASE(12)
+            SW16_CASE(13) SW16_CASE(14) SW16_CASE(15) SW16_CASE(16) SW16_CASE(17)
+            SW16_CASE(18) SW16_CASE(19) SW16_CASE(20) SW16_CASE(21) SW16_CASE(22)
+            SW16_CASE(23) SW16_CASE(24) SW16_CASE(25) SW16_CASE(26) SW16_CASE(27)
+            SW16_CASE(28) SW16_CASE(29) SW16_CASE(30) SW16_CASE(31) SW16_CASE(32)
 #undef SW16_CASE
-            }
-            return check_launch(AFFINE ? "sw affine" : "sw linear");
         }
+        return check_launch(AFFINE ? "sw affine" : "sw linear");
     }
     int64_t pairs = ceil_div(n, 2);
     unsigned grid = (unsigned)(pairs < 16384 ? pairs : 16384);
