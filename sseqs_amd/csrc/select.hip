@@ -20,8 +20,13 @@ constexpr int SEL_BINS = 2048;
 constexpr int SEL_TILE = 16384;     // elements per block in count/write passes
 constexpr int SEL_SORT_MAX = 16384;
 
+// prefix / mask / k_rem: the digits of the k-th largest key fixed so far, as
+// an offset from the base key (0, or P in a sampled select), and how many of
+// the keys that share them are taken.  P, ncand, maxkey: see "sampled
+// select" below (P = 0 when every score is a candidate).
 struct SelState {
-    uint32_t prefix, mask, k_rem, pad;
+    uint32_t prefix, mask, k_rem, k;
+    uint32_t P, ncand, maxkey, pad;
 };
 
 __device__ inline uint32_t key_f32(float x) {
@@ -42,19 +47,311 @@ __device__ inline uint32_t load_key(const void* s, int64_t i) {
 
 __global__ void k_sel_init(uint32_t* hist, SelState* st, uint32_t k) {
     for (int i = threadIdx.x; i < SEL_BINS; i += blockDim.x) hist[i] = 0;
-    if (threadIdx.x == 0) {
-        st->prefix = 0;
-        st->mask = 0;
-        st->k_rem = k;
-        st->pad = 0;
+    if (threadIdx.x == 0) *st = SelState{0u, 0u, k, k, 0u, 0u, 0u, 0u};
+}
+
+// ---- sampled select -------------------------------------------------------
+//
+// Selecting few of many scores needs the digits of only the largest keys.  A
+// strided sample gives a key P that about k + 6 sigma + 8 sample steps of the
+// scores reach; one pass over the scores (k_sel_filter) marks every key >= P
+// in a bitmap, counts them and takes the largest key; the digit, count and
+// write passes then read the bitmap and the few marked scores.  One read of
+// the scores instead of five (three digit passes, count, write): 200 M fp32
+// scores, top 100 000.
+//
+// P is only a guess.  If fewer than k keys reach it, or the sample says that
+// more than an eighth of them do (ties), the select is done over all scores
+// as without a sample: every pass decides that on the device from the state,
+// so nothing is read back and the launches can be captured.
+//
+// Bitmap: tile t of SEL_TILE scores is 64 groups of 256; group g of it has
+// four 64-bit words at 32 (64 t + g) bytes, word e, bit l: score 4 l + e of
+// the group.  A wave reads a group with one load of four scores per lane, and
+// its four ballots are the words; the later passes give a lane a group.
+constexpr int SEL_GROUP = 256;
+constexpr int SEL_TILE_BITS = SEL_TILE / 8;  // bitmap bytes of a tile
+constexpr int SEL_SAMPLE = 32768;            // sampled scores: 8 x 4 per thread of 1024
+// blocks of a digit pass over the marked scores: each adds its non-zero bins
+// to the histogram with device atomics, which cost more than the marked
+// scores' reads (200 M scores, 290 k marked: 4096 blocks 42 us, 1024 26 us,
+// 256 50 us)
+constexpr int SEL_MARK_BLOCKS = 1024;
+
+// Whether the passes run over all scores.
+__device__ inline bool sel_full(const SelState* st) {
+    return st->P == 0u || st->ncand < st->k;
+}
+// Key that digits count from.
+__device__ inline uint32_t sel_base(const SelState* st) { return sel_full(st) ? 0u : st->P; }
+
+// Digit of pass p: up to 11 bits below those of the earlier passes, from the
+// top of the largest key's offset from the base (bits = 0: nothing is left).
+template <int DT>
+__device__ inline void sel_digit(const SelState* st, int p, int* shift, int* bits) {
+    constexpr int LB = DT == SSEQS_F16 ? 13 : 0;  // constant low bits of a key
+    int nb = 32 - LB;
+    if (!sel_full(st)) {
+        const uint32_t d = (st->maxkey - st->P) >> LB;
+        nb = d ? 32 - __clz(d) : 1;
     }
+    const int rem = nb - 11 * p;
+    *bits = rem > 11 ? 11 : (rem > 0 ? rem : 0);
+    *shift = LB + (rem > 0 ? rem - *bits : 0);
+}
+
+// Four consecutive scores from i, as loaded (i a multiple of 4, the scores
+// at an address aligned to four of them).
+template <int DT>
+struct Load4 {
+    uint4 v;
+};
+template <>
+struct Load4<SSEQS_F16> {
+    uint2 v;
+};
+template <int DT>
+__device__ inline Load4<DT> load4(const void* s, int64_t i) {
+    Load4<DT> r;
+    if constexpr (DT == SSEQS_F16)
+        r.v = *reinterpret_cast<const uint2*>(static_cast<const _Float16*>(s) + i);
+    else
+        r.v = *reinterpret_cast<const uint4*>(static_cast<const uint32_t*>(s) + i);
+    return r;
+}
+// Key of score e of the four.
+template <int DT>
+__device__ inline uint32_t key4(const Load4<DT>& r, int e) {
+    if constexpr (DT == SSEQS_F16) {
+        const uint32_t w = e < 2 ? r.v.x : r.v.y;
+        const _Float16 h =
+            __builtin_bit_cast(_Float16, (uint16_t)((e & 1) ? w >> 16 : w & 0xffffu));
+        return key_f32((float)h) & ~0x1FFFu;
+    } else {
+        const uint32_t w = e == 0 ? r.v.x : e == 1 ? r.v.y : e == 2 ? r.v.z : r.v.w;
+        if constexpr (DT == SSEQS_F32) return key_f32(__uint_as_float(w));
+        return w ^ 0x80000000u;
+    }
+}
+
+// One block: clears the state and takes the sample's rank-th largest key as
+// P.  n >= 4 SEL_SAMPLE, so the sampled quadruples are distinct.
+template <int DT>
+__global__ __launch_bounds__(1024) void k_sel_sample(const void* s, int64_t n, uint32_t* hist,
+                                                     SelState* st, uint32_t k, int rank) {
+    constexpr int PER = SEL_SAMPLE / 4096;
+    __shared__ uint32_t lh[SEL_BINS];
+    __shared__ uint32_t wsum[16], wmax[16];
+    __shared__ uint32_t pick[2];
+    const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+    for (int i = t; i < SEL_BINS; i += 1024) hist[i] = 0;
+    uint32_t key[PER * 4];
+    const int64_t step = n / (SEL_SAMPLE / 4);  // scores per sampled quadruple, >= 16
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int q = j * 1024 + t;
+        // a different place in every step, so that no period of the scores is followed
+        const int64_t at = (int64_t)q * step + (int64_t)((uint32_t)q * 2654435761u % (uint32_t)min(step - 7, (int64_t)1 << 30));
+        const Load4<DT> v = load4<DT>(s, at & ~(int64_t)3);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) key[4 * j + e] = key4<DT>(v, e);
+    }
+    // digits from the top of the sample's key range: two of 11 bits resolve it
+    // to 2^-22, which is enough for a guess, and spread its keys over the bins
+    uint32_t lo = key[0], hi = key[0];
+#pragma unroll
+    for (int j = 1; j < PER * 4; ++j) {
+        lo = min(lo, key[j]);
+        hi = max(hi, key[j]);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
+    }
+    if (lane == 0) {
+        wsum[wid] = lo;
+        wmax[wid] = hi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        lo = min(lo, wsum[w]);
+        hi = max(hi, wmax[w]);
+    }
+    const int nb = hi > lo ? 32 - __clz(hi - lo) : 1;
+    uint32_t prefix = 0, mask = 0, need = (uint32_t)rank, got = 0;
+    int shift = 0;
+    for (int p = 0; p < 2; ++p) {
+        const int rem = nb - 11 * p;
+        if (rem <= 0) break;
+        const int bits = min(rem, 11);
+        shift = rem - bits;
+        __syncthreads();  // wsum of the step before is read
+        for (int i = t; i < SEL_BINS; i += 1024) lh[i] = 0;
+        __syncthreads();
+        const uint32_t bm = (1u << bits) - 1u;
+        // one LDS atomic per run of equal bins (neighbouring scores often tie)
+        uint32_t run_bin = 0, run = 0;
+#pragma unroll
+        for (int j = 0; j < PER * 4; ++j) {
+            const uint32_t d = key[j] - lo;
+            if ((d & mask) != prefix) continue;
+            const uint32_t b = (d >> shift) & bm;
+            if (run && b == run_bin) {
+                ++run;
+            } else {
+                if (run) atomicAdd(&lh[run_bin], run);
+                run_bin = b;
+                run = 1;
+            }
+        }
+        if (run) atomicAdd(&lh[run_bin], run);
+        __syncthreads();
+        // thread t holds bins 2047 - 2t and 2046 - 2t: a scan from the top
+        const uint32_t c_hi = lh[SEL_BINS - 1 - 2 * t], c_lo = lh[SEL_BINS - 2 - 2 * t];
+        const uint32_t c = c_hi + c_lo;
+        uint32_t inc = c;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += v;
+        }
+        if (lane == 63) wsum[wid] = inc;
+        __syncthreads();
+        uint32_t above = inc - c;
+        for (int w = 0; w < wid; ++w) above += wsum[w];
+        if (above < need && need <= above + c) {
+            const bool h = need <= above + c_hi;
+            pick[0] = (uint32_t)(SEL_BINS - 1 - 2 * t - (h ? 0 : 1));
+            pick[1] = above + (h ? 0u : c_hi);
+        }
+        __syncthreads();
+        prefix |= pick[0] << shift;
+        mask |= bm << shift;
+        got += pick[1];
+        need -= pick[1];
+    }
+    // sample keys >= P: the ones in the bins above, and those in its last bin
+    const uint32_t P = lo + prefix;
+    __syncthreads();
+    if (t == 0) {
+        const uint32_t last = lh[(prefix >> shift) & (SEL_BINS - 1)];
+        *st = SelState{0u, 0u, k, k, got + last <= SEL_SAMPLE / 8 ? P : 0u, 0u, 0u, 0u};
+    }
+}
+
+// The pass over the scores: bitmap of the keys >= P, their count and the
+// largest key.  A wave takes a tile in steps of eight groups (eight loads of
+// four scores per lane in flight) and stores a step's 32 words together.
+template <int DT>
+__global__ __launch_bounds__(256) void k_sel_filter(const void* s, int64_t n, int64_t nb,
+                                                    SelState* st, uint32_t* bitmap) {
+    const uint32_t P = st->P;
+    if (P == 0u) return;
+    __shared__ uint32_t s_cnt[4], s_max[4];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    uint32_t cnt = 0, mx = 0;
+    for (int64_t tile = (int64_t)blockIdx.x * 4 + wid; tile < nb; tile += (int64_t)gridDim.x * 4) {
+        const int64_t base = tile * SEL_TILE;
+        for (int g0 = 0; g0 < SEL_TILE / SEL_GROUP; g0 += 8) {
+            const int64_t i0 = base + (int64_t)g0 * SEL_GROUP + 4 * lane;
+            uint64_t word = 0;  // lane 4 u + e: word e of group g0 + u
+            if (base + (int64_t)(g0 + 8) * SEL_GROUP <= n) {
+                Load4<DT> v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = load4<DT>(s, i0 + u * SEL_GROUP);
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint32_t key = key4<DT>(v[u], e);
+                        mx = max(mx, key);
+                        const uint64_t m = __ballot(key >= P);
+                        cnt += (uint32_t)__popcll(m);
+                        word = lane == 4 * u + e ? m : word;
+                    }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int64_t i = i0 + u * SEL_GROUP + e;
+                        const uint32_t key = i < n ? load_key<DT>(s, i) : 0u;
+                        mx = max(mx, key);
+                        const uint64_t m = __ballot(key >= P);
+                        cnt += (uint32_t)__popcll(m);
+                        word = lane == 4 * u + e ? m : word;
+                    }
+            }
+            if (lane < 32)
+                reinterpret_cast<uint64_t*>(bitmap)[tile * (SEL_TILE_BITS / 8) + g0 * 4 + lane] = word;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, 64));
+    if (lane == 0) {
+        s_cnt[wid] = cnt;
+        s_max[wid] = mx;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t c = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+        const uint32_t m = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+        if (c) atomicAdd(&st->ncand, c);
+        atomicMax(&st->maxkey, m);
+    }
+}
+
+// A lane's group of a tile: f(index, key) for its marked scores in index order.
+template <int DT, class F>
+__device__ inline void sel_group(const void* s, const uint32_t* bitmap, int64_t tile, int lane,
+                                 F f) {
+    const uint4* b = reinterpret_cast<const uint4*>(bitmap) + tile * (SEL_TILE_BITS / 16) + 2 * lane;
+    const uint4 lo = b[0], hi = b[1];
+    const uint64_t w[4] = {((uint64_t)lo.y << 32) | lo.x, ((uint64_t)lo.w << 32) | lo.z,
+                           ((uint64_t)hi.y << 32) | hi.x, ((uint64_t)hi.w << 32) | hi.z};
+    const int64_t base = tile * SEL_TILE + lane * SEL_GROUP;
+    for (uint64_t any = w[0] | w[1] | w[2] | w[3]; any; any &= any - 1) {
+        const int l = __ffsll((unsigned long long)any) - 1;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if ((w[e] >> l) & 1ull) f(base + 4 * l + e, load_key<DT>(s, base + 4 * l + e));
+    }
+}
+
+// The digit pass over the marked scores (a wave per tile); false when the
+// pass runs over all of them.
+template <int DT>
+__device__ inline bool sel_marked_hist(const void* s, int64_t n, const SelState* st,
+                                       uint32_t* hist, int pass, const uint32_t* bitmap,
+                                       uint32_t* lh) {
+    if (sel_full(st)) return false;
+    int shift, bits;
+    sel_digit<DT>(st, pass, &shift, &bits);
+    const int64_t nb = (n + SEL_TILE - 1) / SEL_TILE;
+    const int nblk = min((int)gridDim.x, SEL_MARK_BLOCKS);
+    if (bits == 0 || (int)blockIdx.x >= nblk) return true;  // uniform over the block
+    for (int i = threadIdx.x; i < SEL_BINS; i += 256) lh[i] = 0;
+    __syncthreads();
+    const uint32_t prefix = st->prefix, mask = st->mask, bm = (1u << bits) - 1u, P = st->P;
+    for (int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); tile < nb;
+         tile += (int64_t)nblk * 4)
+        sel_group<DT>(s, bitmap, tile, threadIdx.x & 63, [&](int64_t, uint32_t key) {
+            const uint32_t d = key - P;
+            if ((d & mask) == prefix) atomicAdd(&lh[(d >> shift) & bm], 1u);
+        });
+    __syncthreads();
+    for (int i = threadIdx.x; i < SEL_BINS; i += 256)
+        if (lh[i]) atomicAdd(&hist[i], lh[i]);
+    return true;
 }
 
 template <int DT>
 __global__ __launch_bounds__(256) void k_sel_hist(const void* s, int64_t n,
-                                                  const SelState* st, uint32_t* hist, int shift,
-                                                  int bits) {
+                                                  const SelState* st, uint32_t* hist, int pass,
+                                                  const uint32_t* bitmap) {
     __shared__ uint32_t lh[SEL_BINS];
+    if (sel_marked_hist<DT>(s, n, st, hist, pass, bitmap, lh)) return;
+    int shift, bits;
+    sel_digit<DT>(st, pass, &shift, &bits);
     for (int i = threadIdx.x; i < SEL_BINS; i += 256) lh[i] = 0;
     __syncthreads();
     const uint32_t prefix = st->prefix, mask = st->mask, bm = (1u << bits) - 1u;
@@ -63,10 +360,22 @@ __global__ __launch_bounds__(256) void k_sel_hist(const void* s, int64_t n,
         uint32_t key[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) key[e] = load_key<DT>(s, min(i0 + e * 256 + threadIdx.x, n - 1));
+        // one LDS atomic per run of equal bins: tied scores and constant top
+        // digits (int32 scores) would otherwise queue at one address
+        uint32_t run_bin = 0, run = 0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (i0 + e * 256 + threadIdx.x < n && (key[e] & mask) == prefix)
-                atomicAdd(&lh[(key[e] >> shift) & bm], 1u);
+        for (int e = 0; e < 4; ++e) {
+            if (i0 + e * 256 + threadIdx.x >= n || (key[e] & mask) != prefix) continue;
+            const uint32_t b = (key[e] >> shift) & bm;
+            if (run && b == run_bin) {
+                ++run;
+            } else {
+                if (run) atomicAdd(&lh[run_bin], run);
+                run_bin = b;
+                run = 1;
+            }
+        }
+        if (run) atomicAdd(&lh[run_bin], run);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < SEL_BINS; i += 256)
@@ -77,11 +386,14 @@ __global__ __launch_bounds__(256) void k_sel_hist(const void* s, int64_t n,
 // (from the top) where the keys above it fall short of k_rem and the keys
 // above plus those in it do not; the counts above every bin come from one
 // block-wide scan of the bins in descending order.
-__global__ __launch_bounds__(1024) void k_sel_pick(SelState* st, uint32_t* hist, int shift,
-                                                   int bits) {
+template <int DT>
+__global__ __launch_bounds__(1024) void k_sel_pick(SelState* st, uint32_t* hist, int pass) {
     __shared__ uint32_t wsum[16];
     __shared__ int pick_b;
     __shared__ uint32_t pick_above, cnt0;
+    int shift, bits;
+    sel_digit<DT>(st, pass, &shift, &bits);
+    if (bits == 0) return;
     const int nb = 1 << bits;
     const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
     // thread t holds bins hi = nb-1-2t and lo = hi-1, so ascending t walks
@@ -127,11 +439,71 @@ __global__ __launch_bounds__(1024) void k_sel_pick(SelState* st, uint32_t* hist,
     }
 }
 
+// Counts of keys > T and == T per tile from the marked scores (a wave per
+// tile); false when the pass runs over all scores.
+template <int DT>
+__device__ inline bool sel_marked_count(const void* s, int64_t nb, const SelState* st, uint32_t T,
+                                        int64_t* cgt, int64_t* ceq, const uint32_t* bitmap) {
+    if (sel_full(st)) return false;
+    const int lane = threadIdx.x & 63;
+    for (int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); tile < nb;
+         tile += (int64_t)gridDim.x * 4) {
+        int gt = 0, eq = 0;
+        sel_group<DT>(s, bitmap, tile, lane, [&](int64_t, uint32_t key) {
+            gt += key > T;
+            eq += key == T;
+        });
+        for (int o = 32; o > 0; o >>= 1) {
+            gt += __shfl_xor(gt, o, 64);
+            eq += __shfl_xor(eq, o, 64);
+        }
+        if (lane == 0) {
+            cgt[tile] = gt;
+            ceq[tile] = eq;
+        }
+    }
+    return true;
+}
+
+// The write pass over the marked scores (a wave per tile, its lanes' groups
+// in index order); false when the pass runs over all scores.
+template <int DT>
+__device__ inline bool sel_marked_write(const void* s, int64_t nb, const SelState* st, uint32_t T,
+                                        const int64_t* bgt, const int64_t* beq, int64_t k,
+                                        int64_t* out, const uint32_t* bitmap) {
+    if (sel_full(st)) return false;
+    const int64_t keq = st->k_rem;
+    const int lane = threadIdx.x & 63;
+    for (int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); tile < nb;
+         tile += (int64_t)gridDim.x * 4) {
+        uint32_t c = 0;  // the group's (count > T) << 16 | (count == T), each <= 256
+        sel_group<DT>(s, bitmap, tile, lane, [&](int64_t, uint32_t key) {
+            c += (key > T ? 0x10000u : 0u) + (key == T ? 1u : 0u);
+        });
+        uint32_t inc = c;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += v;
+        }
+        if (c == 0) continue;  // no barrier below
+        int64_t gb = bgt[tile] + ((inc - c) >> 16), eb = beq[tile] + ((inc - c) & 0xffffu);
+        sel_group<DT>(s, bitmap, tile, lane, [&](int64_t i, uint32_t key) {
+            const bool g = key > T, q = key == T;
+            const int64_t slot = gb + min(eb, keq);
+            if ((g || (q && eb < keq)) && slot < k) out[slot] = i;
+            gb += g;
+            eb += q;
+        });
+    }
+    return true;
+}
+
 template <int DT>
 __global__ __launch_bounds__(256) void k_sel_count(const void* s, int64_t n,
                                                    int64_t nb, const SelState* st, int64_t* cgt,
-                                                   int64_t* ceq) {
-    const uint32_t T = st->prefix;
+                                                   int64_t* ceq, const uint32_t* bitmap) {
+    const uint32_t T = sel_base(st) + st->prefix;
+    if (sel_marked_count<DT>(s, nb, st, T, cgt, ceq, bitmap)) return;
     __shared__ int rg[256], re[256];
     for (int64_t tile = blockIdx.x; tile < nb; tile += gridDim.x) {
     const int64_t base = tile * SEL_TILE;
@@ -163,34 +535,77 @@ __global__ __launch_bounds__(256) void k_sel_count(const void* s, int64_t n,
     }
 }
 
-// Exclusive scan of two arrays of nb counts, one block.
+// Exclusive scan of two arrays of nb counts (each at most SEL_TILE), one
+// block.  Wave w holds SCAN_ROWS rows of 64 consecutive counts of each array
+// in registers per round, so every load is coalesced and all are in flight;
+// a row is scanned across the lanes in 32 bits.  (Twelve consecutive counts
+// per thread, 12 207 in all, take 35 us.)
+constexpr int SCAN_ROWS = 8;
+
+// Inclusive sum over the lanes of a wave: shifts by 1, 2, 4, 8 within the
+// rows of 16, then the rows' totals (lane 15 of each row to the next row,
+// lane 31 to the upper half).
+template <int CTRL, int ROWS>
+__device__ inline int scan_dpp(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+__device__ inline int wave_scan_i32(int v) {
+    v += scan_dpp<0x111, 0xf>(v);
+    v += scan_dpp<0x112, 0xf>(v);
+    v += scan_dpp<0x114, 0xf>(v);
+    v += scan_dpp<0x118, 0xf>(v);
+    v += scan_dpp<0x142, 0xa>(v);
+    v += scan_dpp<0x143, 0xc>(v);
+    return v;
+}
+
 __global__ __launch_bounds__(1024) void k_sel_scan(int64_t* a, int64_t* b, int64_t nb) {
-    __shared__ int64_t pa[1024], pb[1024];
-    int64_t per = (nb + 1023) / 1024;
-    int64_t lo = threadIdx.x * per, hi = min(nb, lo + per);
-    int64_t sa = 0, sb = 0;
-    for (int64_t i = lo; i < hi; ++i) {
-        sa += a[i];
-        sb += b[i];
-    }
-    pa[threadIdx.x] = sa;
-    pb[threadIdx.x] = sb;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        int64_t ta = threadIdx.x >= off ? pa[threadIdx.x - off] : 0;
-        int64_t tb = threadIdx.x >= off ? pb[threadIdx.x - off] : 0;
+    __shared__ int wa[16], wb[16];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    int64_t ra = 0, rb = 0;  // totals of the rounds before
+    for (int64_t r0 = 0; r0 < nb; r0 += 1024 * SCAN_ROWS) {
+        // rows per wave of this round (a short round is spread over the waves)
+        const int rows = (int)min((int64_t)SCAN_ROWS, (nb - r0 + 1023) / 1024);
+        const int64_t w0 = r0 + (int64_t)wid * rows * 64 + lane;
+        int va[SCAN_ROWS], vb[SCAN_ROWS];
+#pragma unroll
+        for (int i = 0; i < SCAN_ROWS; ++i) {  // clamped, so unconditional
+            const int64_t at = min(w0 + 64 * min(i, rows - 1), nb - 1);
+            va[i] = (int)a[at];
+            vb[i] = (int)b[at];
+        }
+        int ta = 0, tb = 0;  // totals of the wave's rows: at most 64 SCAN_ROWS SEL_TILE
+        int ea[SCAN_ROWS], eb[SCAN_ROWS];
+#pragma unroll
+        for (int i = 0; i < SCAN_ROWS; ++i) {
+            const bool in = i < rows && w0 + 64 * i < nb;
+            const int ca = in ? va[i] : 0, cb = in ? vb[i] : 0;
+            const int ia = wave_scan_i32(ca), ib = wave_scan_i32(cb);
+            ea[i] = ta + ia - ca;
+            eb[i] = tb + ib - cb;
+            ta += __builtin_amdgcn_readlane(ia, 63);
+            tb += __builtin_amdgcn_readlane(ib, 63);
+        }
+        if (lane == 0) {
+            wa[wid] = ta;
+            wb[wid] = tb;
+        }
         __syncthreads();
-        pa[threadIdx.x] += ta;
-        pb[threadIdx.x] += tb;
+        int64_t ba = ra, bb = rb;
+        for (int w = 0; w < 16; ++w) {
+            const int xa = wa[w], xb = wb[w];
+            ba += w < wid ? xa : 0;
+            bb += w < wid ? xb : 0;
+            ra += xa;
+            rb += xb;
+        }
+#pragma unroll
+        for (int i = 0; i < SCAN_ROWS; ++i)
+            if (i < rows && w0 + 64 * i < nb) {
+                a[w0 + 64 * i] = ba + ea[i];
+                b[w0 + 64 * i] = bb + eb[i];
+            }
         __syncthreads();
-    }
-    int64_t ra = pa[threadIdx.x] - sa, rb = pb[threadIdx.x] - sb;
-    for (int64_t i = lo; i < hi; ++i) {
-        int64_t xa = a[i], xb = b[i];
-        a[i] = ra;
-        b[i] = rb;
-        ra += xa;
-        rb += xb;
     }
 }
 
@@ -198,8 +613,10 @@ template <int DT>
 __global__ __launch_bounds__(256) void k_sel_write(const void* s, int64_t n,
                                                    int64_t nb, const SelState* st,
                                                    const int64_t* bgt, const int64_t* beq,
-                                                   int64_t k, int64_t* out) {
-    const uint32_t T = st->prefix;
+                                                   int64_t k, int64_t* out,
+                                                   const uint32_t* bitmap) {
+    const uint32_t T = sel_base(st) + st->prefix;
+    if (sel_marked_write<DT>(s, nb, st, T, bgt, beq, k, out, bitmap)) return;
     const int64_t keq = st->k_rem;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
@@ -279,9 +696,12 @@ __device__ inline uint32_t keys8_f16(const _Float16* s, int64_t i, int64_t n, ui
 }
 
 __global__ __launch_bounds__(256) void k_sel_hist_h8(const _Float16* __restrict__ s, int64_t n,
-                                                     const SelState* st, uint32_t* hist, int shift,
-                                                     int bits) {
+                                                     const SelState* st, uint32_t* hist, int pass,
+                                                     const uint32_t* bitmap) {
     __shared__ uint32_t lh[SEL_BINS];
+    if (sel_marked_hist<SSEQS_F16>(s, n, st, hist, pass, bitmap, lh)) return;
+    int shift, bits;
+    sel_digit<SSEQS_F16>(st, pass, &shift, &bits);
     for (int i = threadIdx.x; i < SEL_BINS; i += 256) lh[i] = 0;
     __syncthreads();
     const uint32_t prefix = st->prefix, mask = st->mask, bm = (1u << bits) - 1u;
@@ -312,8 +732,10 @@ __global__ __launch_bounds__(256) void k_sel_hist_h8(const _Float16* __restrict_
 
 __global__ __launch_bounds__(256) void k_sel_count_h8(const _Float16* __restrict__ s, int64_t n,
                                                       int64_t nb, const SelState* st,
-                                                      int64_t* cgt, int64_t* ceq) {
-    const uint32_t T = st->prefix;
+                                                      int64_t* cgt, int64_t* ceq,
+                                                      const uint32_t* bitmap) {
+    const uint32_t T = sel_base(st) + st->prefix;
+    if (sel_marked_count<SSEQS_F16>(s, nb, st, T, cgt, ceq, bitmap)) return;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     __shared__ int rg[4], re[4];
     for (int64_t tile = blockIdx.x; tile < nb; tile += gridDim.x) {
@@ -350,8 +772,10 @@ __global__ __launch_bounds__(256) void k_sel_count_h8(const _Float16* __restrict
 __global__ __launch_bounds__(256) void k_sel_write_h8(const _Float16* __restrict__ s, int64_t n,
                                                       int64_t nb, const SelState* st,
                                                       const int64_t* bgt, const int64_t* beq,
-                                                      int64_t k, int64_t* out) {
-    const uint32_t T = st->prefix;
+                                                      int64_t k, int64_t* out,
+                                                      const uint32_t* bitmap) {
+    const uint32_t T = sel_base(st) + st->prefix;
+    if (sel_marked_write<SSEQS_F16>(s, nb, st, T, bgt, beq, k, out, bitmap)) return;
     const int64_t keq = st->k_rem;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     // wave totals of a step, (count > T) << 16 | (count == T), by step parity:
@@ -644,21 +1068,34 @@ using namespace sseqs;
             hipLaunchKernelGGL(KERNEL<SSEQS_I32>, __VA_ARGS__);                   \
     } while (0)
 
-extern "C" size_t sseqs_topk_ws_bytes(int64_t n) {
+// Sampled select: few of many scores, at an address that four of them are
+// aligned to.  Top 100 000, sampled against all passes over the scores (us):
+// fp32 200 M 298 / 1153, 20 M 115 / 233, 8 M 102 / 137; fp16 200 M 209 / 489,
+// 8 M 89 / 109; int32 200 M 274 / 1956.  The marked scores' passes grow with
+// k: at 8 M and k = n / 64 they still win (107 / 137), at 4 M and n / 32 they
+// do not (128 / 96).
+constexpr int64_t SEL_SAMPLE_MIN_N = 1 << 22;
+constexpr int64_t SEL_SAMPLE_MIN_RATIO = 64;
+static bool sel_sampled(const void* scores, int dtype, int64_t n, int64_t k) {
+    const uintptr_t al = dtype == SSEQS_F16 ? 8 : 16;
+    return n >= SEL_SAMPLE_MIN_N && k <= n / SEL_SAMPLE_MIN_RATIO && n <= 0xffffffffLL &&
+           (reinterpret_cast<uintptr_t>(scores) & (al - 1)) == 0;
+}
+
+static size_t sel_ws_base(int64_t n) {
     int64_t nb = ceil_div(n > 0 ? n : 1, SEL_TILE);
     return (size_t)SEL_BINS * 4 + 64 + (size_t)nb * 16 + (size_t)SEL_SORT_MAX * 8 + 256;
 }
 
-extern "C" int sseqs_topk(const void* scores, int dtype, int64_t n, int64_t k, int sorted,
-                          int64_t* out_idx, void* ws, size_t ws_bytes, hipStream_t stream) {
-    if (n < 0 || k < 0) return fail(-1, "topk: negative size");
-    if (k > n) return fail(-1, "topk: k larger than the number of scores");
-    if (dtype != SSEQS_F32 && dtype != SSEQS_F16 && dtype != SSEQS_I32)
-        return fail(-1, "topk: unsupported dtype");
-    if (k == 0) return 0;
-    if (sorted && k > SEL_SORT_MAX) return fail(-1, "topk: sorted output limited to k <= 16384");
-    if (sorted && n > 0xffffffffLL) return fail(-1, "topk: sorted output needs n < 2^32");
-    if (ws_bytes < sseqs_topk_ws_bytes(n)) return fail(-2, "topk: workspace too small");
+extern "C" size_t sseqs_topk_ws_bytes(int64_t n) {
+    // plus the bitmap of a sampled select, at a 16-byte aligned address
+    return sel_ws_base(n) +
+           (n >= SEL_SAMPLE_MIN_N ? (size_t)ceil_div(n, SEL_TILE) * SEL_TILE_BITS + 16 : 0);
+}
+
+// bitmap_ok: the workspace holds the bitmap of a sampled select.
+static int topk_impl(const void* scores, int dtype, int64_t n, int64_t k, int sorted,
+                     int64_t* out_idx, void* ws, bool bitmap_ok, hipStream_t stream) {
     uint8_t* w = static_cast<uint8_t*>(ws);
     uint32_t* hist = reinterpret_cast<uint32_t*>(w);
     SelState* st = reinterpret_cast<SelState*>(w + SEL_BINS * 4);
@@ -666,15 +1103,29 @@ extern "C" int sseqs_topk(const void* scores, int dtype, int64_t n, int64_t k, i
     int64_t* cgt = reinterpret_cast<int64_t*>(w + SEL_BINS * 4 + 64);
     int64_t* ceq = cgt + nb;
     int64_t* tmp = ceq + nb;  // SEL_SORT_MAX entries for the sorted path
+    uint32_t* bitmap = nullptr;
 
-    hipLaunchKernelGGL(k_sel_init, dim3(1), dim3(256), 0, stream, hist, st, (uint32_t)k);
-    if (int r = check_launch("topk init")) return r;
-    // keys of fp16 scores have their low 13 bits zero: two passes fix the rest
-    const int shifts32[3] = {21, 10, 0}, bits32[3] = {11, 11, 10};
-    const int shifts16[2] = {21, 13}, bits16[2] = {11, 8};
+    if (bitmap_ok && sel_sampled(scores, dtype, n, k)) {
+        bitmap = reinterpret_cast<uint32_t*>(
+            (reinterpret_cast<uintptr_t>(w + sel_ws_base(n)) + 15) & ~(uintptr_t)15);
+        // expected sample keys among the top k, plus six standard deviations
+        // and eight: P then keeps at least k keys unless the sample misleads
+        const double mu = (double)k / (double)n * SEL_SAMPLE;
+        const int rank = (int)(mu + 6.0 * sqrt(mu) + 8.0) + 1;
+        SEL_DISPATCH(k_sel_sample, dim3(1), dim3(1024), 0, stream, scores, n, hist, st,
+                     (uint32_t)k, rank);
+        if (int r = check_launch("topk sample")) return r;
+        const int64_t fb = ceil_div(nb, 4);
+        SEL_DISPATCH(k_sel_filter, dim3((unsigned)(fb < 2048 ? fb : 2048)), dim3(256), 0, stream,
+                     scores, n, nb, st, bitmap);
+        if (int r = check_launch("topk filter")) return r;
+    } else {
+        hipLaunchKernelGGL(k_sel_init, dim3(1), dim3(256), 0, stream, hist, st, (uint32_t)k);
+        if (int r = check_launch("topk init")) return r;
+    }
+    // digits of 11 bits; keys of fp16 scores have their low 13 bits zero: two
+    // passes fix the rest
     const bool half = dtype == SSEQS_F16;
-    const int* shifts = half ? shifts16 : shifts32;
-    const int* bits = half ? bits16 : bits32;
     int64_t hb = ceil_div(n, 256 * 16);
     unsigned hgrid = (unsigned)(hb < 4096 ? (hb > 0 ? hb : 1) : 4096);
     // fp16 scores at a 16-byte aligned address: eight per thread and load
@@ -683,30 +1134,30 @@ extern "C" int sseqs_topk(const void* scores, int dtype, int64_t n, int64_t k, i
     for (int p = 0; p < (half ? 2 : 3); ++p) {
         if (h8)
             hipLaunchKernelGGL(k_sel_hist_h8, dim3(hgrid), dim3(256), 0, stream, sh, n, st, hist,
-                               shifts[p], bits[p]);
+                               p, bitmap);
         else
-            SEL_DISPATCH(k_sel_hist, dim3(hgrid), dim3(256), 0, stream, scores, n, st, hist,
-                         shifts[p], bits[p]);
+            SEL_DISPATCH(k_sel_hist, dim3(hgrid), dim3(256), 0, stream, scores, n, st, hist, p,
+                         bitmap);
         if (int r = check_launch("topk hist")) return r;
-        hipLaunchKernelGGL(k_sel_pick, dim3(1), dim3(1024), 0, stream, st, hist, shifts[p], bits[p]);
+        SEL_DISPATCH(k_sel_pick, dim3(1), dim3(1024), 0, stream, st, hist, p);
         if (int r = check_launch("topk pick")) return r;
     }
     if (h8)
         hipLaunchKernelGGL(k_sel_count_h8, dim3(grid_cap(nb, 1)), dim3(256), 0, stream, sh, n, nb,
-                           st, cgt, ceq);
+                           st, cgt, ceq, bitmap);
     else
         SEL_DISPATCH(k_sel_count, dim3(grid_cap(nb, 1)), dim3(256), 0, stream, scores, n,
-                     nb, st, cgt, ceq);
+                     nb, st, cgt, ceq, bitmap);
     if (int r = check_launch("topk count")) return r;
     hipLaunchKernelGGL(k_sel_scan, dim3(1), dim3(1024), 0, stream, cgt, ceq, nb);
     if (int r = check_launch("topk scan")) return r;
     int64_t* dst = sorted ? tmp : out_idx;
     if (h8)
         hipLaunchKernelGGL(k_sel_write_h8, dim3(grid_cap(nb, 1)), dim3(256), 0, stream, sh, n, nb,
-                           st, cgt, ceq, k, dst);
+                           st, cgt, ceq, k, dst, bitmap);
     else
         SEL_DISPATCH(k_sel_write, dim3(grid_cap(nb, 1)), dim3(256), 0, stream, scores, n,
-                     nb, st, cgt, ceq, k, dst);
+                     nb, st, cgt, ceq, k, dst, bitmap);
     if (int r = check_launch("topk write")) return r;
     if (sorted) {
         int P = 1;
@@ -724,6 +1175,25 @@ extern "C" int sseqs_topk(const void* scores, int dtype, int64_t n, int64_t k, i
         if (int r = check_launch("topk sort")) return r;
     }
     return 0;
+}
+
+// Checks shared by the two entry points; 1: nothing to do.
+static int topk_check(int dtype, int64_t n, int64_t k, int sorted) {
+    if (n < 0 || k < 0) return fail(-1, "topk: negative size");
+    if (k > n) return fail(-1, "topk: k larger than the number of scores");
+    if (dtype != SSEQS_F32 && dtype != SSEQS_F16 && dtype != SSEQS_I32)
+        return fail(-1, "topk: unsupported dtype");
+    if (k == 0) return 1;
+    if (sorted && k > SEL_SORT_MAX) return fail(-1, "topk: sorted output limited to k <= 16384");
+    if (sorted && n > 0xffffffffLL) return fail(-1, "topk: sorted output needs n < 2^32");
+    return 0;
+}
+
+extern "C" int sseqs_topk(const void* scores, int dtype, int64_t n, int64_t k, int sorted,
+                          int64_t* out_idx, void* ws, size_t ws_bytes, hipStream_t stream) {
+    if (int r = topk_check(dtype, n, k, sorted)) return r < 0 ? r : 0;
+    if (ws_bytes < sseqs_topk_ws_bytes(n)) return fail(-2, "topk: workspace too small");
+    return topk_impl(scores, dtype, n, k, sorted, out_idx, ws, true, stream);
 }
 
 // ------------------------------------------------ sseqs_topk_noalloc --
@@ -783,7 +1253,8 @@ extern "C" int sseqs_topk_noalloc(const void* scores, int dtype, int64_t n, int6
                             std::to_string(noalloc_max_n()) + " scores");
     void* ws = nullptr;
     if (int r = scratch_ptr(&ws)) return r;
-    return sseqs_topk(scores, dtype, n, k, sorted, out_idx, ws, NOALLOC_SCRATCH_BYTES, stream);
+    if (int r = topk_check(dtype, n, k, sorted)) return r < 0 ? r : 0;
+    return topk_impl(scores, dtype, n, k, sorted, out_idx, ws, false, stream);
 }
 
 extern "C" int sseqs_topk_segments(const void* scores, int dtype, const int64_t* seg_begin,
