@@ -6,9 +6,9 @@ Times, on the GPU it runs on, the choices that the results do not depend on:
   (1-8, 9-16, 17-32 columns per lane): ``item`` (candidates per work item,
   the queue's tile width) and ``blocks_per_cu`` (persistent blocks per
   compute unit, i.e. how many queries' items a CU works on at once);
-* the prefilter's dense kernels (queries whose band does not fit the band
-  kernel) per correlation size N: ``SSEQS_CORR_MT`` (m-tiles per pass, i.e.
-  how many shift tiles reuse each decoded database fragment).
+* the prefilter's dense kernels (where neither the band nor the ring kernel
+  runs) per correlation size N: ``SSEQS_CORR_MT`` (m-tiles per pass, i.e. how
+  many shift tiles reuse each decoded database fragment).
 
 Each candidate is timed with HIP events on the launch stream over the
 workload it is tuned for (queries of that class against the database), the
@@ -86,7 +86,7 @@ def tune_prefilter(db, queries: list[str], log=print) -> dict:
     for query in queries:
         q = prepare(query, device=db.device)
         for N, b, e in db.length_ranges(q.length):
-            if prefilter_kernel_name(q.length, q.k, N).startswith("k_corr_band"):
+            if not prefilter_kernel_name(q.length, q.k, N).startswith("k_corr_db"):
                 continue
             if str(N) in out:
                 continue

@@ -998,6 +998,460 @@ __global__ __launch_bounds__(64, (G == 1 && R <= 8 ? 2 : 1)) void k_corr_band(
         if (prev_sid[gg] >= 0) out[prev_sid[gg]] = prev_best[gg];
 }
 
+// ---------------------------------------------------------------------------
+// Rank-4 ring kernel: the band kernel's product with its diagonals spread
+// over the W waves of a block.
+//
+// Wave w holds the A fragments of the R diagonals d0 + wR .. + R-1 (R <= 8:
+// 128 registers, two waves per SIMD at any query length) and, at chunk v, the
+// accumulators of the m-tiles rel = v + wR .. + R-1 (rel = I - d0 before
+// reduction mod ND, as in the band kernel).  An m-tile meets the diagonals in
+// descending order, so the tile that wave w finishes at chunk v (its rel =
+// v + wR) is the one wave w-1 opens at chunk v+1: accumulators travel down
+// the waves through LDS, one per wave and chunk, and every m-tile's sum is
+// taken in the order one wave holding all the diagonals would take.  Wave 0
+// folds finished tiles into the running maximum, or parks the ones that the
+// circular wrap reaches again.  FULL (W R == ND): the ring is closed, wave 0
+// passes its tiles on to wave W-1, and all tiles are folded after the last
+// chunk.
+//
+// The B fragments of a chunk are decoded once per block: wave w decodes the
+// sub-chunks q = w (mod W) of chunk v+1 into LDS while chunk v is multiplied,
+// with one barrier per chunk (which also covers the hand-over).  That is
+// about 15 VALU instructions per wave and chunk against R * 4 MFMAs, a third
+// of the band kernel's.
+//
+// Sources: the packed stream (5-bit symbols, btab index 32 stands for masked
+// positions, so an '@' inside a span has its own value) or an ASCII batch
+// (bytes, masked index 256).  A tile is staged like the band kernel's: as one
+// byte range, as one slot per sequence, or not at all (symbols are then read
+// from global memory).  Only 16-byte granules that hold a symbol in use are
+// copied: whatever the address and size of the buffer, a copy stays within
+// the granules of its own bytes.
+//
+// What bounds it and what it measured: see plan_prefilter.
+// ---------------------------------------------------------------------------
+struct RingPacked {
+    static constexpr int BITS = 5, TAB = 33, MASKED = 32;
+    const uint8_t* base;  // 16-byte aligned
+    int64_t shift;        // symbols from base to symbol 0
+    const int64_t* off;
+    const int32_t* len;
+    __device__ int64_t offset(int64_t s) const { return off[s]; }
+    __device__ static int code(int c) { return corr_code((uint32_t)c + 64u); }
+    __device__ uint32_t sym(int64_t o, int p) const { return packed_sym(base, o + p) - 64u; }
+};
+struct RingAscii {
+    static constexpr int BITS = 8, TAB = 257, MASKED = 256;
+    const uint8_t* base;
+    int64_t shift;
+    const int32_t* off;
+    const int32_t* len;
+    __device__ int64_t offset(int64_t s) const { return off[s] + shift; }
+    __device__ static int code(int c) { return corr_code((uint32_t)c); }
+    __device__ uint32_t sym(int64_t o, int p) const { return base[o + p]; }
+};
+
+template <int W, int R, bool FULL, bool DBL, class Src, class OutT>
+__global__ __launch_bounds__(64 * W, 2) void k_corr_ring(
+    Src src, int64_t s_begin, int64_t nseq, const uint8_t* __restrict__ qrev, int Lq,
+    const float* __restrict__ lutA, const float* __restrict__ lutB, int V, int N, int maxlen,
+    int CAPB, int d0, int Rn, OutT* __restrict__ out) {
+    constexpr int K = 4, S = Src::BITS;
+    constexpr int TABB = (Src::TAB * 8 + 15) & ~15;
+    extern __shared__ __align__(16) uint8_t smem[];
+    uint64_t* btab4 = reinterpret_cast<uint64_t*>(smem);  // [TAB] x 4 fp16
+    uint8_t* region = smem + TABB;
+    uint64_t* qtab4 = reinterpret_cast<uint64_t*>(region);  // [N+8] x 4 fp16, set-up only
+    float* red = reinterpret_cast<float*>(region);          // [2][W][64]
+    f32x4* hand = reinterpret_cast<f32x4*>(region + 2 * W * 256);  // [2][W][64] (W > 1)
+    half8* bbuf = reinterpret_cast<half8*>(hand + (W > 1 ? 2 * W * 64 : 0));  // [2][4][64]
+    f32x4* save = reinterpret_cast<f32x4*>(bbuf + (W > 1 ? 2 * 4 * 64 : 0));  // [Rn][64], the last one unused
+    uint8_t* stg = reinterpret_cast<uint8_t*>(save + (FULL ? 0 : Rn * 64));
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = W > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : 0;
+    const int Lqe = min(Lq, N);
+    for (int u = tid; u < N + 8; u += 64 * W) {
+        const int t = (N - (u & (N - 1))) & (N - 1);
+        union {
+            _Float16 h[4];
+            uint64_t x;
+        } e;
+#pragma unroll
+        for (int r = 0; r < K; ++r)
+            e.h[r] = (_Float16)(t < Lqe ? 0.5f * lutA[r * V + (int)qrev[t]] : 0.f);
+        qtab4[u] = e.x;
+    }
+    for (int c = tid; c < Src::TAB; c += 64 * W) {
+        union {
+            _Float16 h[4];
+            uint64_t x;
+        } e;
+#pragma unroll
+        for (int r = 0; r < K; ++r)
+            e.h[r] = (_Float16)(c < Src::MASKED ? lutB[r * V + Src::code(c)] : 0.f);
+        btab4[c] = e.x;
+    }
+    __syncthreads();
+    // lane (col, g): A row col, B/C column col, positions 8g .. 8g+7 of a chunk
+    const int col = lane & 15, g = lane >> 4;
+    half8 A[R][4];
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int u = (8 * g + 2 * q - 2 * col - 32 * (d0 + w * R + j)) & (N - 1);
+            union {
+                uint64_t x[2];
+                half8 v;
+            } a;
+            a.x[0] = qtab4[u];
+            a.x[1] = qtab4[u + 1];
+            A[j][q] = a.v;
+        }
+    __syncthreads();  // the region now holds the run-time buffers
+
+    const int ND = N >> 5;
+    const int64_t ntiles = (nseq + 15) / 16;
+    int64_t tile = blockIdx.x;
+    if (tile >= ntiles) return;
+    const int SB = (CAPB + 64 + 15) & ~15;
+
+    // raw index entries of tile t's sequences (clamped into range)
+    auto meta = [&](int64_t t, int64_t* o, int* L) {
+        const int64_t sid = min(t * 16 + col, nseq - 1);
+        *o = src.offset(s_begin + sid);
+        *L = src.len[s_begin + sid];
+    };
+    // first byte of a symbol, and the 16-byte granules that hold symbols o .. o+n-1 (n > 0)
+    auto byte_of = [&](int64_t o) -> int64_t { return (S * o) >> 3; };
+    auto granules = [&](int64_t b_lo, int64_t o, int64_t n) -> int64_t {
+        return (((S * (o + n) - 1) >> 3) - b_lo + 16) >> 4;
+    };
+    struct Tile {
+        int64_t o, b_lo;
+        int Le, C, scb, nchunk;  // scb: 16-byte chunks of a slot, 0 for a range
+        bool in, fast;
+    };
+    auto info = [&](int64_t t, int64_t o, int L) -> Tile {
+        Tile T;
+        T.in = t * 16 + col < nseq;
+        T.Le = T.in ? max(0, min(min(L, maxlen), N)) : 0;
+        // extent of the tile's sequences that hold symbols (the 16 columns are
+        // the 16 lanes of every DPP row)
+        const bool use = T.Le > 0;
+        auto at = [](int64_t v, int l) -> int64_t {
+            return ((int64_t)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32) |
+                   (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+        };
+        // in a length-sorted stream offsets and lengths rise across a tile, so
+        // its first and last sequences bound it
+        const int nin = (int)min((int64_t)16, nseq - t * 16);
+        const int64_t o_prev = dpp_row64<0x111>(o);  // row_shr:1, column col-1
+        const int L_prev = dpp_row<0x111>(T.Le);
+        const bool rising = __ballot(!(col >= nin || (use && (col == 0 || (o > o_prev && T.Le >= L_prev))))) == 0;
+        int kp;
+        int64_t lo, hi, ehi;
+        if (rising) {
+            kp = __builtin_amdgcn_readlane(T.Le, nin - 1);
+            lo = at(o, 0);
+            hi = at(o, nin - 1);
+            ehi = hi + kp;
+        } else {
+            kp = __builtin_amdgcn_readfirstlane(row_max(T.Le));
+            lo = at(row_ext64<false>(use ? o : INT64_MAX), 0);
+            hi = at(row_ext64<true>(use ? o : 0), 0);
+            ehi = at(row_ext64<true>(use ? o + T.Le : 0), 0);
+        }
+        T.C = (kp + 31) >> 5;
+        T.o = use ? o : (kp > 0 ? lo : 0);  // idle lanes decode (and mask) inside the stage
+        T.b_lo = kp > 0 ? byte_of(lo) & ~(int64_t)15 : 0;
+        T.scb = 0;
+        T.nchunk = 0;
+        // the last window of a lane ends within 8 bytes of its last position's
+        T.fast = kp == 0 || byte_of(hi + 32 * T.C) + 24 - T.b_lo <= CAPB;
+        if (T.fast) {
+            if (kp > 0) T.nchunk = (int)granules(T.b_lo, lo, ehi - lo);
+        } else {
+            const int scb = ((S * kp + 14) / 8 + 15 + 15) >> 4;
+            if (max(16 * 16 * scb, 15 * 16 * scb + 4 * S * T.C + 15 + 24) <= CAPB) {
+                T.scb = scb;
+                T.fast = true;
+                T.nchunk = 16 * scb;
+            }
+        }
+        return T;
+    };
+    // asynchronous copies global -> LDS, 64 x 16 bytes each, shared out over the waves
+    auto issue = [&](const Tile& T, uint8_t* buf) {
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)buf;
+        for (int c0 = 64 * w; c0 < T.nchunk; c0 += 64 * W) {
+            const int c = c0 + lane;
+            const uint8_t* from = src.base + T.b_lo + 16 * (int64_t)c;
+            bool on = c < T.nchunk;
+            if (T.scb) {  // chunk j of slot s: the sequence of column s
+                const int s = c / T.scb, j = c - s * T.scb;
+                const int64_t os = __shfl(T.o, s & 15);
+                const int ls = __shfl(T.Le, s & 15);
+                const int64_t bb = byte_of(os) & ~(int64_t)15;
+                on = on && ls > 0 && j < granules(bb, os, ls);
+                from = src.base + bb + 16 * j;
+            }
+            if (on)
+                asm volatile("global_load_lds_dwordx4 %1, off"
+                             :
+                             : "{m0}"(lds0 + 16u * (uint32_t)c0), "v"(from)
+                             : "memory");
+        }
+    };
+
+    int64_t o_n = 0, o_c;
+    int L_n = 0, L_c;
+    meta(tile, &o_c, &L_c);
+    if (tile + gridDim.x < ntiles) meta(tile + gridDim.x, &o_n, &L_n);
+    Tile cur = info(tile, o_c, L_c);
+    issue(cur, stg);
+    if constexpr (W > 1) {  // what wave W-1 opens stays zero (not FULL)
+        hand[w * 64 + lane] = f32x4{0.f, 0.f, 0.f, 0.f};
+        hand[(W + w) * 64 + lane] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    // the previous tile's result: reduced over the waves and stored after the
+    // next barrier (W > 1)
+    int64_t prev = -1;
+    bool prev_in = false;
+    auto store_prev = [&](int par) {
+        if (w != 0 || prev < 0) return;
+        float m = red[par * W * 64 + lane];
+#pragma unroll
+        for (int i = 1; i < W; ++i) m = fmaxf(m, red[(par * W + i) * 64 + lane]);
+        // the four lane groups hold different rows of the same columns
+        m = fmaxf(m, __shfl_xor(m, 16, 64));
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        if (g == 0 && prev_in) store_score<OutT>(out, prev * 16 + col, m);
+    };
+    int sb = 0, par = 0;
+    for (;;) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();  // the tile's bytes are in; the previous tile's buffers are free
+        const int64_t tn = tile + gridDim.x;
+        Tile nxt{};
+        if (tn < ntiles) {
+            nxt = info(tn, o_n, L_n);
+            if (DBL) issue(nxt, stg + (sb ^ 1) * SB);
+        }
+        if (tn + gridDim.x < ntiles) meta(tn + gridDim.x, &o_n, &L_n);
+        store_prev(par ^ 1);
+        const uint8_t* sbuf = stg + (DBL ? sb * SB : 0);
+        const int C = cur.C;
+        const int x = FULL ? 0 : max(0, C - ND + Rn - 1);
+        // bit of this lane's sequence in the stage
+        const int relbit = cur.scb ? 128 * cur.scb * col + (int)(S * cur.o - 8 * (byte_of(cur.o) & ~(int64_t)15))
+                                   : (int)(S * cur.o - 8 * cur.b_lo);
+        float best = -INFINITY;
+        // Decode of sub-chunk q of chunk v (positions pb, pb + 1 of this lane's
+        // sequence) in two steps: the stage words that hold its symbols, and
+        // the symbols' table entries.
+        struct Raw {
+            uint32_t w0, w1;
+        };
+        auto words = [&](auto fast_tag, int v, int q) -> Raw {
+            const int pb = 32 * v + 8 * g + 2 * q;
+            if constexpr (decltype(fast_tag)::value) {
+                const int bit = relbit + S * pb;
+                const uint32_t* p = reinterpret_cast<const uint32_t*>(sbuf + ((bit >> 3) & ~3));
+                return Raw{p[0], p[1]};
+            } else {
+                return Raw{pb < cur.Le ? src.sym(cur.o, pb) : 0u,
+                           pb + 1 < cur.Le ? src.sym(cur.o, pb + 1) : 0u};
+            }
+        };
+        auto symbol = [&](auto fast_tag, Raw r, int v, int q, int e) -> uint32_t {
+            const int pb = 32 * v + 8 * g + 2 * q;
+            uint32_t c;
+            if constexpr (!decltype(fast_tag)::value) {
+                c = e ? r.w1 : r.w0;
+            } else if constexpr (S == 8) {
+                const uint32_t byte = (uint32_t)((relbit >> 3) + pb);
+                c = (__builtin_amdgcn_alignbyte(r.w1, r.w0, byte & 3u) >> (8 * e)) & 255u;
+            } else {
+                const int bit = relbit + S * pb;
+                const uint64_t be = ((uint64_t)__builtin_bswap32(r.w0) << 32) | __builtin_bswap32(r.w1);
+                c = ((uint32_t)((be << (bit & 31)) >> 32) >> (27 - 5 * e)) & 31u;
+            }
+            return pb + e < cur.Le ? c : (uint32_t)Src::MASKED;
+        };
+        auto pair = [&](auto fast_tag, Raw r, int v, int q) -> half8 {
+            union {
+                uint64_t x[2];
+                half8 v;
+            } u;
+            u.x[0] = btab4[symbol(fast_tag, r, v, q, 0)];
+            u.x[1] = btab4[symbol(fast_tag, r, v, q, 1)];
+            return u.v;
+        };
+        // The tile's chunks; one instance for staged symbols, one for symbols
+        // read from global memory.
+        auto run = [&](auto fast_tag) {
+            // sub-chunks decoded by this wave (W == 8: half of one)
+            constexpr int NQ = W == 1 ? 4 : W == 2 ? 2 : 1;
+            auto sub = [&](int i) { return W == 1 ? i : W == 2 ? 2 * i + w : w & 3; };
+            auto put = [&](int v, int i, Raw r) {  // table entries of sub-chunk sub(i) to LDS
+                half8* dst = &bbuf[((v & 1) * 4 + sub(i)) * 64 + lane];
+                if constexpr (W == 8)
+                    reinterpret_cast<uint64_t*>(dst)[w >> 2] =
+                        btab4[symbol(fast_tag, r, v, w & 3, w >> 2)];
+                else
+                    *dst = pair(fast_tag, r, v, sub(i));
+            };
+            f32x4 acc[R];
+#pragma unroll
+            for (int t = 0; t < R; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            half8 bcur[4];  // W == 1
+            if (C > 0) {
+#pragma unroll
+                for (int i = 0; i < NQ; ++i) {
+                    const Raw r = words(fast_tag, 0, sub(i));
+                    if constexpr (W == 1)
+                        bcur[i] = pair(fast_tag, r, 0, i);
+                    else
+                        put(0, i, r);
+                }
+                if constexpr (W > 1) hand[w * 64 + lane] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            for (int vb = 0; vb < C; vb += R) {
+#pragma unroll
+                for (int s = 0; s < R; ++s) {
+                    const int v = vb + s;
+                    if (v < C) {
+                        // the next chunk (the last one again at the end: its
+                        // buffer is then written for nobody)
+                        const int vn = min(v + 1, C - 1);
+                        half8 b[4], bnxt[4];
+                        Raw raw[NQ];
+                        if constexpr (W > 1) {
+                            __syncthreads();
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) b[q] = bbuf[((v & 1) * 4 + q) * 64 + lane];
+                            // the tile opened here: handed over by the wave above
+                            acc[(s + R - 1) % R] = hand[((v & 1) * W + w) * 64 + lane];
+                        } else {
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) b[q] = bcur[q];
+                        }
+#pragma unroll
+                        for (int i = 0; i < NQ; ++i) raw[i] = words(fast_tag, vn, sub(i));
+                        auto products = [&](int q) {
+#pragma unroll
+                            for (int j = 0; j < R; ++j)
+                                acc[(s + j) % R] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                    A[j][q], b[q], acc[(s + j) % R], 0, 0, 0);
+                        };
+                        if constexpr (W == 1) {
+#pragma unroll
+                            for (int i = 0; i < NQ; ++i) bnxt[i] = pair(fast_tag, raw[i], vn, i);
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) products(q);
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) bcur[q] = bnxt[q];
+                        } else {
+                            // the decode's two LDS latencies under the products
+                            __builtin_amdgcn_sched_barrier(0);
+                            products(0);
+                            __builtin_amdgcn_sched_barrier(0);
+                            uint64_t e[2 * NQ];
+#pragma unroll
+                            for (int i = 0; i < NQ; ++i) {
+                                if constexpr (W == 8) {
+                                    e[0] = btab4[symbol(fast_tag, raw[0], vn, w & 3, w >> 2)];
+                                } else {
+                                    e[2 * i] = btab4[symbol(fast_tag, raw[i], vn, sub(i), 0)];
+                                    e[2 * i + 1] = btab4[symbol(fast_tag, raw[i], vn, sub(i), 1)];
+                                }
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
+                            products(1);
+                            products(2);
+                            __builtin_amdgcn_sched_barrier(0);
+                            // chunk v + 1's buffer, also when vn is the last chunk again
+#pragma unroll
+                            for (int i = 0; i < NQ; ++i) {
+                                uint64_t* dst = reinterpret_cast<uint64_t*>(
+                                    &bbuf[(((v + 1) & 1) * 4 + sub(i)) * 64 + lane]);
+                                if constexpr (W == 8) {
+                                    dst[w >> 2] = e[0];
+                                } else {
+                                    dst[0] = e[2 * i];
+                                    dst[1] = e[2 * i + 1];
+                                }
+                            }
+                            products(3);
+                        }
+                        // tile rel = v + wR is done (after the last chunk: also
+                        // still in acc, and folded below)
+                        if (W > 1 && (FULL || w > 0)) {
+                            hand[(((v + 1) & 1) * W + (w + W - 1) % W) * 64 + lane] = acc[s];
+                        } else if (!FULL) {
+                            const bool park = v < x;
+                            save[(park ? v : Rn - 1) * 64 + lane] = acc[s];
+                            const float m = max4(acc[s]);
+                            best = park ? best : fmaxf(best, m);
+                        }
+                        if (W == 1 && !FULL && v + 1 < C) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+                }
+            }
+            if (!FULL && W > 1) __syncthreads();  // the parked tiles are in LDS
+            if (C == 0) {
+                best = 0.f;
+            } else {
+                const int first = (C - 1) % R;  // slot of rel = C - 1 + wR
+#pragma unroll
+                for (int t = 0; t < R; ++t) {
+                    if (FULL) {
+                        best = fmaxf(best, max4(acc[t]));
+                    } else {
+                        const int j = t >= first ? t - first : t - first + R;
+                        const int rel = C - 1 + w * R + j;
+                        if (rel < ND)
+                            best = fmaxf(best, max4(acc[t]));
+                        else if (rel - ND < x)
+                            best = fmaxf(best, max4(acc[t] + save[(rel - ND) * 64 + lane]));
+                    }
+                }
+                if (!FULL && C + Rn - 1 < ND) best = fmaxf(best, 0.f);  // unreached m-tiles
+            }
+        };
+        if (cur.fast)
+            run(std::true_type{});
+        else
+            run(std::false_type{});
+        if constexpr (W > 1) {
+            red[(par * W + w) * 64 + lane] = best;
+            prev = tile;
+            prev_in = cur.in;
+            par ^= 1;
+        } else {
+            best = fmaxf(best, __shfl_xor(best, 16, 64));
+            best = fmaxf(best, __shfl_xor(best, 32, 64));
+            if (g == 0 && cur.in) store_score<OutT>(out, tile * 16 + col, best);
+        }
+        tile = tn;
+        if (tile >= ntiles) break;
+        if (!DBL) {
+            __syncthreads();  // the stage is no longer read
+            issue(nxt, stg);
+        } else {
+            sb ^= 1;
+        }
+        cur = nxt;
+    }
+    if constexpr (W > 1) {
+        __syncthreads();
+        store_prev(par ^ 1);
+    }
+}
+
 // Nonzero diagonals of the band kernel: diagonal d's A blocks read lags
 // (32d + e) mod N, e in [-31, 30], and the query fills lags [0, Lqe).  The
 // nonzero ones form one circular run; returns its start and length.
@@ -1046,6 +1500,93 @@ static int launch_corr(const Src& src, int64_t s_begin, int64_t nseq, const uint
 
 using namespace sseqs;
 
+// Launch shape of the ring kernel for a rank-4 correlation of size N >= 128
+// whose query has rn > 0 nonzero diagonals.
+struct RingPlan {
+    int W = 0, R = 0;  // waves per block, diagonals per wave (0: no shape)
+    bool full = false, dbl = true;
+    int capb = 0;      // stage capacity (bytes)
+    size_t lds = 0;    // dynamic LDS (bytes)
+    unsigned blocks = 0;  // blocks that are resident at once
+};
+
+static RingPlan plan_ring(int N, int rn, int mlen, int bits, int tab) {
+    RingPlan P;
+    const int ND = N / 32;
+    static const int shapes[][2] = {{1, 4}, {1, 6}, {1, 8}, {2, 5}, {2, 6}, {2, 8}, {4, 5},
+                                    {4, 6}, {4, 7}, {4, 8}, {8, 5}, {8, 6}, {8, 7}, {8, 8}};
+    for (const auto& sh : shapes)
+        if (!P.W && sh[0] * sh[1] >= rn && sh[0] * sh[1] <= ND) {
+            P.W = sh[0];
+            P.R = sh[1];
+        }
+    if (!P.W) return P;
+    P.full = P.W * P.R == ND;
+    // the stage holds 16 sequences of up to span symbols back to back, or
+    // (where that leaves two waves per SIMD) one slot each
+    const int span = (min(mlen, N) + 31) & ~31;
+    const int scb = ((bits * span + 14) / 8 + 15 + 15) >> 4;
+    const int range = (int)((((int64_t)16 * (span + 1) * bits) / 8 + 48 + 15) & ~15);
+    const int slots = (max(16 * 16 * scb, 15 * 16 * scb + 4 * bits * (span / 32) + 39) + 15) & ~15;
+    const size_t tabb = ((size_t)tab * 8 + 15) & ~(size_t)15;
+    const size_t fixed = (size_t)2 * P.W * 256 + (P.W > 1 ? 2 * P.W * 1024 + 8192 : 0) +
+                         (P.full ? 0 : (size_t)rn * 1024);
+    const size_t qt = (size_t)(N + 8) * 8;
+    auto lds_for = [&](int cap, int nbuf) {
+        const size_t run = fixed + nbuf * (size_t)((cap + 64 + 15) & ~15);
+        return tabb + ((max(qt, run) + 15) & ~(size_t)15);
+    };
+    const size_t budget = (size_t)160 * 1024 * P.W / 8;  // eight waves per CU
+    // one wave per block: a second buffer only while eight blocks fit a CU
+    // (261 000 ASCII segments of 305: eight with one buffer 100 us, seven
+    // with two 111 us)
+    P.dbl = P.W > 1 || lds_for(range, 2) <= budget;
+    const int nbuf = P.dbl ? 2 : 1;
+    P.capb = slots > range && lds_for(slots, nbuf) <= budget ? slots : range;
+    P.lds = lds_for(P.capb, nbuf);
+    const size_t fit = (size_t)160 * 1024 / P.lds;
+    P.blocks = (unsigned)(256 * max((size_t)1, min((size_t)(8 / P.W), fit)));
+    return P;
+}
+
+static bool ring_fits(const RingPlan& P) { return P.W && P.lds <= 160 * 1024; }
+
+template <class Src, class OutT>
+static int launch_ring(const RingPlan& P, const Src& src, int64_t s_begin, int64_t nseq,
+                       const uint8_t* qrev, int Lq, const float* lutA, const float* lutB, int V,
+                       int N, int mlen, int d0, int rn, OutT* out, hipStream_t stream) {
+    const int64_t tiles = ceil_div(nseq, 16);
+    const unsigned grid = (unsigned)(tiles < P.blocks ? tiles : P.blocks);
+    auto go = [&](auto kern) -> int {
+        if (P.lds > 64 * 1024 &&
+            hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)P.lds) != hipSuccess)
+            return fail(-3, "prefilter: cannot enable large LDS");
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * P.W), P.lds, stream, src, s_begin, nseq,
+                           qrev, Lq, lutA, lutB, V, N, mlen, P.capb, d0, rn, out);
+        return check_launch("prefilter");
+    };
+    switch (100 * P.W + 10 * P.R + (P.full ? 1 : 0)) {
+#define RING1(R, F, ID)                                                         \
+    case ID:                                                                    \
+        return P.dbl ? go(&k_corr_ring<1, R, F, true, Src, OutT>)               \
+                     : go(&k_corr_ring<1, R, F, false, Src, OutT>);
+#define RINGW(W, R, F, ID) \
+    case ID:               \
+        return go(&k_corr_ring<W, R, F, true, Src, OutT>);
+        RING1(4, true, 141) RING1(4, false, 140) RING1(6, false, 160) RING1(8, true, 181)
+        RING1(8, false, 180) RINGW(2, 5, false, 250) RINGW(2, 6, false, 260)
+        RINGW(2, 8, true, 281) RINGW(2, 8, false, 280) RINGW(4, 5, false, 450)
+        RINGW(4, 6, false, 460) RINGW(4, 7, false, 470) RINGW(4, 8, true, 481)
+        RINGW(4, 8, false, 480) RINGW(8, 5, false, 850) RINGW(8, 6, false, 860)
+        RINGW(8, 7, false, 870) RINGW(8, 8, true, 881)
+#undef RING1
+#undef RINGW
+    }
+    return fail(-1, "prefilter: no kernel of this shape");
+}
+
 extern "C" int launch_warp_corr(uint16_t* corr, const uint8_t* qrev, const float* lutA,
                                 const float* W_db, const uint8_t* flat, const int32_t* offsets,
                                 const int32_t* lengths, float* out_stats, int B, int vocab_size,
@@ -1055,6 +1596,20 @@ extern "C" int launch_warp_corr(uint16_t* corr, const uint8_t* qrev, const float
     (void)query_rfft;
     if (B < 0) return fail(-1, "warp_corr: negative segment count");
     if (B == 0) return 0;
+    const int mlen = maxlen < 0 ? 0 : maxlen, Lqe = min(query_len, N_full);
+    if (k == 4 && vocab_size >= 1 && N_full >= 128 && N_full <= 2048 &&
+        !(N_full & (N_full - 1)) && Lqe > 0 && !getenv("SSEQS_CORR_NO_BAND")) {
+        int d0, rn;
+        band_diagonals(N_full, Lqe, &d0, &rn);
+        const RingPlan P = plan_ring(N_full, rn, mlen, RingAscii::BITS, RingAscii::TAB);
+        if (ring_fits(P)) {
+            const uintptr_t at = reinterpret_cast<uintptr_t>(flat);
+            const RingAscii src{reinterpret_cast<const uint8_t*>(at & ~(uintptr_t)15),
+                                (int64_t)(at & 15), offsets, lengths};
+            return launch_ring(P, src, 0, B, qrev, query_len, lutA, W_db, vocab_size, N_full,
+                               mlen, d0, rn, reinterpret_cast<_Float16*>(corr), stream);
+        }
+    }
     CorrAscii src{flat, offsets, lengths};
     return launch_corr<CorrAscii, _Float16, false>(src, 0, B, qrev, query_len, lutA, W_db,
                                                    vocab_size, k, N_full, maxlen,
@@ -1063,7 +1618,7 @@ extern "C" int launch_warp_corr(uint16_t* corr, const uint8_t* qrev, const float
 
 // Which kernel and launch shape sseqs_db_prefilter uses for a length range.
 struct PrefilterPlan {
-    enum Kind { BAND, DB4, DB } kind;
+    enum Kind { BAND, RING, DB4, DB } kind;
     int R = 0;        // band: ring size (diagonals held in registers)
     int G = 1;        // band: groups of 16 sequences per tile
     bool full = false, dbl = false;
@@ -1072,6 +1627,7 @@ struct PrefilterPlan {
     int capb = 0;     // stage capacity (bytes)
     size_t lds = 0;   // dynamic LDS (bytes)
     int tile = 32;    // sequences per tile
+    RingPlan ring;
 };
 
 static PrefilterPlan plan_prefilter(int query_len, int k, int N, int mlen, bool allow_band = true) {
@@ -1080,12 +1636,16 @@ static PrefilterPlan plan_prefilter(int query_len, int k, int N, int mlen, bool 
     if (allow_band && k == 4 && N >= 128 && Lqe > 0 && !getenv("SSEQS_CORR_NO_BAND")) {
         band_diagonals(N, Lqe, &P.d0, &P.rn);
         const int ND = N / 32;
-        P.full = P.rn == ND;
+        for (int c : {4, 6, 8, 12, 16, 18})
+            if (!P.R && P.rn <= c) P.R = c;
+        // every m-tile stays live: no closing, parking or reopening per chunk.
+        // Taken wherever the ring holds all diagonals, also when some of them
+        // are zero: N = 512 with 13-15 nonzero ones 3.05 against 3.67 ms, N =
+        // 256 with 7 0.63 against 0.71 ms (a database of 8 M sequences)
+        P.full = P.R >= ND;
         if (P.full) {
-            P.R = ND <= 16 ? ND : 0;
-        } else {
-            for (int c : {4, 6, 8, 12, 16, 18})
-                if (!P.R && P.rn <= c) P.R = c;
+            P.R = ND;
+            P.d0 = 0;
         }
         if (P.R) {
             P.kind = PrefilterPlan::BAND;
@@ -1118,6 +1678,26 @@ static PrefilterPlan plan_prefilter(int query_len, int k, int N, int mlen, bool 
             return P;
         }
     }
+    // Past the band kernel's 18 diagonals (queries of about 515 residues and
+    // more), and for spans that may hold '@': the ring kernel.  4 M sequences
+    // (0.77 GB packed), this against the dense rank-4 kernel below: 560
+    // residues 2.7 / 5.0 ms, 900 3.15 / 5.06 ms.  Bound by the matrix cores: a
+    // chunk of 128 diagonal products runs at 1.6 PF/s (independent products
+    // of one wave pair per SIMD sustain 1.7-1.8), each tile adds about two
+    // chunks.  Up to 18 diagonals one wave holds them all and the band kernel
+    // is faster (18 diagonals, 8 M sequences: 4.76 / 5.4 ms; 12: 3.0 / 3.2).
+    // An ASCII batch takes it at any rank-4 size (launch_warp_corr): 261 000
+    // segments of 305 at 200 residues 100 us, 1337 us on the generic kernel.
+    if (k == 4 && N >= 128 && Lqe > 0 && !getenv("SSEQS_CORR_NO_BAND")) {
+        band_diagonals(N, Lqe, &P.d0, &P.rn);
+        P.ring = plan_ring(N, P.rn, mlen, RingPacked::BITS, RingPacked::TAB);
+        if (ring_fits(P.ring)) {
+            P.kind = PrefilterPlan::RING;
+            P.tile = 16;
+            P.lds = P.ring.lds;
+            return P;
+        }
+    }
     P.kind = k == 4 ? PrefilterPlan::DB4 : PrefilterPlan::DB;
     const int KPmax = (min(mlen, N) + 15) & ~15;
     // a length-sorted tile spans about 32 sequences of at most KPmax symbols
@@ -1143,6 +1723,9 @@ static std::string plan_name(const PrefilterPlan& P) {
     if (P.kind == PrefilterPlan::BAND)
         snprintf(b, sizeof b, "k_corr_band<%d, %s, %s, %d>", P.R, P.full ? "true" : "false",
                  P.dbl ? "true" : "false", P.G);
+    else if (P.kind == PrefilterPlan::RING)
+        snprintf(b, sizeof b, "k_corr_ring<%d, %d, %s>", P.ring.W, P.ring.R,
+                 P.ring.full ? "true" : "false");
     else
         snprintf(b, sizeof b, "%s<%d>", P.kind == PrefilterPlan::DB4 ? "k_corr_db4" : "k_corr_db",
                  P.nmt);
@@ -1206,6 +1789,11 @@ static int db_prefilter(const uint8_t* packed, const int64_t* seq_off, const int
             }
         };
         return P.dbl ? pick(std::true_type{}) : pick(std::false_type{});
+    }
+    if (P.kind == PrefilterPlan::RING) {
+        const RingPacked src{packed, 0, seq_off, seq_len};
+        return launch_ring(P.ring, src, s_begin, nseq, qrev, query_len, lutA, lutB, vocab_size, N,
+                           mlen, P.d0, P.rn, scores, stream);
     }
     if (P.kind == PrefilterPlan::DB4) {
         auto go4 = [&](auto kern) -> int {

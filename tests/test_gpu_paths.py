@@ -90,3 +90,59 @@ def test_topk_sampled(dev, n, k, dtype, kind):
         _lib.call("sseqs_topk_noalloc", s.data_ptr(), ops._DT[s.dtype], n, k, 0, out.data_ptr(),
                   _lib.stream_of(dev))
         assert np.array_equal(out.cpu().numpy(), np.sort(want))
+
+
+RING_SHAPES = [(128, 40), (128, 100), (256, 60), (256, 150), (256, 250), (512, 120), (512, 200), (512, 300),
+               (512, 500), (1024, 90), (1024, 350), (1024, 450), (1024, 560), (1024, 690), (1024, 820),
+               (1024, 1000), (1024, 1500), (2048, 200), (2048, 1100), (2048, 1400), (2048, 1700), (2048, 2000)]
+
+
+@pytest.mark.parametrize("N,Lq", RING_SHAPES)
+def test_rank4_ring(orc, dev, N, Lq):
+    """Every shape of the rank-4 ring kernel on an ASCII batch: segments of
+    every kind of length (empty, one, chunk edges, the whole N, past it), any
+    byte inside them, in order and scattered over the batch (slots, and no
+    stage), batches at odd addresses, one segment alone; and on packed spans
+    that hold '@'."""
+    from sseqs_amd import ops
+    from sseqs_amd._lib import call, ptr, stream_of
+    announce(f"ring N={N} Lq={Lq}")
+    rng = np.random.default_rng(7 * N + Lq)
+    query = rand_seq(rng, Lq)
+    A, B = orc.weighted_luts(query, 4)
+    qrev = orc.encode_query_rev(query)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)  # noqa: E731
+    edges = [0, 1, 31, 32, 33, N // 2, N - 32, N - 31, N - 1, N, N + 5]
+    lens = np.array(edges + list(rng.integers(1, N + 1, 60)), np.int32)
+    for order in ("sorted", "shuffled", "scattered"):
+        ln = np.sort(lens) if order == "sorted" else rng.permutation(lens).astype(np.int32)
+        gap = 40 * N if order == "scattered" else 1
+        off = np.concatenate([[0], np.cumsum(ln + gap)[:-1]]).astype(np.int32)
+        letters = np.frombuffer((AA * 20 + "XBZ*-@").encode(), np.uint8)
+        flat = letters[rng.integers(0, letters.size, int(off[-1] + ln[-1] + 1))].copy()
+        for o, n in zip(off, ln):  # homologous stretches, and bytes that are no letters
+            if n > 40:
+                q = np.frombuffer(query.encode(), np.uint8)[: int(n)]
+                flat[o:o + q.size] = q
+            flat[o + int(rng.integers(0, n)) if n else 0] = rng.choice([0, 255, 64, 42, 1])
+        maxlen = int(ln.max()) if order != "shuffled" else max(1, N - 40)
+        want = orc.corr(qrev, A, B, 4, flat.tobytes(), off, ln, maxlen, N)
+        tol = orc.corr_tol(qrev, A, B, 4, flat.tobytes(), off, ln, maxlen, N, want)
+        for lead, sel in ((0, slice(None)), (5, slice(None)), (0, slice(3, 4))):
+            f = torch.cat([torch.zeros(lead, dtype=torch.uint8, device=dev), t(flat)])[lead:]
+            scores = torch.zeros(ln[sel].size, dtype=torch.float16, device=dev)
+            ops.warp_corr(scores, t(qrev), t(A), t(B), f, t(off[sel]), t(ln[sel]), 4, Lq, maxlen, N,
+                          torch.zeros(1, dtype=torch.float16, device=dev))
+            got = scores.float().cpu().numpy()
+            assert (np.abs(got - want[sel]) <= tol[sel]).all(), (order, lead)
+        # the same symbols packed, as spans that may hold '@' (5 bits hold letters only)
+        sym = np.where((flat >= 64) & (flat < 96), flat, 64).astype(np.uint8)
+        want = orc.corr(qrev, A, B, 4, sym.tobytes(), off, ln, maxlen, N)
+        tol = orc.corr_tol(qrev, A, B, 4, sym.tobytes(), off, ln, maxlen, N, want)
+        packed = torch.cat([ops.compress(t(sym)), torch.zeros(64, dtype=torch.uint8, device=dev)])
+        out = torch.empty(ln.size, dtype=torch.float32, device=dev)
+        lutB = torch.cat([t(B).reshape(-1), torch.zeros(1, device=dev)])
+        keep = [t(off.astype(np.int64)), t(ln), t(qrev), t(A), lutB]
+        call("sseqs_db_prefilter_spans", ptr(packed), ptr(keep[0]), ptr(keep[1]), 0, ln.size, ptr(keep[2]), Lq,
+             ptr(keep[3]), ptr(keep[4]), 21, 4, N, maxlen, ptr(out), stream_of(dev))
+        assert (np.abs(out.cpu().numpy() - want) <= tol).all(), order
