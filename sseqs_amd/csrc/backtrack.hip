@@ -11,15 +11,10 @@
 // H == Iy -> left, stop at H == 0).  Those comparisons depend only on the
 // cell, so two bits per cell (the move) are stored instead of six bytes.
 //
-// One wave per target.  The query is processed in strips of 64 rows; lane l
-// owns row 64k+l+1 and handles column j at step j+l-1, receiving H, Ix and the
-// target residue of the cell above from lane l-1 through one DPP wave shift
-// per step (a systolic anti-diagonal sweep).  The strip's last row is kept in
-// LDS for the next strip.  The 64 moves of one step are two 64-bit ballots,
-// stored as one 16-byte record: record (k, s) holds the moves of cells
-// (64k+l+1, s-l+1), l = 0..63.  End cell: the first cell in row-major order
-// that holds the maximum (sseqs/sw.py:620-637); the wave then follows the
-// moves through windows of 128 records staged in LDS.
+// One wave per target sweeps anti-diagonals of query strips (one row per lane
+// in k_backtrack_global, two in k_backtrack) and then follows the moves from
+// the end cell, the first cell in row-major order that holds the maximum
+// (sseqs/sw.py:620-637).
 #include "common.h"
 
 namespace sseqs {
@@ -160,63 +155,78 @@ __global__ __launch_bounds__(64) void k_backtrack_global(
     inf[5] = best;
 }
 
-__device__ inline int dpp_shr1(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
-}
-// wave_shr:1 with bound_ctrl: lane 0 reads 0 (callers replace lane 0's value)
-__device__ inline uint32_t dpp_shr1u(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x138, 0xf, 0xf, true);
-}
-
 // Two 16-bit lanes per register: low half the strip's upper row of a lane,
 // high half its lower row.
 typedef short bt_i16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short bt_u16x2 __attribute__((ext_vector_type(2)));
 __device__ inline bt_i16x2 bt_v(uint32_t u) { return __builtin_bit_cast(bt_i16x2, u); }
 __device__ inline uint32_t bt_u(bt_i16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ inline bt_i16x2 bt_max(bt_i16x2 a, bt_i16x2 b) { return __builtin_elementwise_max(a, b); }
 
-constexpr int BT_WIN = 128;  // steps per traceback window (two 16-byte records each)
-// LDS bytes shared by the row buffer and the traceback window
-__host__ __device__ inline int bt_region_bytes(int tcap) {
-    const int rbb = 8 * (tcap > 0 ? tcap : 0), wb = BT_WIN * 32;
-    return ((rbb > wb ? rbb : wb) + 15) & ~15;
-}
+// Longest target of k_backtrack (16-bit cells and, past it, LDS); longer ones take
+// the 32-bit k_backtrack_global.
+constexpr int BT_MAX_T = 5416;
 constexpr uint32_t BT_NEG2 = 0xC000C000u;  // BT_NEG in both halves
+constexpr int BT_LETTERS = 22;             // 20 residues, 20 any other letter, 21 outside the target
+constexpr int BT_PAD = 21;
+constexpr int BT_TAG_MAX_LEN = 744;   // 4 * 11 * 744 + 3 < 2^15
+constexpr int BT_TAG_MAX_GAP = 1024;  // gap parameters of the tagged cells (4 * 1024 above BT_NEG)
+// Dynamic LDS of k_backtrack: score pairs | strip boundary | BLOSUM62 |
+// target codes.
+__host__ __device__ inline int bt_rb_words(int tcap) { return 128 + ((tcap + 7) & ~7) + 144; }
+__host__ __device__ inline int bt_lds_bytes(int tcap) {
+    return BT_LETTERS * 256 + 4 * bt_rb_words(tcap) + 400 + ((128 + tcap + 160 + 15) & ~15);
+}
 
-// Move records of target b start at uint4 2 * NS * (cell_off[b] / Lq + 128 b),
-// NS = ceil(Lq / 128) strips of T + 128 steps, two records per step.
+// Move words of target b start at byte 32 * NS * (cell_off[b] / Lq + 128 b),
+// NS = ceil(Lq / 128) strips of 32 * (T + 128) bytes.
 //
 // One wave per target.  The query is processed in strips of 128 rows; lane l
 // owns rows 128k + 2l + 1 (the "a" row, low halves) and 128k + 2l + 2 (the
 // "b" row, high halves) and at step s handles column s - 2l + 1 of its a row
-// and one column less of its b row, every cell update in packed 16-bit
-// arithmetic for both rows at once (DP values stay within +-22528 + the gap
-// parameters, so 16 bits are exact).  The a row takes H and Ix of the cell
-// above from lane l-1's b row through one DPP wave shift per step; the b row
-// takes them from the lane's own a row one step earlier.  The strip's last
-// row (lane 63's b row) is kept in LDS for the next strip.  A step's moves
-// are four 64-bit ballots (two per row), stored as two 16-byte records:
-// record 2 (k (T + 128) + s) + h holds the moves of the cells of row
-// 128k + 2l + 1 + h at column s - 2l + 1 - h, bit l.  End cell: the first
-// cell in row-major order that holds the maximum (sseqs/sw.py:620-637); the
-// wave then follows the moves through windows of 128 steps staged in LDS.
+// and one column less of its b row, both cells in packed 16-bit arithmetic.
+// The a row takes H and Ix of the cell above from lane l-1's b row through one
+// DPP wave shift per step, the b row from the lane's own a row one step
+// earlier.  Eight steps form a block: the strip's last row (lane 63's b row)
+// enters and leaves LDS, and the moves leave for memory, once per block.
 //
-// Dynamic LDS: one region for the row buffer (tcap x int2, the DP) and then
-// the traceback window (BT_WIN x 32 B) | BLOSUM 400 B | target residues tcap
-// B.  Sharing the region keeps a wave's LDS near 5 KB for 500-residue
-// targets, so that eight waves fit a SIMD to hide each step's latency.
+// The kernel is bound by the instructions of one step, few waves being in
+// flight (one per target), so a step does as little as the two cells allow:
+// * Scores: tab[letter][lane] holds the scores of both rows of a lane against
+//   a letter, written once per strip, so a step reads one word without bank
+//   conflicts, a block ahead (the target is known; only H is a recurrence).
+// * Moves (TAG): cells hold 4 times the score plus, in the two low bits, the
+//   move's rank 3 stop (0), 2 diagonal, 1 up, 0 left, and the maximum picks
+//   value and move at once, with the ties of the definition.  A lane keeps
+//   the bits of eight steps of both rows in one word and the wave stores 256
+//   contiguous bytes per block (word 64 (s / 8) + 63 - l of the strip: the
+//   last, partial block holds cells only of the last lanes, so that its words
+//   end within the strip's bytes).
+// * Borders (TAG): columns outside the target and rows outside the query score
+//   BT_NEG.  With gap parameters >= 0 such cells hold 0 before the target and
+//   never more than the first valid cell of their value after it, and Iy = -o
+//   in column 0 gives column 1 the value of the border, so no cell is masked.
+// Without TAG (16 bits do not hold 4 x the scores, or odd gap parameters)
+// cells are masked and the moves come from comparisons.  4096 homologs at 200
+// residues: 927 -> 289 us against a wave with four ballots, masks and byte reads
+// per step.
+//
+// End cell: the first cell in row-major order that holds the maximum
+// (sseqs/sw.py:620-637).  Traceback: lane x reads the move of the cell x
+// diagonal steps back, so one round takes the whole run of diagonal moves
+// and the gap move that ends it.
 // Targets longer than tcap are rejected (info all -2).
+template <bool TAG>
 __global__ __launch_bounds__(64) void k_backtrack(
     const uint8_t* __restrict__ query, int Lq, const uint8_t* __restrict__ targets,
     const int64_t* __restrict__ t_off, const int32_t* __restrict__ t_len,
     const int64_t* __restrict__ cell_off, int go, int ge, int A, uint8_t* __restrict__ out_q,
-    uint8_t* __restrict__ out_t, int32_t* __restrict__ info, uint4* __restrict__ recs_all,
+    uint8_t* __restrict__ out_t, int32_t* __restrict__ info, uint32_t* __restrict__ moves_all,
     int tcap, Blosum bl) {
     extern __shared__ __align__(16) uint8_t smem[];
-    uint4* win = reinterpret_cast<uint4*>(smem);
-    int2* rb = reinterpret_cast<int2*>(smem);
-    const int region = bt_region_bytes(tcap);
-    int8_t* s_bl = reinterpret_cast<int8_t*>(smem + region);
+    uint32_t* tab = reinterpret_cast<uint32_t*>(smem);
+    uint32_t* rb = tab + BT_LETTERS * 64;
+    int8_t* s_bl = reinterpret_cast<int8_t*>(rb + bt_rb_words(tcap));
     uint8_t* tq = reinterpret_cast<uint8_t*>(s_bl + 400);
     const int lane = threadIdx.x;
     const int b = blockIdx.x;
@@ -226,17 +236,26 @@ __global__ __launch_bounds__(64) void k_backtrack(
         if (lane < 6) inf[lane] = -2;
         return;
     }
+    constexpr int SC = TAG ? 4 : 1;
+    constexpr uint32_t XNEG = TAG ? 0xC001u : 0xC000u;
     for (int i = lane; i < 400; i += 64) s_bl[i] = bl.v[i];
     const uint8_t* tg = targets + t_off[b];
-    for (int j = lane; j < T; j += 64) tq[j] = (uint8_t)aa_index(tg[j]);
+    // codes of columns -127 .. T + 160; rb[128 + j - 1]: (H, Ix) of the row
+    // above the strip in column j, the border for the first strip
+    for (int j = lane; j < 128 + T + 160; j += 64)
+        tq[j] = j >= 128 && j < 128 + T ? (uint8_t)aa_index(tg[j - 128]) : (uint8_t)BT_PAD;
+    for (int j = lane; j < 128 + ((T + 7) & ~7) + 144; j += 64) rb[j] = XNEG;
     __syncthreads();
 
     const int NS = (Lq + 127) >> 7;
-    const int RS = T + 128;  // steps per strip
-    uint4* recs = recs_all + (Lq > 0 ? 2LL * NS * (cell_off[b] / Lq + 128LL * b) : 0);
-    const bt_i16x2 GO = bt_v((uint32_t)(uint16_t)go * 0x10001u);
-    const bt_i16x2 GE = bt_v((uint32_t)(uint16_t)ge * 0x10001u);
-    const bt_i16x2 ZERO = bt_v(0u);
+    const int RS = T + 128;
+    const int NB = (T + 127 + 7) >> 3;  // blocks of eight steps
+    uint32_t* moves = moves_all + (Lq > 0 ? 8LL * NS * (cell_off[b] / Lq + 128LL * b) : 0);
+    const bt_i16x2 GO = bt_v((uint32_t)(uint16_t)(SC * go) * 0x10001u);
+    const bt_i16x2 GE = bt_v((uint32_t)(uint16_t)(SC * ge) * 0x10001u);
+    const bt_i16x2 GOX = bt_v((uint32_t)(uint16_t)(SC * go - (TAG ? 1 : 0)) * 0x10001u);
+    const bt_i16x2 FLOOR = bt_v(TAG ? 0x00030003u : 0u);
+    const bt_i16x2 ONE = bt_v(0x00010001u);
     int best = 0, bi = 0, bj = 0;  // this lane's first maximum, in (row, column) order
     if (Lq > 0 && T > 0) {
         for (int k = 0; k < NS; ++k) {
@@ -244,98 +263,128 @@ __global__ __launch_bounds__(64) void k_backtrack(
             const bool oka = ia <= Lq, okb = ib <= Lq;
             const int qa = oka ? aa_index(query[ia - 1]) : 20;
             const int qb = okb ? aa_index(query[ib - 1]) : 20;
-            const int8_t* browa = s_bl + (qa < 20 ? qa : 0) * 20;
-            const int8_t* browb = s_bl + (qb < 20 ? qb : 0) * 20;
-            const bool resa = qa < 20, resb = qb < 20;
+#pragma unroll 2
+            for (int t = 0; t < BT_LETTERS; ++t) {
+                int va = qa < 20 && t < 20 ? (int)s_bl[qa * 20 + t] : -5;
+                int vb = qb < 20 && t < 20 ? (int)s_bl[qb * 20 + t] : -5;
+                va = TAG && (t == BT_PAD || !oka) ? BT_NEG : SC * va;
+                vb = TAG && (t == BT_PAD || !okb) ? BT_NEG : SC * vb;
+                const int rank = TAG ? 2 : 0;
+                tab[t * 64 + lane] = ((uint32_t)(va + rank) & 0xffffu) | ((uint32_t)(vb + rank) << 16);
+            }
+            __syncthreads();
             // state of both rows: H (the cell to the left, and what the next
             // lane sees above), Ix, Iy; the cell above-left (diagonal)
-            uint32_t H = 0, X = BT_NEG2, Y = BT_NEG2, diag = 0;
-            int bestA = 0, bjA = 0, bestB = 0, bjB = 0;
-            // Software pipeline: each step reads the next step's substitution
-            // scores and lane 0's inputs (the row above from rb, the target
-            // residue two steps ahead), so no LDS read sits in a step's chain.
-            // The a row's residue at step s+1 is lane l-1's b-row residue at
-            // step s; the b row's is the lane's own a-row residue at step s.
-            int2 r_next = k > 0 && T > 0 ? rb[0] : make_int2(0, BT_NEG);
-            int tA = lane == 0 && T > 0 ? (int)tq[0] : 20, tB = 20;
-            int t_next = T > 1 ? (int)tq[1] : 20;
-            int sa = (resa && tA < 20) ? (int)browa[tA] : -5;
-            int sb = (resb && tB < 20) ? (int)browb[tB] : -5;
-            const int steps = T + 127;
-            for (int s = 0; s < steps; ++s) {
-                const int ja = s - 2 * lane + 1, jb = ja - 1;
-                const int2 r = r_next;
-                const uint32_t sc = ((uint32_t)sa & 0xffffu) | ((uint32_t)sb << 16);
-                int tA_next = (int)dpp_shr1u((uint32_t)tB);
-                tA_next = lane == 0 ? t_next : tA_next;
-                const int tB_next = tA;
-                // unconditional in-range reads, then the select
-                const int ga = (int)browa[tA_next < 20 ? tA_next : 0];
-                const int gb = (int)browb[tB_next < 20 ? tB_next : 0];
-                const int sa_next = (resa && tA_next < 20) ? ga : -5;
-                const int sb_next = (resb && tB_next < 20) ? gb : -5;
-                const int sn = s + 1;  // lane 0's a-row column at step sn is sn + 1
-                const int2 rr = rb[sn < T ? sn : T - 1];
-                r_next = k > 0 && sn < T ? rr : make_int2(0, BT_NEG);
-                const int tt = (int)tq[s + 2 < T ? s + 2 : T - 1];
-                const int t_nn = s + 2 < T ? tt : 20;
-                // the cells above: the a row's from lane l-1's b row (lane 0:
-                // the previous strip's last row), the b row's from its a row
-                uint32_t hin = dpp_shr1u(H), xin = dpp_shr1u(X);
-                hin = lane == 0 ? (uint32_t)r.x << 16 : hin;
-                xin = lane == 0 ? (uint32_t)r.y << 16 : xin;
-                const uint32_t up = __builtin_amdgcn_alignbit(H, hin, 16);
-                const uint32_t upX = __builtin_amdgcn_alignbit(X, xin, 16);
-                const bool va = ja >= 1 && ja <= T && oka;
-                const bool vb = jb >= 1 && jb <= T && okb;
-                const bt_i16x2 m = bt_v(sc) + bt_v(diag);
-                const bt_i16x2 x = bt_max(bt_v(up) - GO, bt_v(upX) - GE);
-                const bt_i16x2 y = bt_max(bt_v(H) - GO, bt_v(Y) - GE);
-                const bt_i16x2 h = bt_max(bt_max(m, x), bt_max(y, ZERO));
-                // move: 0 stop (h == 0), 1 diagonal (h == m), 2 up (h == x), 3 left
-                const bool nza = h.x != 0, hma = h.x == m.x, hxa = h.x == x.x;
-                const bool nzb = h.y != 0, hmb = h.y == m.y, hxb = h.y == x.y;
-                const uint64_t p0a = __ballot(va && nza && (hma || !hxa));
-                const uint64_t p1a = __ballot(va && nza && !hma);
-                const uint64_t p0b = __ballot(vb && nzb && (hmb || !hxb));
-                const uint64_t p1b = __ballot(vb && nzb && !hmb);
-                if (lane == 0) {
-                    uint4* rec = recs + 2 * ((int64_t)k * RS + s);
-                    rec[0] = make_uint4((uint32_t)p0a, (uint32_t)(p0a >> 32), (uint32_t)p1a,
-                                        (uint32_t)(p1a >> 32));
-                    rec[1] = make_uint4((uint32_t)p0b, (uint32_t)(p0b >> 32), (uint32_t)p1b,
-                                        (uint32_t)(p1b >> 32));
+            uint32_t H = 0, X = XNEG * 0x10001u, Y = BT_NEG2, diag = 0;
+            uint32_t bv = 0, bs = 0;  // both rows' maxima and the steps they were reached at
+            const uint8_t* tl = tq + 128 - 2 * lane;  // code of step s's a-row column
+            // the code c of a step gives byte address 256 c + 4 lane of tab
+            const uint32_t lane4 = 4u * (uint32_t)lane;
+            uint32_t P[8], L[4], R[8];
+            uint32_t last = 0;  // score pair of the previous step
+#define BT_LETTER_LOAD(q)                                                                        \
+    do {                                                                                         \
+        _Pragma("unroll") for (int u = 0; u < 4; ++u) L[u] =                                     \
+            *reinterpret_cast<const uint16_t*>(tl + 8 * (q) + 2 * u);                            \
+    } while (0)
+#define BT_SCORE_LOAD(dst)                                                                       \
+    do {                                                                                         \
+        _Pragma("unroll") for (int u = 0; u < 8; ++u) dst[u] = *reinterpret_cast<const uint32_t*>( \
+            smem + __builtin_amdgcn_perm(L[u >> 1], lane4, u & 1 ? 0x0c0c0500u : 0x0c0c0400u));  \
+    } while (0)
+#define BT_ROW_LOAD(dst, q)                                                                      \
+    do {                                                                                         \
+        const uint4 r0 = *reinterpret_cast<const uint4*>(rb + 128 + 8 * (q));                    \
+        const uint4 r1 = *reinterpret_cast<const uint4*>(rb + 132 + 8 * (q));                    \
+        dst[0] = r0.x, dst[1] = r0.y, dst[2] = r0.z, dst[3] = r0.w;                              \
+        dst[4] = r1.x, dst[5] = r1.y, dst[6] = r1.z, dst[7] = r1.w;                              \
+    } while (0)
+            BT_LETTER_LOAD(0);
+            BT_SCORE_LOAD(P);
+            BT_LETTER_LOAD(1);
+            BT_ROW_LOAD(R, 0);
+            uint32_t* mv = moves + (int64_t)k * RS * 8 + 63 - lane;
+            for (int q = 0; q < NB; ++q) {
+                uint32_t Pn[8], Rn[8], O[8], acc = 0;
+                BT_SCORE_LOAD(Pn);
+                BT_LETTER_LOAD(q + 2);
+                BT_ROW_LOAD(Rn, q + 1);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const uint32_t sc = (P[u] & 0xffffu) | (last & 0xffff0000u);
+                    last = P[u];
+                    // the cells above: the a row's from lane l-1's b row (lane 0:
+                    // the previous strip's last row), the b row's from its a row
+                    const uint32_t hin = (uint32_t)__builtin_amdgcn_update_dpp(
+                        (int)R[u], (int)H, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+                    const uint32_t xin = (uint32_t)__builtin_amdgcn_update_dpp(
+                        (int)(R[u] << 16), (int)X, 0x138, 0xf, 0xf, false);
+                    const uint32_t up = __builtin_amdgcn_alignbit(H, hin, 16);
+                    const uint32_t upX = __builtin_amdgcn_alignbit(X, xin, 16);
+                    const bt_i16x2 m = bt_v(sc) + bt_v(diag);
+                    const bt_i16x2 x = bt_max(bt_v(up) - GOX, bt_v(upX) - GE);
+                    const bt_i16x2 y = bt_max(bt_v(H) - GO, bt_v(Y) - GE);
+                    const bt_i16x2 h = bt_max(bt_max(m, bt_max(y, FLOOR)), x);
+                    const int s = 8 * q + u;
+                    if constexpr (TAG) {
+                        acc = (acc << 2) | (bt_u(h) & 0x00030003u);
+                        H = bt_u(h) & 0xfffcfffcu;
+                        X = bt_u(x);
+                        Y = bt_u(y);
+                    } else {
+                        const auto ne = [&](bt_i16x2 v) {  // 1 where h differs
+                            const bt_u16x2 d = __builtin_bit_cast(bt_u16x2, h) -
+                                               __builtin_bit_cast(bt_u16x2, v);
+                            return __builtin_bit_cast(bt_i16x2, __builtin_elementwise_min(
+                                d, __builtin_bit_cast(bt_u16x2, ONE)));
+                        };
+                        const bt_i16x2 nm = ne(m), nx = ne(x), nz = ne(bt_v(0u));
+                        const bt_i16x2 code = bt_v(0x00030003u) - nz * (ONE + nm + nm * nx);
+                        acc = (acc << 2) | bt_u(code);
+                        // rows update only on their valid cells; before a row starts
+                        // its state stays (H 0, Ix and Iy BT_NEG), the left boundary
+                        const int ja = s - 2 * lane + 1, jb = ja - 1;
+                        const uint32_t msk = (ja >= 1 && ja <= T && oka ? 0xffffu : 0u) |
+                                             (jb >= 1 && jb <= T && okb ? 0xffff0000u : 0u);
+                        H = (bt_u(h) & msk) | (H & ~msk);
+                        X = (bt_u(x) & msk) | (X & ~msk);
+                        Y = (bt_u(y) & msk) | (Y & ~msk);
+                    }
+                    O[u] = __builtin_amdgcn_perm(H, X, 0x07060302u);
+                    const bt_i16x2 nb = bt_max(bt_v(bv), bt_v(H));
+                    uint32_t better;  // 0xffff in the halves that grew (opaque: as a
+                                      // compare it becomes two per half)
+                    asm("v_pk_ashrrev_i16 %0, 15, %1 op_sel_hi:[0,1]" : "=v"(better) : "v"(bt_v(bv) - nb));
+                    bs = (better & ((uint32_t)s * 0x10001u)) | (~better & bs);
+                    bv = bt_u(nb);
+                    diag = up;
                 }
-                const bool betterA = va && h.x > bestA, betterB = vb && h.y > bestB;
-                bestA = betterA ? h.x : bestA;
-                bjA = betterA ? ja : bjA;
-                bestB = betterB ? h.y : bestB;
-                bjB = betterB ? jb : bjB;
-                // rows update only on their valid cells; before a row starts its
-                // state stays (H 0, Ix and Iy BT_NEG), the left boundary
-                const uint32_t msk = (va ? 0xffffu : 0u) | (vb ? 0xffff0000u : 0u);
-                H = (bt_u(h) & msk) | (H & ~msk);
-                X = (bt_u(x) & msk) | (X & ~msk);
-                Y = (bt_u(y) & msk) | (Y & ~msk);
-                if (lane == 63 && vb) rb[jb - 1] = make_int2(h.y, x.y);
-                diag = up;
-                tA = tA_next;
-                tB = tB_next;
-                sa = sa_next;
-                sb = sb_next;
-                t_next = t_nn;
+                if (64 * q + 63 - lane < 8 * RS) mv[64 * q] = acc;
+                if (lane == 63) {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) rb[8 * q + u + 1] = O[u];
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    P[u] = Pn[u];
+                    R[u] = Rn[u];
+                }
             }
+#undef BT_LETTER_LOAD
+#undef BT_SCORE_LOAD
+#undef BT_ROW_LOAD
             // the lane's rows in order: a strictly larger value replaces, so
             // ties keep the earlier row (and the earlier column within a row)
+            const int bestA = (int)(bv & 0xffffu) / SC, bestB = (int)(bv >> 16) / SC;
             if (bestA > best) {
                 best = bestA;
                 bi = ia;
-                bj = bjA;
+                bj = (int)(bs & 0xffffu) - 2 * lane + 1;
             }
             if (bestB > best) {
                 best = bestB;
                 bi = ib;
-                bj = bjB;
+                bj = (int)(bs >> 16) - 2 * lane;
             }
             __syncthreads();  // the strip's last row is in rb
         }
@@ -351,52 +400,39 @@ __global__ __launch_bounds__(64) void k_backtrack(
                 bj = oj;
             }
         }
-        __threadfence();  // the move records are visible to the loads below
+        __threadfence();  // the moves are visible to the loads below
     }
-    // traceback: every lane follows the same path; lane 0 writes the rows
     int n = 0, ci = -1, cj = -1, ei = -1, ej = -1;
     if (best > 0) {
         ei = bi;
         ej = bj;
         int i = ei, j = ej;
-        int w = A - 1;
-        int wk = -1, wlo = 0;  // strip and first step held in the window
-        while (i > 0 && j > 0 && w >= 0) {
-            const int k = (i - 1) >> 7, rr = (i - 1) & 127, l = rr >> 1, hh = rr & 1;
-            const int st = j - 1 + 2 * l + hh;
-            if (k != wk || st < wlo || st >= wlo + BT_WIN) {
-                wk = k;
-                wlo = max(0, st - (BT_WIN - 1));
-                __syncthreads();
-                for (int t = lane; t < 2 * BT_WIN; t += 64)
-                    if (wlo + (t >> 1) < RS) win[t] = recs[2 * ((int64_t)k * RS + wlo) + t];
-                __syncthreads();
+        while (i > 0 && j > 0 && n < A) {
+            // the cell `lane` diagonal steps back
+            const int ix = i - lane, jx = j - lane;
+            int code = 3;
+            if (ix > 0 && jx > 0) {
+                const int k = (ix - 1) >> 7, r = (ix - 1) & 127;
+                const int st = jx - 1 + r;
+                const uint32_t v = moves[(int64_t)k * RS * 8 + 64 * (st >> 3) + 63 - (r >> 1)];
+                code = (int)(v >> (16 * (r & 1) + 2 * (7 - (st & 7)))) & 3;
             }
-            const uint4 r = win[2 * (st - wlo) + hh];
-            const uint32_t w0 = l < 32 ? r.x : r.y, w1 = l < 32 ? r.z : r.w;
-            const int d = (int)((w0 >> (l & 31)) & 1u) | (int)(((w1 >> (l & 31)) & 1u) << 1);
-            if (d == 0) break;
-            uint8_t qc, tc;
-            if (d == 1) {
-                qc = query[i - 1];
-                tc = tg[j - 1];
-                --i;
-                --j;
-            } else if (d == 2) {
-                qc = query[i - 1];
-                tc = '-';
-                --i;
-            } else {
-                qc = '-';
-                tc = tg[j - 1];
-                --j;
+            const uint64_t stop = __ballot(code != 2);
+            const int run = stop ? __builtin_ctzll(stop) : 64;
+            const int end = run < 64 ? __builtin_amdgcn_readlane(code, run) : 2;
+            // columns written this round: the run, then the gap move
+            const int cols = min(run + (end < 2 ? 1 : 0), A - n);
+            if (lane < cols) {
+                const int64_t w = (int64_t)b * A + A - 1 - n - lane;
+                const bool gap = lane == run;
+                out_q[w] = gap && end == 0 ? (uint8_t)'-' : query[ix - 1];
+                out_t[w] = gap && end == 1 ? (uint8_t)'-' : tg[jx - 1];
             }
-            if (lane == 0) {
-                out_q[(int64_t)b * A + w] = qc;
-                out_t[(int64_t)b * A + w] = tc;
-            }
-            --w;
-            ++n;
+            const int dg = min(run, cols), gp = cols - dg;
+            i -= dg + (end == 1 ? gp : 0);
+            j -= dg + (end == 0 ? gp : 0);
+            n += cols;
+            if (end == 3) break;
         }
         ci = i;
         cj = j;
@@ -422,7 +458,7 @@ __global__ __launch_bounds__(64) void k_backtrack(
 
 using namespace sseqs;
 
-// Workspace: the move records of k_backtrack or, for targets too long for
+// Workspace: the move words of k_backtrack or, for targets too long for
 // its LDS row buffer, the direction bytes + row buffer of k_backtrack_global.
 static size_t bt_records_bytes(int query_len, int64_t total_cells, int B) {
     if (query_len <= 0) return 0;
@@ -452,13 +488,13 @@ extern "C" int sseqs_backtrack(const uint8_t* query, int query_len, const uint8_
         return fail(-2, "backtrack: workspace too small");
     // targets are at most max_align - query_len - 1 long (the documented bound)
     const int tcap = max_align - query_len - 1;
-    const size_t lds = ((size_t)bt_region_bytes(tcap) + 400 + (size_t)(tcap > 0 ? tcap : 0) + 15) &
-                       ~(size_t)15;
-    if (tcap >= 1 && lds <= 48 * 1024) {
-        hipLaunchKernelGGL(k_backtrack, dim3((unsigned)B), dim3(64), lds, stream, query,
-                           query_len, targets, t_off, t_len, cell_off, gap_open, gap_extend,
-                           max_align, out_q, out_t, info, static_cast<uint4*>(ws), tcap,
-                           blosum62());
+    if (tcap >= 1 && tcap <= BT_MAX_T) {
+        const bool tag = (query_len < tcap ? query_len : tcap) <= BT_TAG_MAX_LEN && gap_open >= 0 &&
+                         gap_open <= BT_TAG_MAX_GAP && gap_extend >= 0 && gap_extend <= BT_TAG_MAX_GAP;
+        hipLaunchKernelGGL(tag ? k_backtrack<true> : k_backtrack<false>, dim3((unsigned)B), dim3(64),
+                           (size_t)bt_lds_bytes(tcap), stream, query, query_len, targets, t_off, t_len,
+                           cell_off, gap_open, gap_extend, max_align, out_q, out_t, info,
+                           static_cast<uint32_t*>(ws), tcap, blosum62());
         return check_launch("backtrack");
     }
     uint8_t* dirs = static_cast<uint8_t*>(ws);

@@ -28,15 +28,25 @@ inline Blosum blosum62() {
 
 // ASCII -> 0..19 residue index, 20 otherwise (the CUDA SW kernels score any
 // non-residue as -4, sseqs/sw.cu:128-130).
-__host__ __device__ inline int aa_index(uint32_t c) {
-    switch (c) {
-    case 'A': return 0;  case 'R': return 1;  case 'N': return 2;  case 'D': return 3;
-    case 'C': return 4;  case 'Q': return 5;  case 'E': return 6;  case 'G': return 7;
-    case 'H': return 8;  case 'I': return 9;  case 'L': return 10; case 'K': return 11;
-    case 'M': return 12; case 'F': return 13; case 'P': return 14; case 'S': return 15;
-    case 'T': return 16; case 'W': return 17; case 'Y': return 18; case 'V': return 19;
-    default: return 20;
+// Letters A-L, M-X and Y-Z are five bits each of three constants: a dozen
+// instructions without a branch, where a switch over the letters was some
+// hundred with a divergent branch for most.
+constexpr uint64_t aa_pack(int first) {
+    uint64_t v = 0;
+    for (int l = 0; l < 12; ++l) {
+        uint64_t code = 20;
+        for (int a = 0; a < 20; ++a)
+            if ("ARNDCQEGHILKMFPSTWYV"[a] == 'A' + first + l) code = (uint64_t)a;
+        v |= code << (5 * l);
     }
+    return v;
+}
+__host__ __device__ inline int aa_index(uint32_t c) {
+    constexpr uint64_t P0 = aa_pack(0), P1 = aa_pack(12), P2 = aa_pack(24);
+    const uint32_t l = c - 'A';
+    const uint64_t p = l < 12 ? P0 : (l < 24 ? P1 : P2);
+    const uint32_t i = l < 12 ? l : (l < 24 ? l - 12 : l - 24);
+    return l < 26 ? (int)((p >> (5 * (i & 15))) & 31u) : 20;
 }
 
 // Prefilter database code (sseqs/fft.cu:5-15): residues 0..19, X - * -> 20,

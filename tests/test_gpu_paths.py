@@ -146,3 +146,29 @@ def test_rank4_ring(orc, dev, N, Lq):
         call("sseqs_db_prefilter_spans", ptr(packed), ptr(keep[0]), ptr(keep[1]), 0, ln.size, ptr(keep[2]), Lq,
              ptr(keep[3]), ptr(keep[4]), 21, 4, N, maxlen, ptr(out), stream_of(dev))
         assert (np.abs(out.cpu().numpy() - want) <= tol).all(), order
+
+
+@pytest.mark.parametrize("Lq", [1, 2, 127, 128, 129, 255, 257, 744, 745, 900])
+def test_backtrack_edges(orc, dev, Lq):
+    """Alignments around the strips of 128 query rows, the blocks of eight
+    steps and the lengths and gap parameters that choose tagged cells: related
+    targets with indels, unrelated ones, non-residues, empty ones and the
+    largest score there is."""
+    from sseqs_amd.sw import sw_affine_backtrack
+    announce(f"backtrack edges Lq={Lq}")
+    rng = np.random.default_rng(Lq)
+    query = rand_seq(rng, Lq, AA + "XB")
+    tg = ["W" * 3 + query[5:], query[: Lq // 2] + rand_seq(rng, 9) + query[Lq // 2 + 3:], "", "X" * 7]
+    for T in (1, 6, 7, 8, 9, 120, 121, 127, 128, 129, 136, 743, 744, 745, 800):
+        part = list(rand_seq(rng, T))
+        a = int(rng.integers(0, max(1, Lq - T // 2)))
+        piece = query[a: a + T // 2]
+        part[T // 4: T // 4 + len(piece)] = piece
+        tg.append("".join(part)[:T])
+    for q, targets, gaps in ((query, tg, ((11, 1), (0, 0), (1024, 1024), (1025, 3), (-1, 1))),
+                             ("W" * Lq, ["W" * 900, "W" * 744, "W" * 8], ((11, 1),)),
+                             (query, tg[:10], ((11, 1), (3, 0)))):
+        for o, e in gaps:
+            _, _, got = sw_affine_backtrack(q, targets, o, e)
+            for t, g in zip(targets, got):
+                assert g == orc.backtrack(q, t, o, e), (len(t), o, e)
