@@ -52,16 +52,34 @@ __device__ inline float gelu_grad(float x) {
 
 // ------------------------------------------------------------- conv GEMM --
 //
-// Block of 256 threads (4 waves) computes a 128 x BN tile of C; wave
-// (wm, wn) the 64 x BN/2 sub-tile, as 2 x BN/64 MFMA tiles of 32 x 32.
-// K advances 32 per stage: A (128 x 32) and Bt (BN x 32) tiles go through
-// LDS (rows padded to 40 elements), the next stage's global loads are
-// issued before the current stage's MFMAs.
+// A block computes 64 WM - 8 rows x BN columns of C, wave (wm, wn) the rows
+// 64 wm .. + 63 (the last wave's last eight are left out) x the BN / WN
+// columns of wn, as 2 x BN / (32 WN) MFMA tiles of 32 x 32.  The block's
+// 64 WM rows of A are read from memory once and stay in LDS for the nine
+// taps, which only shift the row that a lane reads; without the eight rows
+// that are left out they and two stages of Bt take half the LDS of a CU
+// exactly, so that two blocks share it and one's epilogue and first loads run
+// beside the other's products.  K goes by 32 columns of Bt at a time, in
+// order: the sums are those of a plain loop over K.  Bt is read two stages
+// ahead, into registers; the second half of a stage's operands leaves LDS
+// between the products of the first.  Rows of LDS hold their 16-byte pieces
+// at piece ^ (row mod 16) (A) and ^ (row / 2 mod 4) (Bt), so that neither the
+// row-wise stores nor the operand reads meet in a bank.
 //
 // MFMA 32x32x16 operands: lane (r = lane % 32, h = lane / 32) supplies
-// row r, elements 8h .. 8h+7 of K of both A and Bt; result element e of
-// lane (c = lane % 32, h) is row 8 * (e / 4) + 4 * h + (e % 4), column c.
-constexpr int GM = 128, GK = 32, GPAD = 40;
+// row r, elements 8h .. 8h+7 of K of both operands.  The weights are the
+// first operand: result element e of lane (c, h) is then column
+// 8 * (e / 4) + 4 * h + (e % 4) of C in row c, four consecutive columns to a
+// lane, which go in and out as 8 bytes.
+//
+// Bound by issue slots: the products take 40 % of them, GELU's tanh as many
+// again.  The three layers over 8.6 M rows 16.1 -> 12.3 ms (0.55 -> 0.72
+// PFLOP/s) against 128 x 128 tiles that read every tap's rows from memory;
+// the backward products of 312 k rows 761 -> 477 us.
+constexpr int GM = 128, GK = 32;  // granularity of M; columns of Bt of a stage
+// Wide blocks when they fill the 512 places of the chip (two a CU) once; with
+// fewer, small blocks spread the rows over more CUs.
+constexpr int64_t CONV_WIDE = 512;
 
 enum ConvEpi {
     EPI_FWD = 0,      // u = acc + bias; U = u (optional); Y = gelu(u) * mask
@@ -73,7 +91,8 @@ struct ConvArgs {
     const __bf16* A;     // A row p at A + (p - 4) * lda (rows -4 .. M + 3 readable)
     int lda;             // elements between consecutive rows of A (Cin or Cout)
     const __bf16* Bt;    // N rows of K
-    int M, N, K;
+    int64_t M;
+    int N, K;
     const float* bias;   // EPI_FWD
     const uint8_t* mask; // [M]
     __bf16* U;           // EPI_FWD: pre-activation out (may be null)
@@ -82,9 +101,166 @@ struct ConvArgs {
     float* Yf;           // EPI_BWD_F32
 };
 
-template <int BN, int EPI>
-__global__ __launch_bounds__(256) void k_conv_gemm(ConvArgs a) {
-    constexpr int NT = BN / 64;  // MFMA tiles per wave along N
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// CIN: lda, K = 9 CIN
+template <int CIN, int BN, int EPI, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_gemm(ConvArgs a) {
+    constexpr int NT = BN / (32 * WN);     // MFMA tiles of a wave along N
+    constexpr int TH = 64 * WM * WN, ROWS = 64 * WM, OUT = ROWS - 8;
+    constexpr int RB = 2 * CIN;            // bytes of a row of A
+    constexpr int PA = RB / 16;            // its 16-byte pieces
+    constexpr int SW = PA < 16 ? PA - 1 : 15;
+    constexpr int APT = ROWS * PA / TH, BPT = BN * 4 / TH;  // pieces per thread
+    constexpr int NST = 9 * CIN / GK;      // stages
+    __shared__ __align__(16) uint8_t sA[ROWS * RB];
+    __shared__ __align__(16) uint8_t sB[2][BN * 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int wm = w / WN, wn = w % WN;
+    const int r = lane & 31, h = lane >> 5;
+    // the blocks of one row tile are dealt to one XCD (block id mod 8), whose
+    // L2 then holds the tile's rows for all of them
+    const int nt = a.N / BN, slot = blockIdx.x >> 3;
+    const int64_t m0 = ((int64_t)(slot / nt) * 8 + (blockIdx.x & 7)) * OUT;
+    const int n0 = slot % nt * BN;
+    if (m0 >= a.M) return;
+
+    // Bt through registers: piece tid % 4 of rows tid / 4 + (TH / 4) x
+    const int brow = tid >> 2, bc = tid & 3;
+    const __bf16* gB = a.Bt + (int64_t)(n0 + brow) * a.K + 8 * bc;
+    uint8_t* lB = &sB[0][0] + brow * 64 + 16 * (bc ^ ((brow >> 1) & 3));
+    u32x4 rb[2][BPT];
+#define CONV_LOAD_B(set, st)                                                               \
+    _Pragma("unroll") for (int x = 0; x < BPT; ++x) rb[set][x] =                           \
+        *reinterpret_cast<const u32x4*>(gB + (int64_t)(TH / 4 * x) * a.K + (st) * GK)
+    // TH / 4 is a multiple of 8, so the swizzle is that of brow
+#define CONV_STORE_B(set)                                                                  \
+    _Pragma("unroll") for (int x = 0; x < BPT; ++x) *reinterpret_cast<u32x4*>(             \
+        lB + (set) * (BN * 64) + TH / 4 * x * 64) = rb[set][x]
+    {
+        u32x4 ra[APT];
+        const int prow = tid / PA, pc = tid % PA;
+#pragma unroll
+        for (int x = 0; x < APT; ++x) {  // rows m0 - 4 .. , none past M + 3
+            int64_t row = m0 - 4 + prow + TH / PA * x;
+            row = row < a.M + 3 ? row : a.M + 3;
+            ra[x] = *reinterpret_cast<const u32x4*>(a.A + row * CIN + 8 * pc);
+        }
+        CONV_LOAD_B(0, 0);
+        CONV_LOAD_B(1, 1);
+#pragma unroll
+        for (int x = 0; x < APT; ++x) {
+            const int row = prow + TH / PA * x;
+            *reinterpret_cast<u32x4*>(sA + row * RB + 16 * (pc ^ (row & SW))) = ra[x];
+        }
+        CONV_STORE_B(0);
+    }
+    f32x16 acc[2][NT];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    __syncthreads();
+
+    const uint8_t* fB = &sB[0][0] + (BN / WN * wn + r) * 64 + 16 * (h ^ ((r >> 1) & 3));
+    const int boff = (int)(fB - &sB[0][0]);
+#pragma unroll 1
+    for (int t = 0; t < 9; ++t) {
+        const int row = 64 * wm + r + t;  // past the block's rows: those left out
+        int aoff[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            aoff[i] = ((row + 32 * i) & (ROWS - 1)) * RB + 16 * (h ^ (row & SW));
+#pragma unroll
+        for (int c = 0; c < CIN / GK; ++c) {
+            const int st = t * (CIN / GK) + c;
+            bf16x8 fa[2][2], fb[2][NT];
+#define CONV_LOAD_F(s)                                                                     \
+    do {                                                                                   \
+        _Pragma("unroll") for (int i = 0; i < 2; ++i) fa[s][i] =                           \
+            *reinterpret_cast<const bf16x8*>(sA + (aoff[i] ^ (64 * c + 32 * s)));          \
+        _Pragma("unroll") for (int j = 0; j < NT; ++j) fb[s][j] =                          \
+            *reinterpret_cast<const bf16x8*>(&sB[0][0] + (c & 1) * (BN * 64) +             \
+                                             (boff ^ (32 * s)) + 2048 * j);                \
+    } while (0)
+            CONV_LOAD_F(0);
+            // rb[c & 1] went to LDS a stage ago; the last stages read stage NST - 1 again
+            CONV_LOAD_B(c & 1, st + 2 < NST ? st + 2 : NST - 1);
+            __builtin_amdgcn_sched_barrier(0);  // these loads are on their way first
+            CONV_LOAD_F(1);
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[s][j], fa[s][i],
+                                                                            acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int x = 0; x < 2 + NT; ++x) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            CONV_STORE_B((c + 1) & 1);  // stage st + 1
+            __syncthreads();
+        }
+    }
+#undef CONV_LOAD_B
+#undef CONV_STORE_B
+#undef CONV_LOAD_F
+
+    // epilogue: lane (r, h) holds columns 32 j + 8 q + 4 h .. + 3 of its row
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int mr = 64 * wm + 32 * i + r;
+        const int64_t m = m0 + mr;
+        if (mr >= OUT || m >= a.M) continue;
+        const float mk = a.mask[m] ? 1.f : 0.f;
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int n = n0 + BN / WN * wn + 32 * j + 8 * q + 4 * h;
+                const int64_t o = m * a.N + n;
+                if constexpr (EPI == EPI_FWD) {
+                    const float4 bias = *reinterpret_cast<const float4*>(a.bias + n);
+                    const float bb[4] = {bias.x, bias.y, bias.z, bias.w};
+                    bf16x4 u, y;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        const float v = acc[i][j][4 * q + x] + bb[x];
+                        u[x] = f2bf(v);
+                        y[x] = f2bf(gelu(v) * mk);
+                    }
+                    if (a.U) *reinterpret_cast<bf16x4*>(a.U + o) = u;
+                    *reinterpret_cast<bf16x4*>(a.Y + o) = y;
+                } else if constexpr (EPI == EPI_BWD_GELU) {
+                    const bf16x4 up = *reinterpret_cast<const bf16x4*>(a.Uprev + o);
+                    bf16x4 y;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        y[x] = f2bf(acc[i][j][4 * q + x] * gelu_grad(bf2f(up[x])) * mk);
+                    *reinterpret_cast<bf16x4*>(a.Y + o) = y;
+                } else {
+                    *reinterpret_cast<float4*>(a.Yf + o) =
+                        make_float4(acc[i][j][4 * q] * mk, acc[i][j][4 * q + 1] * mk,
+                                    acc[i][j][4 * q + 2] * mk, acc[i][j][4 * q + 3] * mk);
+                }
+            }
+    }
+}
+
+// Any K and row stride (windows that are not nine whole rows), any alignment
+// of the outputs: 128 x 64 tiles, wave (wm, wn) the 64 x 32 share, both
+// operands' 32 columns of K through LDS (rows padded to 40 elements) per stage.
+constexpr int GPAD = 40;
+template <int EPI>
+__global__ __launch_bounds__(256) void k_conv_any(ConvArgs a) {
+    constexpr int BN = 64, NT = 1;
     __shared__ __align__(16) __bf16 sA[2][GM * GPAD];
     __shared__ __align__(16) __bf16 sB[2][BN * GPAD];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -99,21 +275,18 @@ __global__ __launch_bounds__(256) void k_conv_gemm(ConvArgs a) {
     const __bf16* gA0 = a.A + (m0 + crow - 4) * a.lda + ccol;
     const __bf16* gA1 = gA0 + (int64_t)64 * a.lda;
     const __bf16* gB0 = a.Bt + (int64_t)(n0 + crow) * a.K + ccol;
-    const __bf16* gB1 = gB0 + (int64_t)64 * a.K;
-    uint4 ra0, ra1, rb0, rb1 = make_uint4(0, 0, 0, 0);
+    uint4 ra0, ra1, rb0;
 #define CONV_GLOAD(k0)                                                     \
     do {                                                                   \
         ra0 = *reinterpret_cast<const uint4*>(gA0 + (k0));                 \
         ra1 = *reinterpret_cast<const uint4*>(gA1 + (k0));                 \
         rb0 = *reinterpret_cast<const uint4*>(gB0 + (k0));                 \
-        if (BN == 128) rb1 = *reinterpret_cast<const uint4*>(gB1 + (k0));  \
     } while (0)
 #define CONV_SSTORE(b)                                                                   \
     do {                                                                                 \
         *reinterpret_cast<uint4*>(&sA[b][crow * GPAD + ccol]) = ra0;                     \
         *reinterpret_cast<uint4*>(&sA[b][(crow + 64) * GPAD + ccol]) = ra1;              \
         *reinterpret_cast<uint4*>(&sB[b][crow * GPAD + ccol]) = rb0;                     \
-        if (BN == 128) *reinterpret_cast<uint4*>(&sB[b][(crow + 64) * GPAD + ccol]) = rb1; \
     } while (0)
 
     f32x16 acc[2][NT];
@@ -770,6 +943,40 @@ using namespace sseqs;
 
 // ---------------------------------------------------------------- C ABI --
 
+template <int CIN, int BN, int EPI, int WM, int WN>
+static void launch_conv_tiles(const ConvArgs& a, hipStream_t stream) {
+    const int64_t slots = ceil_div(ceil_div(a.M, 64 * WM - 8), 8) * (a.N / BN);
+    hipLaunchKernelGGL((k_conv_gemm<CIN, BN, EPI, WM, WN>), dim3((unsigned)(8 * slots)),
+                       dim3(64 * WM * WN), 0, stream, a);
+}
+
+template <int CIN, int EPI>
+static void launch_conv_cin(const ConvArgs& a, hipStream_t stream) {
+    constexpr int WM = CIN == 256 ? 2 : 4, WN = CIN == 256 ? 2 : 1;  // A: at most 64 KiB
+    const int64_t rows = a.M / (64 * WM - 8);
+    if (a.N % 128 == 0 && rows * (a.N / 128) >= CONV_WIDE)
+        launch_conv_tiles<CIN, 128, EPI, WM, WN>(a, stream);
+    else if (CIN != 256 && rows * (a.N / 64) >= CONV_WIDE)
+        launch_conv_tiles<CIN, 64, EPI, WM, WN>(a, stream);
+    else
+        launch_conv_tiles<CIN, 64, EPI, 2, CIN == 256 ? 2 : 1>(a, stream);
+}
+
+template <int EPI>
+static void launch_conv(const ConvArgs& a, hipStream_t stream) {
+    // nine whole rows of the encoder's widths, and outputs that take 8- and
+    // 16-byte accesses
+    const uintptr_t out = (uintptr_t)a.U | (uintptr_t)a.Y | (uintptr_t)a.Uprev;
+    const uintptr_t wide = (uintptr_t)a.bias | (uintptr_t)a.Yf;
+    const bool whole = a.K == 9 * a.lda && !(out & 7) && !(wide & 15);
+    if (whole && a.lda == 64) launch_conv_cin<64, EPI>(a, stream);
+    else if (whole && a.lda == 128) launch_conv_cin<128, EPI>(a, stream);
+    else if (whole && a.lda == 256) launch_conv_cin<256, EPI>(a, stream);
+    else
+        hipLaunchKernelGGL((k_conv_any<EPI>), dim3((unsigned)(a.M / GM), (unsigned)(a.N / 64)),
+                           dim3(256), 0, stream, a);
+}
+
 extern "C" int sseqs_enc_conv(const void* A, int lda, const void* Bt, int64_t M, int N, int K,
                               const float* bias, const uint8_t* mask, void* U, void* Y,
                               const void* Uprev, float* Yf, int epi, hipStream_t stream) {
@@ -777,30 +984,17 @@ extern "C" int sseqs_enc_conv(const void* A, int lda, const void* Bt, int64_t M,
     if (K <= 0 || K % GK) return fail(-1, "enc_conv: K must be a positive multiple of 32");
     if (N % 64) return fail(-1, "enc_conv: N must be a multiple of 64");
     if (M / GM > 0x7fffffffLL) return fail(-1, "enc_conv: too many rows");
-    ConvArgs a{static_cast<const __bf16*>(A), lda, static_cast<const __bf16*>(Bt), (int)0, N, K,
-               bias, mask, static_cast<__bf16*>(U), static_cast<__bf16*>(Y),
-               static_cast<const __bf16*>(Uprev), Yf};
-    a.M = (int)(M < 0x7fffffffLL ? M : 0x7fffffffLL);
-    const bool wide = N % 128 == 0;
-    const dim3 grid((unsigned)(M / GM), (unsigned)(N / (wide ? 128 : 64)));
+    if (epi == EPI_FWD && (!Y || !bias)) return fail(-1, "enc_conv: forward needs Y and bias");
+    if (epi == EPI_BWD_GELU && (!Y || !Uprev)) return fail(-1, "enc_conv: backward needs Y and Uprev");
+    if (epi == EPI_BWD_F32 && !Yf) return fail(-1, "enc_conv: backward to the input needs Yf");
+    const ConvArgs a{static_cast<const __bf16*>(A), lda, static_cast<const __bf16*>(Bt), M, N, K,
+                     bias, mask, static_cast<__bf16*>(U), static_cast<__bf16*>(Y),
+                     static_cast<const __bf16*>(Uprev), Yf};
     switch (epi) {
-    case EPI_FWD:
-        if (!Y || !bias) return fail(-1, "enc_conv: forward needs Y and bias");
-        if (wide) hipLaunchKernelGGL((k_conv_gemm<128, EPI_FWD>), grid, dim3(256), 0, stream, a);
-        else hipLaunchKernelGGL((k_conv_gemm<64, EPI_FWD>), grid, dim3(256), 0, stream, a);
-        break;
-    case EPI_BWD_GELU:
-        if (!Y || !Uprev) return fail(-1, "enc_conv: backward needs Y and Uprev");
-        if (wide) hipLaunchKernelGGL((k_conv_gemm<128, EPI_BWD_GELU>), grid, dim3(256), 0, stream, a);
-        else hipLaunchKernelGGL((k_conv_gemm<64, EPI_BWD_GELU>), grid, dim3(256), 0, stream, a);
-        break;
-    case EPI_BWD_F32:
-        if (!Yf) return fail(-1, "enc_conv: backward to the input needs Yf");
-        if (wide) hipLaunchKernelGGL((k_conv_gemm<128, EPI_BWD_F32>), grid, dim3(256), 0, stream, a);
-        else hipLaunchKernelGGL((k_conv_gemm<64, EPI_BWD_F32>), grid, dim3(256), 0, stream, a);
-        break;
-    default:
-        return fail(-1, "enc_conv: unknown epilogue");
+    case EPI_FWD: launch_conv<EPI_FWD>(a, stream); break;
+    case EPI_BWD_GELU: launch_conv<EPI_BWD_GELU>(a, stream); break;
+    case EPI_BWD_F32: launch_conv<EPI_BWD_F32>(a, stream); break;
+    default: return fail(-1, "enc_conv: unknown epilogue");
     }
     return check_launch("enc_conv");
 }

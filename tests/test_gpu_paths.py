@@ -172,3 +172,53 @@ def test_backtrack_edges(orc, dev, Lq):
             _, _, got = sw_affine_backtrack(q, targets, o, e)
             for t, g in zip(targets, got):
                 assert g == orc.backtrack(q, t, o, e), (len(t), o, e)
+
+
+@pytest.mark.parametrize("M,cin,N", [(128, 64, 128), (256, 128, 64), (640, 256, 128), (128 * 251, 128, 256),
+                                     (128 * 497, 64, 64), (128 * 481, 256, 128), (128 * 995, 128, 128)])
+def test_encoder_conv_tiles(dev, M, cin, N):
+    """The convolution's tiled kernels equal its general one (reached by an
+    output that is not aligned) bit for bit, for every epilogue, around the
+    row counts of their tiles and of the rule between them; both lie within
+    bf16's rounding of a product in 64 bits."""
+    from sseqs_amd._lib import call, stream_of
+    announce(f"conv M={M} cin={cin} N={N}")
+    g = torch.Generator(device=dev).manual_seed(M + cin + N)
+    bf = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)  # noqa: E731
+    A = torch.zeros(M + 8, cin, dtype=torch.bfloat16, device=dev)
+    A[4:-4] = bf(M, cin)
+    Bt, bias = bf(N, 9 * cin) * (9 * cin) ** -0.5, torch.randn(N, generator=g, device=dev)
+    mask = (torch.rand(M, generator=g, device=dev) < 0.9).to(torch.uint8)
+    up = bf(M * N + 4)
+    rows = torch.arange(0, M, max(1, M // 257), device=dev)
+    win = torch.stack([A[rows + t] for t in range(9)], 1).reshape(rows.numel(), -1).double()
+    C = win @ Bt.double().T
+    m = mask[rows, None].double()
+    for epi in (0, 1, 2):
+        outs = []
+        for shift in (0, 2):  # elements: 4 bytes off in bf16, 8 in fp32
+            U, Y = (torch.full((M * N + 8,), 7.0, dtype=torch.bfloat16, device=dev) for _ in range(2))
+            Yf = torch.full((M * N + 8,), 7.0, device=dev)
+            call("sseqs_enc_conv", A.data_ptr() + 8 * cin, cin, Bt.data_ptr(), M, N, 9 * cin,
+                 bias.data_ptr() if epi == 0 else None, mask.data_ptr(),
+                 U.data_ptr() + 2 * shift if epi == 0 else None, Y.data_ptr() + 2 * shift if epi < 2 else None,
+                 up.data_ptr() if epi == 1 else None, Yf.data_ptr() + 4 * shift if epi == 2 else None, epi,
+                 stream_of(A.device))
+            for t in (U, Y, Yf):  # nothing before the output or past its end
+                assert (t[:shift] == 7).all() and (t[M * N + shift:] == 7).all()
+            outs.append([t[shift:M * N + shift].clone() for t in (U, Y, Yf)])
+        for a, b in zip(*outs):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), epi
+        U, Y, Yf = (t.view(M, N)[rows].double() for t in outs[0])
+        if epi == 0:
+            want = C + bias.double()
+            assert (U - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+            want = torch.nn.functional.gelu(want, approximate="tanh") * m
+            assert (Y - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+        elif epi == 1:
+            x = up[:M * N].view(M, N)[rows].double().requires_grad_()
+            gelu = torch.nn.functional.gelu(x, approximate="tanh")
+            want = C * torch.autograd.grad(gelu.sum(), x)[0] * m
+            assert (Y - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+        else:
+            assert (Yf - C * m).abs().max() <= 2.0 ** -16 * C.abs().max()
