@@ -28,6 +28,8 @@
 // every database sequence on v_mfma_f32_16x16x32_fp8_fp8.
 #include "common.h"
 
+#include <algorithm>
+
 namespace sseqs {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -103,6 +105,9 @@ struct ConvArgs {
 
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// 16 bytes at the alignment of their elements (the same instructions)
+typedef uint32_t u32x4_el __attribute__((ext_vector_type(4), aligned(2)));
+typedef __bf16 bf16x8_el __attribute__((ext_vector_type(8), aligned(2)));
 
 // CIN: lda, K = 9 CIN
 template <int CIN, int BN, int EPI, int WM, int WN>
@@ -356,79 +361,149 @@ __global__ __launch_bounds__(256) void k_conv_any(ConvArgs a) {
 
 // ---------------------------------------------------------- weight grad --
 //
-// dW[k][o] += sum_p A[p][k] * dU[p][o] over the rows p of this block's
-// range, k = t * Cin + i.  Block: 64 rows of k x 64 columns of o, rows p in
-// steps of 32 through LDS (X rows p-4 .. p+27+4 as the window source, dU
-// rows p .. p+31), MFMA with K = rows: lane (r, h) gathers 8 consecutive
-// rows of one column from LDS.  Partial sums of a block's row range are
-// added to dW (fp32) atomically.
-constexpr int WP = 32;   // rows per step
-constexpr int WROWS = 2048;  // rows per block
+// dW[t * Cin + i][o] += sum_p X[p - 4 + t][i] * dU[p][o] over the rows p of
+// this block's stages.  A block holds 64 channels i x 64 channels o of all
+// nine taps, wave (wm, wn) a 32 x 32 MFMA tile of each tap (144 accumulators),
+// so that a stage's 72 rows of X and 64 of dU come from memory once for nine
+// products of 64 x 64.  K of the products runs over rows: both operands leave
+// LDS through transposing reads, for which a tap is a row offset.  The next
+// stage's global loads are issued before the current stage's products.  The
+// block's sums are added to dW (fp32) atomically at the end.  Bound by the
+// products and those additions: WG_FILL blocks a layer, two to a CU (one to a
+// CU: 520 us).  312 k rows, three layers: 1000 -> 445 us against 64 x 64 tiles
+// of one tap whose operands were gathered from LDS two bytes at a time.
+//
+// ds_read_b64_tr_b16: of 16 lanes, lane 4 j + q reads the four elements q of
+// row j of a 4 x 16 tile, and lane l receives column l: its four rows.
+constexpr int WP = 64;           // rows per stage
+constexpr int WSTRIDE = 192;     // bytes of a row of 64 channels: rows j .. j + 3 meet in no bank
+constexpr int64_t WG_FILL = 512;
 
-__global__ __launch_bounds__(256) void k_conv_wgrad(const __bf16* __restrict__ X, int Cin,
-                                                    const __bf16* __restrict__ dU, int Cout,
-                                                    int64_t M, float* __restrict__ dW) {
-    // tile: k in [k0, k0 + 64) (k = t * Cin + i), o in [o0, o0 + 64); the
-    // k-columns of row p are X[(p - 4) * Cin + k0 .. + 64), contiguous
-    const int k0 = blockIdx.x * 64, o0 = blockIdx.y * 64;
-    const int64_t p_lo = (int64_t)blockIdx.z * WROWS;
-    const int64_t p_hi = min(p_lo + WROWS, M);
-    __shared__ __align__(16) __bf16 sA[WP * 64];
-    __shared__ __align__(16) __bf16 sD[WP * 64];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int r = lane & 31, h = lane >> 5;
-    const int wm = w >> 1, wn = w & 1;  // wave sub-tile: 32 k x 32 o
-    f32x16 acc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-    for (int64_t p0 = p_lo; p0 < p_hi; p0 += WP) {
-        __syncthreads();
-        {   // 32 rows x 64 columns of A and of dU, 8 elements per thread
-            const int row = tid >> 3, col = (tid & 7) * 8;
-            const int64_t p = p0 + row;
-            uint4 va = make_uint4(0, 0, 0, 0), vd = make_uint4(0, 0, 0, 0);
-            if (p < p_hi) {
-                va = *reinterpret_cast<const uint4*>(X + (p - 4) * Cin + k0 + col);
-                vd = *reinterpret_cast<const uint4*>(dU + p * Cout + o0 + col);
-            }
-            *reinterpret_cast<uint4*>(&sA[row * 64 + col]) = va;
-            *reinterpret_cast<uint4*>(&sD[row * 64 + col]) = vd;
-        }
-        __syncthreads();
-        // K of the MFMA runs over rows: lane (r, h) gathers 8 rows of one column
-#pragma unroll
-        for (int s = 0; s < WP / 16; ++s) {
-            bf16x8 fa, fb;
-#pragma unroll
-            for (int x = 0; x < 8; ++x) {
-                const int pp = 16 * s + 8 * h + x;
-                fa[x] = sA[pp * 64 + 32 * wm + r];
-                fb[x] = sD[pp * 64 + 32 * wn + r];
-            }
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb, acc, 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const int k = k0 + 32 * wm + 8 * (e >> 2) + 4 * h + (e & 3);
-        const int o = o0 + 32 * wn + r;
-        atomicAdd(&dW[(int64_t)k * Cout + o], acc[e]);
-    }
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+__device__ inline bf16x8 tr_frag(const uint8_t* p) {  // rows 0..3 and 4..7 of 16 columns per 16 lanes
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * WSTRIDE));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// db[o] += sum over rows of dU[p][o]: a block sums 1024 rows per column
-// (one thread per column of 64, four row phases), then one atomic each.
+__global__ __launch_bounds__(256, 2) void k_conv_wgrad(const __bf16* __restrict__ X, int Cin,
+                                                       const __bf16* __restrict__ dU, int Cout,
+                                                       int64_t M, int64_t per, float* __restrict__ dW) {
+    __shared__ __align__(16) uint8_t sX[2][(WP + 8) * WSTRIDE];
+    __shared__ __align__(16) uint8_t sD[2][WP * WSTRIDE];
+    const int i0 = blockIdx.x * 64, o0 = blockIdx.y * 64;
+    const int64_t s_lo = blockIdx.z * per, s_hi = min(s_lo + per, (M + WP - 1) / WP);
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int wm = w >> 1, wn = w & 1;
+    // 16-byte pieces: X's 576 to threads i, i + 256, i + 512, dU's 512 to i, i + 256
+    const int prow = tid >> 3, pc = tid & 7;
+    u32x4 rx[3], rd[2];
+    const auto load = [&](int64_t st) {
+        const int64_t p0 = st * WP;
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+            int64_t row = p0 - 4 + min(prow + 32 * x, WP + 7);
+            row = row < M + 3 ? row : M + 3;
+            rx[x] = *reinterpret_cast<const u32x4*>(X + row * Cin + i0 + 8 * pc);
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int64_t row = p0 + prow + 32 * x;
+            rd[x] = *reinterpret_cast<const u32x4*>(dU + (row < M ? row : M - 1) * Cout + o0 + 8 * pc);
+            if (row >= M) rd[x] = u32x4{0, 0, 0, 0};
+        }
+    };
+    const auto store = [&](int buf) {
+#pragma unroll
+        for (int x = 0; x < 3; ++x)
+            if (x < 2 || prow < 8)
+                *reinterpret_cast<u32x4*>(sX[buf] + (prow + 32 * x) * WSTRIDE + 16 * pc) = rx[x];
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+            *reinterpret_cast<u32x4*>(sD[buf] + (prow + 32 * x) * WSTRIDE + 16 * pc) = rd[x];
+    };
+    f32x16 acc[9];
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
+    // lane's part of a tile: row 8 h + j, channels 16 (g & 1) + 4 q of the wave's 32
+    const int g = lane >> 4, j = (lane >> 2) & 3, q = lane & 3;
+    const int lrow = (8 * (g >> 1) + j) * WSTRIDE + 2 * (16 * (g & 1) + 4 * q);
+    const int ax = lrow + 64 * wm, ad = lrow + 64 * wn;
+    if (s_lo < s_hi) {
+        load(s_lo);
+        store(0);
+    }
+    __syncthreads();
+    for (int64_t st = s_lo; st < s_hi; ++st) {
+        const int buf = (int)(st - s_lo) & 1;
+        if (st + 1 < s_hi) load(st + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < WP / 16; ++k) {
+            const bf16x8 fb = tr_frag(sD[buf] + ad + 16 * k * WSTRIDE);
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const bf16x8 fa = tr_frag(sX[buf] + ax + (16 * k + t) * WSTRIDE);
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb, acc[t], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (st + 1 < s_hi) store(buf ^ 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int i = i0 + 32 * wm + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+            const int o = o0 + 32 * wn + (lane & 31);
+            atomicAdd(&dW[(int64_t)(t * Cin + i) * Cout + o], acc[t][e]);
+        }
+}
+
+// db[o] += sum over rows of dU[p][o]: a block sums 1024 rows of 64 channels, a
+// thread eight channels of every 32nd row from 16-byte loads (eight in
+// flight), then the 32 row classes in LDS and one atomic per channel: blocks
+// of 256 rows, with four times as many atomics on the same addresses, took twice as
+// long.  312 k rows, three layers: 300 -> 79 us.
+constexpr int CS_ROWS = 1024;
 __global__ __launch_bounds__(256) void k_colsum(const __bf16* __restrict__ dU, int C, int64_t M,
                                                 float* __restrict__ db) {
-    __shared__ float s[4][64];
-    const int c = blockIdx.y * 64 + (threadIdx.x & 63), ph = threadIdx.x >> 6;
-    const int64_t lo = (int64_t)blockIdx.x * 1024, hi = min(lo + 1024, M);
-    float acc = 0.f;
-    for (int64_t p = lo + ph; p < hi; p += 4) acc += bf2f(dU[p * C + c]);
-    s[ph][threadIdx.x & 63] = acc;
+    __shared__ float s[32][65];
+    const int pc = threadIdx.x & 7, ph = threadIdx.x >> 3;
+    const int c0 = blockIdx.y * 64;
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < CS_ROWS; q += 256) {
+        const int64_t lo = (int64_t)blockIdx.x * CS_ROWS + q;
+        if (lo >= M) break;
+        u32x4 v[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+            const int64_t p = lo + ph + 32 * x;
+            v[x] = *reinterpret_cast<const u32x4_el*>(dU + (p < M ? p : M - 1) * C + c0 + 8 * pc);
+            if (p >= M) v[x] = u32x4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                acc[2 * y] += __uint_as_float(v[x][y] << 16);
+                acc[2 * y + 1] += __uint_as_float(v[x][y] & 0xffff0000u);
+            }
+    }
+#pragma unroll
+    for (int y = 0; y < 8; ++y) s[ph][8 * pc + y] = acc[y];
     __syncthreads();
-    if (ph == 0) atomicAdd(&db[c], s[0][threadIdx.x] + s[1][threadIdx.x] + s[2][threadIdx.x] +
-                                       s[3][threadIdx.x]);
+    if (threadIdx.x < 64) {
+        float t = 0.f;
+#pragma unroll
+        for (int x = 0; x < 32; ++x) t += s[x][threadIdx.x];
+        atomicAdd(&db[c0 + threadIdx.x], t);
+    }
 }
 
 // ------------------------------------------------------------ small ops --
@@ -447,19 +522,41 @@ __global__ void k_embed(const uint8_t* __restrict__ code, int64_t M, const float
     *reinterpret_cast<bf16x8*>(x0 + p * 64 + c0) = v;
 }
 
-// dE[code][c] += dX0[p][c]: per-block sums in LDS, then one atomic per entry
-__global__ __launch_bounds__(256) void k_embed_grad(const uint8_t* __restrict__ code, int64_t M,
-                                                    const float* __restrict__ dx0,
-                                                    float* __restrict__ dE) {
-    __shared__ float s[22 * 64];
-    for (int i = threadIdx.x; i < 22 * 64; i += 256) s[i] = 0.f;
+// dE[code][c] += dX0[p][c].  Each wave sums its rows (eight in flight, lane =
+// channel) into a table of its own in LDS, without atomics; the block's
+// tables are added up and go out as one atomic per entry, from one block per
+// CU.  LDS float atomics of one table per block took 117 us for 312 k rows,
+// this 21.
+constexpr int EG_WAVES = 16, EG_ROWS = 8;
+__global__ __launch_bounds__(64 * EG_WAVES) void k_embed_grad(const uint8_t* __restrict__ code,
+                                                              int64_t M,
+                                                              const float* __restrict__ dx0,
+                                                              float* __restrict__ dE) {
+    __shared__ float s[EG_WAVES][22 * 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int i = lane; i < 22 * 64; i += 64) s[w][i] = 0.f;
+    for (int64_t p0 = ((int64_t)blockIdx.x * EG_WAVES + w) * EG_ROWS; p0 < M;
+         p0 += (int64_t)gridDim.x * EG_WAVES * EG_ROWS) {
+        const int n = (int)min((int64_t)EG_ROWS, M - p0);
+        int cd[EG_ROWS];
+        float v[EG_ROWS];
+#pragma unroll
+        for (int x = 0; x < EG_ROWS; ++x) {
+            const int64_t p = p0 + min(x, n - 1);
+            cd[x] = code[p];
+            v[x] = dx0[p * 64 + lane];
+        }
+#pragma unroll
+        for (int x = 0; x < EG_ROWS; ++x)
+            if (x < n) s[w][cd[x] * 64 + lane] += v[x];
+    }
     __syncthreads();
-    const int c = threadIdx.x & 63, sub = threadIdx.x >> 6;
-    for (int64_t p = (int64_t)blockIdx.x * 4 + sub; p < M; p += (int64_t)gridDim.x * 4)
-        atomicAdd(&s[code[p] * 64 + c], dx0[p * 64 + c]);
-    __syncthreads();
-    for (int i = threadIdx.x; i < 20 * 64; i += 256)
-        if (s[i] != 0.f) atomicAdd(&dE[i], s[i]);
+    for (int i = threadIdx.x; i < 20 * 64; i += 64 * EG_WAVES) {
+        float t = 0.f;
+#pragma unroll
+        for (int x = 0; x < EG_WAVES; ++x) t += s[x][i];
+        if (t != 0.f) atomicAdd(&dE[i], t);
+    }
 }
 
 // Sequence s occupies rows [row0[s], row0[s] + len[s]).  z = mean of h3
@@ -518,7 +615,12 @@ __global__ __launch_bounds__(256) void k_pool(const __bf16* __restrict__ h3,
 }
 
 // Backward of the pool and of layer 3's GELU: dz = (de - e (e . de)) / |z|,
-// dU3[p][c] = dz[c] / L * gelu'(U3[p][c]) on the sequence's rows.
+// dU3[p][c] = dz[c] / L * gelu'(U3[p][c]) on the sequence's rows.  Blocks (s, y)
+// share a sequence: each works out dz (256 channels) and takes every
+// gridDim.y-th group of eight rows, a thread eight channels of one row from
+// one 16-byte load.  Bound by gelu' (tanh).  1056 sequences, 312 k rows:
+// 553 -> 100 us against one block and one row at a time per sequence.
+constexpr int PG_SPLIT = 8;
 __global__ __launch_bounds__(256) void k_pool_grad(const float* __restrict__ de,
                                                    const float* __restrict__ e,
                                                    const float* __restrict__ znorm,
@@ -527,7 +629,8 @@ __global__ __launch_bounds__(256) void k_pool_grad(const float* __restrict__ de,
                                                    const int32_t* __restrict__ len, int64_t nseq,
                                                    __bf16* __restrict__ dU3) {
     __shared__ float red[4];
-    const int c = threadIdx.x;
+    __shared__ __align__(16) float s_dz[256];
+    const int c = threadIdx.x, c8 = 8 * (c & 31), ph = c >> 5;
     for (int64_t s = blockIdx.x; s < nseq; s += gridDim.x) {
         const float ev = e[s * 256 + c], dv = de[s * 256 + c];
         float dot = ev * dv;
@@ -537,11 +640,19 @@ __global__ __launch_bounds__(256) void k_pool_grad(const float* __restrict__ de,
         const float d = red[0] + red[1] + red[2] + red[3];
         const float nrm = znorm[s];
         const int L = len[s];
-        const float dz = nrm > 0.f && L > 0 ? (dv - ev * d) / nrm / (float)L : 0.f;
+        s_dz[c] = nrm > 0.f && L > 0 ? (dv - ev * d) / nrm / (float)L : 0.f;
+        __syncthreads();
+        float dz[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) dz[x] = s_dz[c8 + x];
         const int64_t b = row0[s];
-        for (int p = 0; p < L; ++p) {
-            const int64_t o = (b + p) * 256 + c;
-            dU3[o] = f2bf(dz * gelu_grad(bf2f(U3[o])));
+        for (int p = 8 * blockIdx.y + ph; p < L; p += 8 * gridDim.y) {
+            const int64_t o = (b + p) * 256 + c8;
+            const bf16x8 u = *reinterpret_cast<const bf16x8_el*>(U3 + o);
+            bf16x8 v;
+#pragma unroll
+            for (int x = 0; x < 8; ++x) v[x] = f2bf(dz[x] * gelu_grad(bf2f(u[x])));
+            *reinterpret_cast<bf16x8_el*>(dU3 + o) = v;
         }
         __syncthreads();
     }
@@ -1002,11 +1113,13 @@ extern "C" int sseqs_enc_conv(const void* A, int lda, const void* Bt, int64_t M,
 extern "C" int sseqs_enc_wgrad(const void* X, int Cin, const void* dU, int Cout, int64_t M,
                                float* dW, hipStream_t stream) {
     if (M <= 0 || Cin % 64 || Cout % 64) return fail(-1, "enc_wgrad: bad sizes");
-    if (ceil_div(M, WROWS) > 65535) return fail(-1, "enc_wgrad: at most 65535 * 2048 rows");
-    const dim3 grid((unsigned)(9 * Cin / 64), (unsigned)(Cout / 64),
-                    (unsigned)ceil_div(M, WROWS));
+    if (ceil_div(M, 2048) > 65535) return fail(-1, "enc_wgrad: at most 65535 * 2048 rows");
+    const int64_t tiles = (int64_t)(Cin / 64) * (Cout / 64), stages = ceil_div(M, WP);
+    if (tiles == 0) return 0;
+    const int64_t per = std::max(ceil_div(stages, std::max<int64_t>(1, WG_FILL / tiles)), ceil_div(stages, 65535));
+    const dim3 grid((unsigned)(Cin / 64), (unsigned)(Cout / 64), (unsigned)ceil_div(stages, per));
     hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(256), 0, stream, static_cast<const __bf16*>(X),
-                       Cin, static_cast<const __bf16*>(dU), Cout, M, dW);
+                       Cin, static_cast<const __bf16*>(dU), Cout, M, per, dW);
     return check_launch("enc_wgrad");
 }
 
@@ -1014,7 +1127,7 @@ extern "C" int sseqs_enc_bias_grad(const void* dU, int C, int64_t M, float* db,
                                    hipStream_t stream) {
     if (M <= 0) return 0;
     if (C % 64) return fail(-1, "enc_bias_grad: C must be a multiple of 64");
-    hipLaunchKernelGGL(k_colsum, dim3((unsigned)ceil_div(M, 1024), (unsigned)(C / 64)), dim3(256),
+    hipLaunchKernelGGL(k_colsum, dim3((unsigned)ceil_div(M, CS_ROWS), (unsigned)(C / 64)), dim3(256),
                        0, stream, static_cast<const __bf16*>(dU), C, M, db);
     return check_launch("enc_bias_grad");
 }
@@ -1030,8 +1143,8 @@ extern "C" int sseqs_enc_embed(const uint8_t* code, int64_t M, const float* E, v
 extern "C" int sseqs_enc_embed_grad(const uint8_t* code, int64_t M, const float* dx0, float* dE,
                                     hipStream_t stream) {
     if (M <= 0) return 0;
-    hipLaunchKernelGGL(k_embed_grad, dim3(grid_cap(M, 4 * 64)), dim3(256), 0, stream, code, M,
-                       dx0, dE);
+    hipLaunchKernelGGL(k_embed_grad, dim3((unsigned)std::min<int64_t>(256, ceil_div(M, EG_WAVES * EG_ROWS))),
+                       dim3(64 * EG_WAVES), 0, stream, code, M, dx0, dE);
     return check_launch("enc_embed_grad");
 }
 
@@ -1047,7 +1160,7 @@ extern "C" int sseqs_enc_pool_grad(const float* de, const float* e, const float*
                                    const void* U3, const int64_t* row0, const int32_t* len,
                                    int64_t nseq, void* dU3, hipStream_t stream) {
     if (nseq <= 0) return 0;
-    hipLaunchKernelGGL(k_pool_grad, dim3(grid_cap(nseq, 1)), dim3(256), 0, stream, de, e, znorm,
+    hipLaunchKernelGGL(k_pool_grad, dim3(grid_cap(nseq, 1), PG_SPLIT), dim3(256), 0, stream, de, e, znorm,
                        static_cast<const __bf16*>(U3), row0, len, nseq, static_cast<__bf16*>(dU3));
     return check_launch("enc_pool_grad");
 }

@@ -151,9 +151,9 @@ class Encoder:
     # ---------------------------------------------------------- buffers --
     def _buffers(self, M: int, train: bool) -> dict:
         """Activations with four zero margin rows at both ends (the conv
-        windows read rows -4 .. M + 3)."""
+        windows read rows -4 .. M + 3; the passes write the rows between)."""
         dev = self.dev
-        z = lambda C: torch.zeros((M + 8, C), dtype=torch.bfloat16, device=dev)
+        z = lambda C: torch.empty((M + 8, C), dtype=torch.bfloat16, device=dev)  # noqa: E731
         b = {"x0": z(C0), "h1": z(C1), "h2": z(C2),
              "h3": torch.empty((M, C3), dtype=torch.bfloat16, device=dev)}
         if train:
@@ -162,6 +162,10 @@ class Encoder:
                       "u3": torch.empty((M, C3), dtype=torch.bfloat16, device=dev),
                       "du3": z(C3), "du2": z(C2), "du1": z(C1),
                       "dx0": torch.empty((M, C0), dtype=torch.float32, device=dev)})
+        for t in b.values():
+            if t.shape[0] == M + 8:
+                t.view(torch.int32).as_strided((2, 4 * t.shape[1] // 2),
+                                               ((M + 4) * t.shape[1] // 2, 1)).zero_()
         return b
 
     @staticmethod

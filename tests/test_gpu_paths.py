@@ -222,3 +222,68 @@ def test_encoder_conv_tiles(dev, M, cin, N):
             assert (Y - want).abs().max() <= 2.0 ** -8 * want.abs().max()
         else:
             assert (Yf - C * m).abs().max() <= 2.0 ** -16 * C.abs().max()
+
+
+@pytest.mark.parametrize("M,cin,cout", [(1, 64, 64), (63, 64, 128), (64, 128, 64), (65, 128, 256), (1025, 64, 64),
+                                        (32769, 128, 128), (128 * 700, 128, 256)])
+def test_encoder_gradient_sums(dev, M, cin, cout):
+    """Weight, bias and embedding gradients around their stages (64 rows, 1024
+    rows, 128 rows) against sums in 64 bits, added to what is there; the bias
+    gradient also from an odd element's address."""
+    from sseqs_amd._lib import call, stream_of
+    announce(f"gradient sums M={M} cin={cin} cout={cout}")
+    g = torch.Generator(device=dev).manual_seed(M + cin + cout)
+    X = torch.zeros(M + 8, cin, dtype=torch.bfloat16, device=dev)
+    X[4:-4] = torch.randn(M, cin, generator=g, device=dev)
+    flat = torch.randn(M * cout + 1, generator=g, device=dev).to(torch.bfloat16)
+    st = stream_of(X.device)
+    for shift in (0, 1):
+        dU = flat[shift: M * cout + shift].view(M, cout).double()
+        db = torch.full((cout,), 3.0, device=dev)
+        call("sseqs_enc_bias_grad", flat.data_ptr() + 2 * shift, cout, M, db.data_ptr(), st)
+        # fp32 sums of M terms: M 2^-24 of the sum of absolute values is a bound on the rounding
+        tol = M * 2.0 ** -24 * dU.abs().sum(0).max() + 1e-6
+        assert (db.double() - 3 - dU.sum(0)).abs().max() <= tol
+    dU = flat[: M * cout].view(M, cout).double()
+    dW = torch.full((9 * cin, cout), 3.0, device=dev)
+    call("sseqs_enc_wgrad", X.data_ptr() + 8 * cin, cin, flat.data_ptr(), cout, M, dW.data_ptr(), st)
+    for t in range(9):
+        x = X[t: t + M].double()
+        want, tol = x.T @ dU, (x.abs().T @ dU.abs()).max() * M * 2.0 ** -24 + 1e-6
+        assert (dW[t * cin:(t + 1) * cin].double() - 3 - want).abs().max() <= tol, t
+    code = torch.randint(0, 22, (M,), generator=g, device=dev).to(torch.uint8)
+    dx = torch.randn(M, 64, generator=g, device=dev)
+    dE = torch.full((22, 64), 3.0, device=dev)
+    call("sseqs_enc_embed_grad", code.data_ptr(), M, dx.data_ptr(), dE.data_ptr(), st)
+    want = torch.zeros(22, 64, dtype=torch.float64, device=dev).index_add_(0, code.long(), dx.double())
+    want[20:] = 0
+    assert (dE.double() - 3 - want).abs().max() <= M * 2.0 ** -24 * dx.abs().double().sum(0).max() + 1e-6
+
+
+def test_encoder_pool_gradient_rows(dev):
+    """The pool's gradient on sequences of 0 to 70 rows (groups of eight rows
+    over eight blocks), rows outside them untouched."""
+    from sseqs_amd._lib import call, stream_of
+    announce("pool gradient rows")
+    g = torch.Generator(device=dev).manual_seed(5)
+    lens = [0, 1, 7, 8, 9, 63, 64, 65, 70]
+    row0 = torch.tensor(np.cumsum([4] + [n + 4 for n in lens[:-1]]), dtype=torch.int64, device=dev)
+    M = int(row0[-1]) + lens[-1] + 4
+    e = torch.nn.functional.normalize(torch.randn(len(lens), 256, generator=g, device=dev), dim=1)
+    de = torch.randn(len(lens), 256, generator=g, device=dev)
+    zn = torch.rand(len(lens), generator=g, device=dev) + 0.5
+    U = torch.randn(M, 256, generator=g, device=dev).to(torch.bfloat16)
+    tl = torch.tensor(lens, dtype=torch.int32, device=dev)
+    out = torch.full((M, 256), 7.0, dtype=torch.bfloat16, device=dev)
+    call("sseqs_enc_pool_grad", de.data_ptr(), e.data_ptr(), zn.data_ptr(), U.data_ptr(), row0.data_ptr(),
+         tl.data_ptr(), len(lens), out.data_ptr(),
+         stream_of(e.device))
+    torch.cuda.synchronize()
+    want = torch.full((M, 256), 7.0, dtype=torch.float64, device=dev)
+    x = U.double().requires_grad_()
+    gg = torch.autograd.grad(torch.nn.functional.gelu(x, approximate="tanh").sum(), x)[0]
+    for s, n in enumerate(lens):
+        dz = (de[s].double() - e[s].double() * (e[s].double() @ de[s].double())) / zn[s].double() / max(n, 1)
+        want[row0[s]: row0[s] + n] = dz * gg[row0[s]: row0[s] + n]
+    # fp32 steps before one rounding to bf16: half a unit of 2^-8, and room for the cancellation in dz
+    assert ((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6).all()
