@@ -871,6 +871,17 @@ __global__ __launch_bounds__(1024) void k_sel_sort(const void* s, const int64_t*
 // segment's keys in LDS fix the k-th largest key T, then one pass in index
 // order writes the selection (keys > T, then the first keys == T), or the
 // selection is staged in LDS and sorted by (key desc, index asc).
+//
+// The scores of a segment fall into few bins, so a pass over all keys is bound
+// by LDS atomics on the same addresses, and a sweep has fewer segments than
+// the chip has CUs.  A long segment of which little is taken (seg_guess) is
+// therefore first cut down: the R-th largest of SEG_SAMPLE keys, R some
+// deviations past the rank that k has among them, is a key that enough of the
+// segment reaches, and the keys that reach it go to a list in LDS in index
+// order (one pass counts them per wave, one writes them); the passes then
+// read the list.  If they are fewer than k or more than the list holds, the
+// passes read the segment.  72 segments of 281 000 fp16 scores, k = n / 200:
+// 739 -> 283 us.
 
 constexpr int SEG_THREADS = 1024;
 constexpr int SEG_WAVES = SEG_THREADS / 64;
@@ -891,23 +902,104 @@ __device__ inline uint32_t seg_key(const void* s, int64_t i) {
         return load_key<DT>(s, i);
 }
 
+constexpr int SEG_SAMPLE = SEG_THREADS * SEG_E;
+constexpr int SEG_LIST = 12288;     // keys and indices: 96 KiB of LDS
+constexpr int64_t SEG_CUT_MAX = 256;  // segments, one to a CU: the list takes its LDS
+
+// The rank among SEG_SAMPLE of n keys to guess at, or 0 where the passes read
+// the segment itself: below four samples there is little to save, and a list
+// is expected to fill less than seven eighths.
+__device__ inline int seg_guess(int n, int k) {
+    if (n < 4 * SEG_SAMPLE) return 0;
+    const float m = (float)SEG_SAMPLE * (float)k / (float)n;
+    const float r = m + 4.f * sqrtf(m) + 8.f;
+    return r * (float)n <= 0.875f * SEG_LIST * SEG_SAMPLE ? (int)r : 0;
+}
+
+typedef uint32_t seg_u32x4_el __attribute__((ext_vector_type(4), aligned(2)));
+
+// A wave's step: 512 consecutive elements, eight to a lane; SEG_U steps' loads
+// are in flight together.
+constexpr int SEG_U = 4;
+template <int DT>
+struct SegStep {
+    static constexpr int NV = DT == SSEQS_F16 ? 1 : 2;
+    uint32_t w[4 * NV];
+    __device__ void load(const void* s, int i0) {
+        const int i = i0 + 8 * (threadIdx.x & 63);
+        const char* p = static_cast<const char*>(s) + (DT == SSEQS_F16 ? 2 : 4) * (int64_t)i;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const seg_u32x4_el x = reinterpret_cast<const seg_u32x4_el*>(p)[v];
+#pragma unroll
+            for (int y = 0; y < 4; ++y) w[4 * v + y] = x[y];
+        }
+    }
+    // the last, partial step: element by element, past n the last one
+    __device__ void load_tail(const void* s, int i0, int n) {
+        const int i = i0 + 8 * (threadIdx.x & 63);
+#pragma unroll
+        for (int y = 0; y < 4 * NV; ++y) {
+            if constexpr (DT == SSEQS_F16) {
+                const uint16_t* h = static_cast<const uint16_t*>(s);
+                w[y] = h[min(i + 2 * y, n - 1)] | (uint32_t)h[min(i + 2 * y + 1, n - 1)] << 16;
+            } else {
+                w[y] = static_cast<const uint32_t*>(s)[min(i + y, n - 1)];
+            }
+        }
+    }
+    __device__ uint32_t key(int e) const {
+        if constexpr (DT == SSEQS_F16) return key_h16((uint16_t)(w[e >> 1] >> (16 * (e & 1))));
+        else return load_key<DT>(w, e);
+    }
+    // bit e: element i0 + 8 lane + e is below n and its key at least g
+    __device__ uint32_t reach(int i0, int n, uint32_t g) const {
+        const int i = i0 + 8 * (threadIdx.x & 63);
+        uint32_t in = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) in |= key(e) >= g && i + e < n ? 1u << e : 0u;
+        return in;
+    }
+};
+
+// f(first element, step) over the steps of elements lo .. hi - 1
+template <int DT, class F>
+__device__ inline void seg_steps(const void* s, int lo, int hi, int n, F f) {
+    int i0 = lo;
+    for (; i0 + 512 * SEG_U <= hi; i0 += 512 * SEG_U) {
+        SegStep<DT> st[SEG_U];
+#pragma unroll
+        for (int u = 0; u < SEG_U; ++u) st[u].load(s, i0 + 512 * u);
+#pragma unroll
+        for (int u = 0; u < SEG_U; ++u) f(i0 + 512 * u, st[u]);
+    }
+    for (; i0 < hi; i0 += 512) {
+        SegStep<DT> st;
+        if (i0 + 512 <= n) st.load(s, i0);
+        else st.load_tail(s, i0, n);
+        f(i0, st);
+    }
+}
+
 template <int DT>
 __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
     const void* __restrict__ s, const int64_t* __restrict__ seg_begin,
     const int32_t* __restrict__ seg_n, const int32_t* __restrict__ seg_k,
     const int64_t* __restrict__ out_base, int64_t nseg, int sorted, int drop_front,
-    int drop_back, int add_begin, int64_t* __restrict__ out) {
+    int drop_back, int add_begin, int lcap, int64_t* __restrict__ out) {
     __shared__ uint32_t hist[SEL_BINS];
     __shared__ uint64_t comp[SEG_SORT_MAX];
     __shared__ uint32_t wsum[SEG_WAVES];
     __shared__ uint32_t s_pick[2];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    extern __shared__ uint32_t l_key[];  // the list (lcap entries): keys, then indices
+    uint32_t* l_idx = l_key + lcap;
     const int npass = DT == SSEQS_F16 ? 2 : 3;
     const int shifts16[2] = {5, 0}, bits16[2] = {11, 5};
     const int shifts32[3] = {21, 10, 0}, bits32[3] = {11, 11, 10};
     for (int64_t j = blockIdx.x; j < nseg; j += gridDim.x) {
         const int64_t beg = seg_begin[j];
-        const int n = seg_n[j];
+        int n = seg_n[j];
         int k = min(seg_k[j], n);
         if (sorted) k = min(k, SEG_SORT_MAX);
         if (k <= 0) continue;  // uniform over the block
@@ -916,56 +1008,107 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
                            : DT == SSEQS_F32
                                ? static_cast<const void*>(static_cast<const float*>(s) + beg)
                                : static_cast<const void*>(static_cast<const int32_t*>(s) + beg);
-        uint32_t prefix = 0, mask = 0, krem = (uint32_t)k;
-        for (int p = 0; p < npass; ++p) {
-            const int shift = DT == SSEQS_F16 ? shifts16[p] : shifts32[p];
-            const int bits = DT == SSEQS_F16 ? bits16[p] : bits32[p];
-            const uint32_t bm = (1u << bits) - 1u;
-            for (int i = tid; i < SEL_BINS; i += SEG_THREADS) hist[i] = 0;
-            __syncthreads();
-            // SEG_E independent loads in flight per thread
-            for (int i0 = 0; i0 < n; i0 += SEG_THREADS * SEG_E) {
-                uint32_t key[SEG_E];
+        // round 0 (with a guess): the R-th largest key of the sample, and the
+        // list of the keys that reach it; round 1: the k-th largest key
+        const int R = lcap ? seg_guess(n, k) : 0;
+        bool listed = false;
+        uint32_t prefix = 0, mask = 0, krem = 0;
+        for (int round = R > 0 ? 0 : 1; round < 2; ++round) {
+            const int m = round ? n : SEG_SAMPLE;
+            prefix = mask = 0;
+            krem = (uint32_t)(round ? k : R);
+            for (int p = 0; p < npass; ++p) {
+                const int shift = DT == SSEQS_F16 ? shifts16[p] : shifts32[p];
+                const int bits = DT == SSEQS_F16 ? bits16[p] : bits32[p];
+                const uint32_t bm = (1u << bits) - 1u;
+                for (int i = tid; i < SEL_BINS; i += SEG_THREADS) hist[i] = 0;
+                __syncthreads();
+                // SEG_E independent loads in flight per thread
+                for (int i0 = 0; i0 < m; i0 += SEG_THREADS * SEG_E) {
+                    uint32_t key[SEG_E];
 #pragma unroll
-                for (int e = 0; e < SEG_E; ++e) {
-                    // clamped index: the loads are unconditional and all in flight
-                    const int i = min(i0 + e * SEG_THREADS + tid, n - 1);
-                    key[e] = seg_key<DT>(base, i);
-                }
-#pragma unroll
-                for (int e = 0; e < SEG_E; ++e) {
-                    const int i = i0 + e * SEG_THREADS + tid;
-                    if (i < n && (key[e] & mask) == prefix)
-                        atomicAdd(&hist[(key[e] >> shift) & bm], 1u);
-                }
-            }
-            __syncthreads();
-            if (wid == 0) {
-                // lane L holds bins 32L..32L+31; the lane whose bins contain
-                // the krem-th largest key walks them from the top
-                uint32_t sum = 0;
-                for (int t = 0; t < 32; ++t) sum += hist[lane * 32 + t];
-                uint32_t incl = sum;  // keys in bins of lanes >= this one
-                for (int off = 1; off < 64; off <<= 1) {
-                    const uint32_t t = __shfl_down(incl, off, 64);
-                    if (lane + off < 64) incl += t;
-                }
-                uint32_t above = incl - sum;
-                if (above < krem && krem <= incl) {
-                    int b = lane * 32 + 31;
-                    for (; b > lane * 32; --b) {
-                        if (above + hist[b] >= krem) break;
-                        above += hist[b];
+                    for (int e = 0; e < SEG_E; ++e) {
+                        // clamped index: the loads are unconditional and all in flight
+                        const int i = min(i0 + e * SEG_THREADS + tid, m - 1);
+                        key[e] = listed ? l_key[i]
+                                        : seg_key<DT>(base, round ? i : (int)((int64_t)i * n / SEG_SAMPLE));
                     }
-                    s_pick[0] = (uint32_t)b;
-                    s_pick[1] = krem - above;
+#pragma unroll
+                    for (int e = 0; e < SEG_E; ++e) {
+                        const int i = i0 + e * SEG_THREADS + tid;
+                        if (i < m && (key[e] & mask) == prefix)
+                            atomicAdd(&hist[(key[e] >> shift) & bm], 1u);
+                    }
                 }
+                __syncthreads();
+                if (wid == 0) {
+                    // lane L holds bins 32L..32L+31; the lane whose bins contain
+                    // the krem-th largest key walks them from the top
+                    uint32_t sum = 0;
+                    for (int t = 0; t < 32; ++t) sum += hist[lane * 32 + ((t + lane) & 31)];
+                    uint32_t incl = sum;  // keys in bins of lanes >= this one
+                    for (int off = 1; off < 64; off <<= 1) {
+                        const uint32_t t = __shfl_down(incl, off, 64);
+                        if (lane + off < 64) incl += t;
+                    }
+                    uint32_t above = incl - sum;
+                    if (above < krem && krem <= incl) {
+                        int b = lane * 32 + 31;
+                        for (; b > lane * 32; --b) {
+                            if (above + hist[b] >= krem) break;
+                            above += hist[b];
+                        }
+                        s_pick[0] = (uint32_t)b;
+                        s_pick[1] = krem - above;
+                    }
+                }
+                __syncthreads();
+                prefix |= s_pick[0] << shift;
+                mask |= bm << shift;
+                krem = s_pick[1];
+                __syncthreads();
             }
-            __syncthreads();
-            prefix |= s_pick[0] << shift;
-            mask |= bm << shift;
-            krem = s_pick[1];
-            __syncthreads();
+            if (round == 0) {
+                // wave w takes the w-th sixteenth of the segment, 512 elements a step
+                const int per = (n + 512 * SEG_WAVES - 1) / (512 * SEG_WAVES) * 512;
+                const int lo = min(n, wid * per), hi = min(n, lo + per);
+                int cnt = 0;
+                seg_steps<DT>(base, lo, hi, n, [&](int i0, const SegStep<DT>& st) {
+                    cnt += __popc(st.reach(i0, n, prefix));
+                });
+                for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
+                if (lane == 0) wsum[wid] = (uint32_t)cnt;
+                __syncthreads();
+                int at = 0, total = 0;
+#pragma unroll
+                for (int w = 0; w < SEG_WAVES; ++w) {
+                    at += w < wid ? (int)wsum[w] : 0;
+                    total += (int)wsum[w];
+                }
+                listed = total >= k && total <= lcap;
+                if (listed) {
+                    seg_steps<DT>(base, lo, hi, n, [&](int i0, const SegStep<DT>& st) {
+                        const uint32_t in = st.reach(i0, n, prefix);
+                        if (!__any(in)) return;
+                        int inc = __popc(in);
+                        for (int o = 1; o < 64; o <<= 1) {
+                            const int t = __shfl_up(inc, o, 64);
+                            if (lane >= o) inc += t;
+                        }
+                        int slot = at + inc - __popc(in);
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            if ((in >> e) & 1u) {
+                                l_key[slot] = st.key(e);
+                                l_idx[slot] = (uint32_t)(i0 + 8 * lane + e);
+                                ++slot;
+                            }
+                        at += __shfl(inc, 63, 64);
+                    });
+                    n = total;
+                }
+                __syncthreads();
+            }
         }
         // keys > T are all taken, keys == T while fewer than krem came
         // before.  Each thread takes SEG_E consecutive elements of a chunk;
@@ -981,7 +1124,8 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
             const int ib = i0 + tid * SEG_E;
             uint32_t key[SEG_E];
 #pragma unroll
-            for (int e = 0; e < SEG_E; ++e) key[e] = seg_key<DT>(base, min(ib + e, n - 1));
+            for (int e = 0; e < SEG_E; ++e)
+                key[e] = listed ? l_key[min(ib + e, n - 1)] : seg_key<DT>(base, min(ib + e, n - 1));
             uint32_t cnt = 0;
 #pragma unroll
             for (int e = 0; e < SEG_E; ++e) {
@@ -1013,10 +1157,11 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
                 const bool q = in && key[e] == T;
                 const int slot = gb + min(eb, keq);
                 if ((g || (q && eb < keq)) && slot < k) {
+                    const uint32_t at = listed ? l_idx[ib + e] : (uint32_t)(ib + e);
                     if (sorted)
-                        comp[slot] = ((uint64_t)(~key[e]) << 32) | (uint64_t)(uint32_t)(ib + e);
+                        comp[slot] = ((uint64_t)(~key[e]) << 32) | (uint64_t)at;
                     else if (slot >= drop_front && slot < hi)
-                        out[ob + slot] = add + ib + e;
+                        out[ob + slot] = add + at;
                 }
                 gb += g;
                 eb += q;
@@ -1272,8 +1417,9 @@ extern "C" int sseqs_topk_segments(const void* scores, int dtype, const int64_t*
     if (!scores || !seg_begin || !seg_n || !seg_k || !out_base || !out_idx)
         return fail(-1, "topk_segments: null pointer");
     const unsigned grid = (unsigned)(nseg < 8192 ? nseg : 8192);
-    SEL_DISPATCH(k_seg_topk, dim3(grid), dim3(SEG_THREADS), 0, stream, scores,
+    const int lcap = nseg <= SEG_CUT_MAX ? SEG_LIST : 0;
+    SEL_DISPATCH(k_seg_topk, dim3(grid), dim3(SEG_THREADS), (size_t)8 * lcap, stream, scores,
                        seg_begin, seg_n, seg_k, out_base, nseg, sorted, drop_front, drop_back,
-                       add_begin, out_idx);
+                       add_begin, lcap, out_idx);
     return check_launch("topk_segments");
 }

@@ -287,3 +287,46 @@ def test_encoder_pool_gradient_rows(dev):
         want[row0[s]: row0[s] + n] = dz * gg[row0[s]: row0[s] + n]
     # fp32 steps before one rounding to bf16: half a unit of 2^-8, and room for the cancellation in dz
     assert ((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32", "i32"])
+@pytest.mark.parametrize("sorted_", [False, True])
+def test_topk_segments_cut(dev, dtype, sorted_):
+    """Segments around the length (32768) and the counts that choose the cut
+    to a list: random, equal, rising and bunched scores (a sample that
+    misleads), NaN and infinities, begins of any alignment."""
+    from sseqs_amd import ops
+    announce(f"topk_segments cut {dtype} sorted={sorted_}")
+    rng = np.random.default_rng(3)
+    segs = [(n, k, kind) for n in (32767, 32768, 32769 + 512, 70001, 400003) for k in (1, 163, n // 200, 1600, 2049)
+            for kind in ("normal", "special")]
+    segs += [(50000, 300, "equal"), (50000, 300, "rising"), (50000, 300, "bunched"), (281001, 1405, "ties")]
+    parts = []
+    for n, k, kind in segs:
+        x = rng.normal(21.0, 2.5, n)
+        if kind == "equal":
+            x[:] = 3.0
+        elif kind == "rising":
+            x = np.arange(n) / 64.0
+        elif kind == "bunched":
+            x[1000:1400] += 50.0
+        elif kind == "ties":
+            x = np.round(x)
+        elif kind == "special" and dtype != "i32":
+            x[::7], x[3::50], x[5::9] = np.nan, np.inf, -np.inf
+        parts.append(x)
+    n = np.array([p.size for p in parts])
+    begin = np.concatenate([[1], 1 + np.cumsum(n + 1)[:-1]])  # a score between segments
+    flat = np.full(int(n.sum() + n.size + 1), 7.0)
+    for b, p in zip(begin, parts):
+        flat[b: b + p.size] = p
+    flat = flat.astype({"f16": np.float16, "f32": np.float32, "i32": np.int32}[dtype])
+    k = np.minimum([s[1] for s in segs], 4096)
+    got, base = ops.topk_segments(torch.from_numpy(flat).to(dev), begin, n, k, sorted=sorted_)
+    got = got.cpu().numpy()
+    for j in range(len(segs)):
+        x = flat[begin[j]: begin[j] + n[j]].astype(np.float64)
+        if dtype != "i32":
+            x = np.where(np.isnan(x), -np.inf, np.where(x == -np.inf, -1e300, x))
+        want = np.argsort(-x, kind="stable")[: k[j]]
+        assert np.array_equal(got[base[j]: base[j] + k[j]], want if sorted_ else np.sort(want)), segs[j]
