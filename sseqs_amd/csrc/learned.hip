@@ -39,6 +39,16 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ inline float bf2f(__bf16 v) { return (float)v; }
 __device__ inline __bf16 f2bf(float v) { return (__bf16)v; }
 
+// Orders a wave's LDS accesses across its lanes (no barrier between waves):
+// wavefront-scope release/acquire fences keep the compiler's memory
+// operations on either side, and the hardware runs one wave's LDS
+// instructions in order.
+__device__ __forceinline__ void lds_wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // GELU, tanh form, and its derivative.
 __device__ inline float gelu(float x) {
     const float c = 0.7978845608028654f;  // sqrt(2 / pi)
@@ -50,6 +60,40 @@ __device__ inline float gelu_grad(float x) {
     const float u = c * (x + 0.044715f * x * x * x);
     const float t = tanhf(u);
     return 0.5f * (1.f + t) + 0.5f * x * (1.f - t * t) * c * (1.f + 3.f * 0.044715f * x * x);
+}
+
+// bf16 of gelu(x0) * m0 and gelu(x1) * m1 (low and high half), equal to the
+// functions above bit for bit.  tanhf is a divergent branch of some 40
+// instructions, twice the products' own time in the narrow layers.  Here
+// tanh u = 2 g - 1 with g = 1 / (1 + exp(-2u)) comes from the hardware's
+// exponential and reciprocal, once with g a little too small and once a little
+// too large (GELU_EPS: for every float the tanhf of gelu() lies between, and
+// the rounding to 24 bits that makes 1 + tanh u coarse for negative u is the
+// same).  Each further step is monotonic, so where both ends round to one
+// bf16 that is gelu's; where they differ (about 1 in 2000), gelu() itself is
+// evaluated.
+constexpr float GELU_EPS = 3e-6f;
+__device__ inline uint32_t gelu_bf16x2(float x0, float x1, float m0, float m1) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const float x[2] = {x0, x1}, m[2] = {m0, m1};
+    bf16x2 lo, hi;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float c = 0.7978845608028654f;  // sqrt(2 / pi)
+        const float u = c * (x[i] + 0.044715f * x[i] * x[i] * x[i]);
+        const float g =
+            __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-2.f * 1.4426950408889634f * u));
+        const float h = 0.5f * x[i] * m[i];
+        lo[i] = f2bf(h * (1.f + fmaf(g, 2.f - GELU_EPS, -1.f)));
+        hi[i] = f2bf(h * (1.f + fmaf(g, 2.f + GELU_EPS, -1.f)));
+    }
+    uint32_t v = __builtin_bit_cast(uint32_t, lo);
+    if (v != __builtin_bit_cast(uint32_t, hi)) {
+        lo[0] = f2bf(gelu(x0) * m0);
+        lo[1] = f2bf(gelu(x1) * m1);
+        v = __builtin_bit_cast(uint32_t, lo);
+    }
+    return v;
 }
 
 // ------------------------------------------------------------- conv GEMM --
@@ -72,12 +116,14 @@ __device__ inline float gelu_grad(float x) {
 // row r, elements 8h .. 8h+7 of K of both operands.  The weights are the
 // first operand: result element e of lane (c, h) is then column
 // 8 * (e / 4) + 4 * h + (e % 4) of C in row c, four consecutive columns to a
-// lane, which go in and out as 8 bytes.
+// lane.
 //
-// Bound by issue slots: the products take 40 % of them, GELU's tanh as many
-// again.  The three layers over 8.6 M rows 16.1 -> 12.3 ms (0.55 -> 0.72
-// PFLOP/s) against 128 x 128 tiles that read every tap's rows from memory;
-// the backward products of 312 k rows 761 -> 477 us.
+// Bound by issue slots: the products take 55 % of them, GELU most of the rest.
+// The three layers over 8.6 M rows 16.1 -> 10.0 ms (0.55 -> 0.88 PFLOP/s)
+// against 128 x 128 tiles that read every tap's rows from memory, with tanhf
+// and two-byte stores; in steps 12.3 (rows kept, wide waves), 10.6
+// (gelu_bf16x2) and 10.0 (whole lines out). The backward products of 312 k
+// rows 761 -> 466 us.
 constexpr int GM = 128, GK = 32;  // granularity of M; columns of Bt of a stage
 // Wide blocks when they fill the 512 places of the chip (two a CU) once; with
 // fewer, small blocks spread the rows over more CUs.
@@ -218,44 +264,98 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_gemm(ConvArgs a) {
 #undef CONV_STORE_B
 #undef CONV_LOAD_F
 
-    // epilogue: lane (r, h) holds columns 32 j + 8 q + 4 h .. + 3 of its row
+    // epilogue: lane (r, h) holds columns 32 j + 8 q + 4 h .. + 3 of its row.
+    // bf16 rows pass through the wave's part of LDS (free after the last
+    // stage's barrier), 32 at a time, so that whole lines of them come and go:
+    // 8-byte accesses of 32 rows at once made 16-byte requests.  Row r holds
+    // its 16-byte pieces at piece ^ (r mod 16).
+    constexpr int WC = BN / WN, PW = 2 * WC / 16;  // the wave's columns, pieces of their row
+    static_assert(WM * WN * 32 * 2 * WC <= ROWS * RB, "the waves' rows fit the place of A");
+    uint8_t* lw = sA + w * (32 * 2 * WC);
+    const int nw = n0 + WC * wn;
+    const auto place = [&](int row, int piece) { return row * 2 * WC + 16 * (piece ^ (row & (PW - 1))); };
+    // rows 64 wm + 32 i .. + 31 of the block, a whole row to PW lanes
+    const auto rows_out = [&](__bf16* out, int i) {
+        lds_wave_fence();
+#pragma unroll
+        for (int x = 0; x < 32 * PW / 64; ++x) {
+            const int row = lane / PW + 64 / PW * x, pc = lane % PW;
+            const int mr = 64 * wm + 32 * i + row;
+            const u32x4 v = *reinterpret_cast<const u32x4*>(lw + place(row, pc));
+            if (mr < OUT && m0 + mr < a.M)
+                *reinterpret_cast<u32x4*>(out + (m0 + mr) * a.N + nw + 8 * pc) = v;
+        }
+        lds_wave_fence();
+    };
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int mr = 64 * wm + 32 * i + r;
         const int64_t m = m0 + mr;
-        if (mr >= OUT || m >= a.M) continue;
-        const float mk = a.mask[m] ? 1.f : 0.f;
+        const bool in = mr < OUT && m < a.M;
+        const float mk = in && a.mask[m] ? 1.f : 0.f;
+        if constexpr (EPI == EPI_FWD) {
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+            for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int n = n0 + BN / WN * wn + 32 * j + 8 * q + 4 * h;
-                const int64_t o = m * a.N + n;
-                if constexpr (EPI == EPI_FWD) {
-                    const float4 bias = *reinterpret_cast<const float4*>(a.bias + n);
-                    const float bb[4] = {bias.x, bias.y, bias.z, bias.w};
-                    bf16x4 u, y;
+                for (int q = 0; q < 4; ++q) {
+                    const float4 bias =
+                        *reinterpret_cast<const float4*>(a.bias + nw + 32 * j + 8 * q + 4 * h);
+                    acc[i][j][4 * q] += bias.x;
+                    acc[i][j][4 * q + 1] += bias.y;
+                    acc[i][j][4 * q + 2] += bias.z;
+                    acc[i][j][4 * q + 3] += bias.w;
+                }
+            if (a.U) {
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) {
-                        const float v = acc[i][j][4 * q + x] + bb[x];
-                        u[x] = f2bf(v);
-                        y[x] = f2bf(gelu(v) * mk);
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        bf16x4 u;
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) u[x] = f2bf(acc[i][j][4 * q + x]);
+                        *reinterpret_cast<bf16x4*>(lw + place(r, 4 * j + q) + 8 * h) = u;
                     }
-                    if (a.U) *reinterpret_cast<bf16x4*>(a.U + o) = u;
-                    *reinterpret_cast<bf16x4*>(a.Y + o) = y;
-                } else if constexpr (EPI == EPI_BWD_GELU) {
-                    const bf16x4 up = *reinterpret_cast<const bf16x4*>(a.Uprev + o);
+                rows_out(a.U, i);
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<uint2*>(lw + place(r, 4 * j + q) + 8 * h) = make_uint2(
+                        gelu_bf16x2(acc[i][j][4 * q], acc[i][j][4 * q + 1], mk, mk),
+                        gelu_bf16x2(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3], mk, mk));
+            rows_out(a.Y, i);
+        } else if constexpr (EPI == EPI_BWD_GELU) {
+#pragma unroll
+            for (int x = 0; x < 32 * PW / 64; ++x) {
+                const int row = lane / PW + 64 / PW * x, pc = lane % PW;
+                const int64_t mu = min(m0 + 64 * wm + 32 * i + row, a.M - 1);
+                *reinterpret_cast<u32x4*>(lw + place(row, pc)) =
+                    *reinterpret_cast<const u32x4*>(a.Uprev + mu * a.N + nw + 8 * pc);
+            }
+            lds_wave_fence();
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    bf16x4* at = reinterpret_cast<bf16x4*>(lw + place(r, 4 * j + q) + 8 * h);
+                    const bf16x4 up = *at;
                     bf16x4 y;
 #pragma unroll
                     for (int x = 0; x < 4; ++x)
                         y[x] = f2bf(acc[i][j][4 * q + x] * gelu_grad(bf2f(up[x])) * mk);
-                    *reinterpret_cast<bf16x4*>(a.Y + o) = y;
-                } else {
-                    *reinterpret_cast<float4*>(a.Yf + o) =
+                    *at = y;
+                }
+            rows_out(a.Y, i);
+        } else if (in) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<float4*>(a.Yf + m * a.N + nw + 32 * j + 8 * q + 4 * h) =
                         make_float4(acc[i][j][4 * q] * mk, acc[i][j][4 * q + 1] * mk,
                                     acc[i][j][4 * q + 2] * mk, acc[i][j][4 * q + 3] * mk);
-                }
-            }
+        }
     }
 }
 
@@ -861,16 +961,6 @@ constexpr int PROP_ROWS = 128 * PROP_SUB;  // table rows per block and step
 constexpr int PROP_MAX_SLOTS = 32;         // output rows of a MAXQ launch
 static_assert(PROP_ROWS == 256, "the MAXQ fold gives each of 256 threads one table row");
 
-// Orders a wave's LDS accesses across its lanes (no barrier between waves):
-// wavefront-scope release/acquire fences keep the compiler's memory
-// operations on either side, and the hardware runs one wave's LDS
-// instructions in order.
-__device__ __forceinline__ void lds_wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Output rows of a MAXQ launch, as runs of query rows: query rows lo .. hi-1
 // are folded, bit q of starts marks the first row of a run, and output row o
 // is the maximum over the rows of run o.
@@ -1075,11 +1165,10 @@ static void launch_conv_cin(const ConvArgs& a, hipStream_t stream) {
 
 template <int EPI>
 static void launch_conv(const ConvArgs& a, hipStream_t stream) {
-    // nine whole rows of the encoder's widths, and outputs that take 8- and
-    // 16-byte accesses
-    const uintptr_t out = (uintptr_t)a.U | (uintptr_t)a.Y | (uintptr_t)a.Uprev;
-    const uintptr_t wide = (uintptr_t)a.bias | (uintptr_t)a.Yf;
-    const bool whole = a.K == 9 * a.lda && !(out & 7) && !(wide & 15);
+    // nine whole rows of the encoder's widths, and outputs that take 16-byte accesses
+    const uintptr_t out = (uintptr_t)a.U | (uintptr_t)a.Y | (uintptr_t)a.Uprev |
+                          (uintptr_t)a.bias | (uintptr_t)a.Yf;
+    const bool whole = a.K == 9 * a.lda && !(out & 15);
     if (whole && a.lda == 64) launch_conv_cin<64, EPI>(a, stream);
     else if (whole && a.lda == 128) launch_conv_cin<128, EPI>(a, stream);
     else if (whole && a.lda == 256) launch_conv_cin<256, EPI>(a, stream);

@@ -330,3 +330,29 @@ def test_topk_segments_cut(dev, dtype, sorted_):
             x = np.where(np.isnan(x), -np.inf, np.where(x == -np.inf, -1e300, x))
         want = np.argsort(-x, kind="stable")[: k[j]]
         assert np.array_equal(got[base[j]: base[j] + k[j]], want if sorted_ else np.sort(want)), segs[j]
+
+
+def test_encoder_gelu_rounding(dev):
+    """The tiled kernels' GELU equals the general kernel's on 2^21 values (all
+    magnitudes, both signs, the steep range densely) as bias of zero products,
+    on rows with and without a mask: no bf16 differs, infinities included."""
+    from sseqs_amd._lib import call, stream_of
+    announce("gelu rounding")
+    g = torch.Generator(device=dev).manual_seed(11)
+    bits = torch.randint(-2 ** 31, 2 ** 31, (1 << 20,), generator=g, device=dev, dtype=torch.int64).to(torch.int32)
+    vals = torch.cat([bits.view(torch.float32), torch.rand(1 << 20, generator=g, device=dev) * 14 - 9])
+    vals = torch.where(torch.isnan(vals), torch.full_like(vals, -float("inf")), vals)
+    N, M = 1 << 15, 128
+    A = torch.zeros(M + 8, 64, dtype=torch.bfloat16, device=dev)
+    Bt = torch.zeros(N, 576, dtype=torch.bfloat16, device=dev)
+    mask = (torch.arange(M, device=dev) % 5 != 0).to(torch.uint8)
+    for bias in vals.view(-1, N):
+        out = []
+        for shift in (0, 2):
+            Y = torch.empty(M * N + 8, dtype=torch.bfloat16, device=dev)
+            call("sseqs_enc_conv", A.data_ptr() + 8 * 64, 64, Bt.data_ptr(), M, N, 576, bias.data_ptr(),
+                 mask.data_ptr(), None, Y.data_ptr() + 2 * shift, None, None, 0, stream_of(A.device))
+            out.append(Y[shift: M * N + shift])
+        a, b = (y.view(torch.int16) for y in out)
+        assert torch.equal(torch.isnan(out[0]), torch.isnan(out[1]))
+        assert bool(((a == b) | torch.isnan(out[0])).all())
