@@ -110,6 +110,11 @@ int launch_sw_cuda_affine(const uint8_t* query_seq_indices_ptr, int query_length
 size_t sseqs_db_index_ws_bytes(int64_t n_syms);
 int sseqs_db_index(const uint8_t* packed, int64_t n_syms, int64_t* seq_off, int32_t* seq_len,
                    int64_t cap, int64_t* d_nseq, void* ws, size_t ws_bytes, hipStream_t stream);
+/* The (offset, length) pass alone, on the stream of a preceding sseqs_db_index
+ * of the same packed, n_syms and ws (for instance with cap 0, to learn the
+ * count), whose scanned tile counts ws still holds. */
+int sseqs_db_index_write(const uint8_t* packed, int64_t n_syms, int64_t* seq_off, int32_t* seq_len,
+                         int64_t cap, const void* ws, size_t ws_bytes, hipStream_t stream);
 
 /* launch_warp_corr's score for sequences s in [s_begin, s_end) of the
  * resident database (symbols unpacked on the fly from `packed`), all with

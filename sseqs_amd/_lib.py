@@ -48,6 +48,7 @@ SIGNATURES = {
     "launch_sw_cuda_affine": (_i32, [_vp, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp]),
     "sseqs_db_index_ws_bytes": (_sz, [_i64]),
     "sseqs_db_index": (_i32, [_vp, _i64, _vp, _vp, _i64, _vp, _vp, _sz, _vp]),
+    "sseqs_db_index_write": (_i32, [_vp, _i64, _vp, _vp, _i64, _vp, _sz, _vp]),
     "sseqs_db_prefilter": (_i32, [_vp, _vp, _vp, _i64, _i64, _vp, _i32, _vp, _vp, _i32, _i32, _i32,
                                   _i32, _vp, _vp]),
     "sseqs_db_prefilter_spans": (_i32, [_vp, _vp, _vp, _i64, _i64, _vp, _i32, _vp, _vp, _i32, _i32,

@@ -459,6 +459,15 @@ extern "C" size_t sseqs_db_index_ws_bytes(int64_t n_syms) {
     return (size_t)(2 * nt + ceil_div(nt, SCAN_PER) + 1) * sizeof(int64_t);
 }
 
+// tiles: the scanned tile counts, then the first-'@' table
+static int launch_idx_write(const uint8_t* packed, int64_t n_syms, int64_t* seq_off, int32_t* seq_len,
+                            int64_t cap, const int64_t* tiles, hipStream_t stream) {
+    const int64_t nt = ceil_div(n_syms, IDX_TILE);
+    hipLaunchKernelGGL(k_idx_write, dim3(grid_cap(nt, 1)), dim3(256), 0, stream, packed, n_syms, nt,
+                       tiles, tiles + nt, seq_off, seq_len, cap);
+    return check_launch("db_index write");
+}
+
 extern "C" int sseqs_db_index(const uint8_t* packed, int64_t n_syms, int64_t* seq_off,
                               int32_t* seq_len, int64_t cap, int64_t* d_nseq, void* ws,
                               size_t ws_bytes, hipStream_t stream) {
@@ -481,7 +490,18 @@ extern "C" int sseqs_db_index(const uint8_t* packed, int64_t n_syms, int64_t* se
     hipLaunchKernelGGL(k_scan_down, dim3(grid_cap(nb, 1)), dim3(1024), 0, stream, tiles, nt, part);
     if (int r = check_launch("db_index scan")) return r;
     if (cap <= 0) return 0;
-    hipLaunchKernelGGL(k_idx_write, dim3(grid_cap(nt, 1)), dim3(256), 0, stream, packed, n_syms, nt,
-                       tiles, first_at, seq_off, seq_len, cap);
-    return check_launch("db_index write");
+    return launch_idx_write(packed, n_syms, seq_off, seq_len, cap, tiles, stream);
+}
+
+extern "C" int sseqs_db_index_write(const uint8_t* packed, int64_t n_syms, int64_t* seq_off,
+                                    int32_t* seq_len, int64_t cap, const void* ws, size_t ws_bytes,
+                                    hipStream_t stream) {
+    if (n_syms <= 0) return fail(-1, "db_index_write: empty database");
+    if (!packed || !ws || (cap > 0 && (!seq_off || !seq_len)))
+        return fail(-1, "db_index_write: null pointer");
+    if (reinterpret_cast<uintptr_t>(packed) & 3)
+        return fail(-1, "db_index_write: packed must be 4-byte aligned");
+    if (ws_bytes < sseqs_db_index_ws_bytes(n_syms)) return fail(-2, "db_index_write: workspace too small");
+    if (cap <= 0) return 0;
+    return launch_idx_write(packed, n_syms, seq_off, seq_len, cap, static_cast<const int64_t*>(ws), stream);
 }

@@ -147,21 +147,23 @@ class SeqDB:
         if n_syms is None:
             n_syms = nbytes * 8 // 5
         if (n_syms * 5 + 7) // 8 + PAD > nbytes:
-            buf = torch.zeros((n_syms * 5 + 7) // 8 + PAD, dtype=torch.uint8, device=dev)
-            buf[: min(nbytes, buf.numel())] = packed[: buf.numel()]
+            buf = torch.empty((n_syms * 5 + 7) // 8 + PAD, dtype=torch.uint8, device=dev)
+            have = min(nbytes, buf.numel())
+            buf[:have] = packed[:have]
+            buf[have:].zero_()
             packed = buf
         lib = _lib.load()
         ws = _lib.workspace(lib.sseqs_db_index_ws_bytes(n_syms), dev)
         cnt = torch.zeros(1, dtype=torch.int64, device=dev)
-        # pass 1 with capacity 0 only counts; pass 2 writes
+        # capacity 0 only counts; the write pass reads the counts that ws holds
         dummy = torch.empty(1, dtype=torch.int64, device=dev)
         call("sseqs_db_index", ptr(packed), n_syms, ptr(dummy), ptr(dummy), 0, ptr(cnt), ptr(ws),
              ws.numel(), stream_of(dev))
         n = int(cnt.item())
         off = torch.empty(n, dtype=torch.int64, device=dev)
         ln = torch.empty(n, dtype=torch.int32, device=dev)
-        call("sseqs_db_index", ptr(packed), n_syms, ptr(off), ptr(ln), n, ptr(cnt), ptr(ws),
-             ws.numel(), stream_of(dev))
+        call("sseqs_db_index_write", ptr(packed), n_syms, ptr(off), ptr(ln), n, ptr(ws), ws.numel(),
+             stream_of(dev))
         orig = None
         if n > 1 and bool((ln[1:] < ln[:-1]).any().item()):
             orig = torch.sort(ln, stable=True).indices

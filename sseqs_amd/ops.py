@@ -43,7 +43,7 @@ def compress(input: torch.Tensor) -> torch.Tensor:
     x = input.contiguous().to(device="cuda" if not input.is_cuda else input.device,
                               dtype=torch.uint8)
     n = x.numel()
-    out = torch.zeros((n * 5 + 7) // 8, dtype=torch.uint8, device=x.device)
+    out = torch.empty((n * 5 + 7) // 8, dtype=torch.uint8, device=x.device)  # every byte is written
     if n:
         call("compress_launcher", ptr(x), ptr(out), n, stream_of(x.device))
     return out

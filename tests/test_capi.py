@@ -97,3 +97,19 @@ def test_prefilter_kernel_plan_needs_no_gpu():
     assert name(200, 3, 256) == "k_corr_db<4>"
     assert name(50, 4, 64) == "k_corr_db4<1>"
     assert lib.sseqs_db_prefilter_kernel(200, 4, 300, 300, buf, 64) == -1
+
+
+def test_index_write_refusals_need_no_gpu():
+    """sseqs_db_index_write refuses what sseqs_db_index refuses, before any
+    launch, and has nothing to do for a capacity of 0."""
+    from sseqs_amd import _lib
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("library not built")
+    lib = _lib.load()
+    assert lib.sseqs_db_index_write(64, 0, 8, 8, 1, 8, 1 << 20, None) == -1
+    assert lib.sseqs_db_index_write(None, 100, 8, 8, 1, 8, 1 << 20, None) == -1
+    assert lib.sseqs_db_index_write(64, 100, None, 8, 1, 8, 1 << 20, None) == -1
+    assert lib.sseqs_db_index_write(3, 100, 8, 8, 1, 8, 1 << 20, None) == -1
+    assert b"aligned" in lib.sseqs_last_error()
+    assert lib.sseqs_db_index_write(64, 100, 8, 8, 1, 8, 8, None) == -2
+    assert lib.sseqs_db_index_write(64, 100, None, None, 0, 8, 1 << 20, None) == 0

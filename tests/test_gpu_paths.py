@@ -356,3 +356,28 @@ def test_encoder_gelu_rounding(dev):
         a, b = (y.view(torch.int16) for y in out)
         assert torch.equal(torch.isnan(out[0]), torch.isnan(out[1]))
         assert bool(((a == b) | torch.isnan(out[0])).all())
+
+
+@pytest.mark.parametrize("n", [1, 39, 64, 16384, 16385, 8192 * 16384 // 64 + 7])
+def test_packed_stream_without_tail(orc, dev, n):
+    """compress and from_packed on streams around the chunks of 32 symbols and
+    the index's tiles: bytes equal to the oracle's, no byte of the output left
+    as it was allocated, runs as numpy finds them."""
+    from sseqs_amd import ops
+    from sseqs_amd.db import SeqDB
+    announce(f"packed stream n={n}")
+    rng = np.random.default_rng(n)
+    a = rng.integers(65, 91, n).astype(np.uint8)
+    a[rng.random(n) < 0.02] = 64
+    a[0] = 65
+    torch.full((1 << 20,), 255, dtype=torch.uint8, device=dev)  # what the allocator hands out again
+    packed = ops.compress(torch.from_numpy(a).to(dev))
+    assert np.array_equal(packed.cpu().numpy(), orc.xbit_pack(a))
+    db = SeqDB.from_packed(packed, n)
+    d = np.diff(np.concatenate([[0], (a != 64).astype(np.int8), [0]]))
+    off, end = np.nonzero(d == 1)[0], np.nonzero(d == -1)[0]
+    order = np.argsort(end - off, kind="stable")
+    assert np.array_equal(db.seq_off.cpu().numpy(), off[order])
+    assert np.array_equal(db.seq_len.cpu().numpy(), (end - off)[order])
+    tail = db.packed[(n * 5 + 7) // 8:]
+    assert tail.numel() >= 64 and not bool(tail.any())
