@@ -904,7 +904,11 @@ __device__ inline uint32_t seg_key(const void* s, int64_t i) {
 
 constexpr int SEG_SAMPLE = SEG_THREADS * SEG_E;
 constexpr int SEG_LIST = 12288;     // keys and indices: 96 KiB of LDS
-constexpr int64_t SEG_CUT_MAX = 256;  // segments, one to a CU: the list takes its LDS
+// Selections in index order of at least so many are of long segments (a
+// cascade takes 1/200): the list pays (710 segments of 281 000, k = 1405: 711 ->
+// 372 us). Of short segments the LDS it takes costs more than it gives (1000 of
+// 5000, k = 25: 46 -> 54 us; sorted, 710 of 1400, k = 7: 57 -> 63 us).
+constexpr int SEG_CUT_K = 128;
 
 // The rank among SEG_SAMPLE of n keys to guess at, or 0 where the passes read
 // the segment itself: below four samples there is little to save, and a list
@@ -981,19 +985,19 @@ __device__ inline void seg_steps(const void* s, int lo, int hi, int n, F f) {
     }
 }
 
-template <int DT>
+template <int DT, bool CUT>
 __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
     const void* __restrict__ s, const int64_t* __restrict__ seg_begin,
     const int32_t* __restrict__ seg_n, const int32_t* __restrict__ seg_k,
     const int64_t* __restrict__ out_base, int64_t nseg, int sorted, int drop_front,
-    int drop_back, int add_begin, int lcap, int64_t* __restrict__ out) {
+    int drop_back, int add_begin, int64_t* __restrict__ out) {
     __shared__ uint32_t hist[SEL_BINS];
     __shared__ uint64_t comp[SEG_SORT_MAX];
     __shared__ uint32_t wsum[SEG_WAVES];
     __shared__ uint32_t s_pick[2];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    extern __shared__ uint32_t l_key[];  // the list (lcap entries): keys, then indices
-    uint32_t* l_idx = l_key + lcap;
+    extern __shared__ uint32_t l_key[];  // CUT: the list, keys, then indices
+    uint32_t* l_idx = l_key + SEG_LIST;
     const int npass = DT == SSEQS_F16 ? 2 : 3;
     const int shifts16[2] = {5, 0}, bits16[2] = {11, 5};
     const int shifts32[3] = {21, 10, 0}, bits32[3] = {11, 11, 10};
@@ -1010,10 +1014,10 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
                                : static_cast<const void*>(static_cast<const int32_t*>(s) + beg);
         // round 0 (with a guess): the R-th largest key of the sample, and the
         // list of the keys that reach it; round 1: the k-th largest key
-        const int R = lcap ? seg_guess(n, k) : 0;
+        const int R = CUT ? seg_guess(n, k) : 0;
         bool listed = false;
         uint32_t prefix = 0, mask = 0, krem = 0;
-        for (int round = R > 0 ? 0 : 1; round < 2; ++round) {
+        for (int round = CUT && R > 0 ? 0 : 1; round < 2; ++round) {
             const int m = round ? n : SEG_SAMPLE;
             prefix = mask = 0;
             krem = (uint32_t)(round ? k : R);
@@ -1030,8 +1034,9 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
                     for (int e = 0; e < SEG_E; ++e) {
                         // clamped index: the loads are unconditional and all in flight
                         const int i = min(i0 + e * SEG_THREADS + tid, m - 1);
-                        key[e] = listed ? l_key[i]
-                                        : seg_key<DT>(base, round ? i : (int)((int64_t)i * n / SEG_SAMPLE));
+                        key[e] = CUT && listed
+                                     ? l_key[i]
+                                     : seg_key<DT>(base, !CUT || round ? i : (int)((int64_t)i * n / SEG_SAMPLE));
                     }
 #pragma unroll
                     for (int e = 0; e < SEG_E; ++e) {
@@ -1068,7 +1073,7 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
                 krem = s_pick[1];
                 __syncthreads();
             }
-            if (round == 0) {
+            if (CUT && round == 0) {
                 // wave w takes the w-th sixteenth of the segment, 512 elements a step
                 const int per = (n + 512 * SEG_WAVES - 1) / (512 * SEG_WAVES) * 512;
                 const int lo = min(n, wid * per), hi = min(n, lo + per);
@@ -1085,7 +1090,7 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
                     at += w < wid ? (int)wsum[w] : 0;
                     total += (int)wsum[w];
                 }
-                listed = total >= k && total <= lcap;
+                listed = total >= k && total <= SEG_LIST;
                 if (listed) {
                     seg_steps<DT>(base, lo, hi, n, [&](int i0, const SegStep<DT>& st) {
                         const uint32_t in = st.reach(i0, n, prefix);
@@ -1125,7 +1130,7 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
             uint32_t key[SEG_E];
 #pragma unroll
             for (int e = 0; e < SEG_E; ++e)
-                key[e] = listed ? l_key[min(ib + e, n - 1)] : seg_key<DT>(base, min(ib + e, n - 1));
+                key[e] = CUT && listed ? l_key[min(ib + e, n - 1)] : seg_key<DT>(base, min(ib + e, n - 1));
             uint32_t cnt = 0;
 #pragma unroll
             for (int e = 0; e < SEG_E; ++e) {
@@ -1157,7 +1162,7 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
                 const bool q = in && key[e] == T;
                 const int slot = gb + min(eb, keq);
                 if ((g || (q && eb < keq)) && slot < k) {
-                    const uint32_t at = listed ? l_idx[ib + e] : (uint32_t)(ib + e);
+                    const uint32_t at = CUT && listed ? l_idx[ib + e] : (uint32_t)(ib + e);
                     if (sorted)
                         comp[slot] = ((uint64_t)(~key[e]) << 32) | (uint64_t)at;
                     else if (slot >= drop_front && slot < hi)
@@ -1402,6 +1407,17 @@ extern "C" int sseqs_topk_noalloc(const void* scores, int dtype, int64_t n, int6
     return topk_impl(scores, dtype, n, k, sorted, out_idx, ws, false, stream);
 }
 
+template <bool CUT, class... Args>
+static void launch_segments(int dtype, unsigned grid, hipStream_t stream, Args... args) {
+    const size_t lds = CUT ? (size_t)8 * SEG_LIST : 0;
+    if (dtype == SSEQS_F32)
+        hipLaunchKernelGGL((k_seg_topk<SSEQS_F32, CUT>), dim3(grid), dim3(SEG_THREADS), lds, stream, args...);
+    else if (dtype == SSEQS_F16)
+        hipLaunchKernelGGL((k_seg_topk<SSEQS_F16, CUT>), dim3(grid), dim3(SEG_THREADS), lds, stream, args...);
+    else
+        hipLaunchKernelGGL((k_seg_topk<SSEQS_I32, CUT>), dim3(grid), dim3(SEG_THREADS), lds, stream, args...);
+}
+
 extern "C" int sseqs_topk_segments(const void* scores, int dtype, const int64_t* seg_begin,
                                    const int32_t* seg_n, const int32_t* seg_k,
                                    const int64_t* out_base, int64_t nseg, int max_k, int sorted,
@@ -1417,9 +1433,11 @@ extern "C" int sseqs_topk_segments(const void* scores, int dtype, const int64_t*
     if (!scores || !seg_begin || !seg_n || !seg_k || !out_base || !out_idx)
         return fail(-1, "topk_segments: null pointer");
     const unsigned grid = (unsigned)(nseg < 8192 ? nseg : 8192);
-    const int lcap = nseg <= SEG_CUT_MAX ? SEG_LIST : 0;
-    SEL_DISPATCH(k_seg_topk, dim3(grid), dim3(SEG_THREADS), (size_t)8 * lcap, stream, scores,
-                       seg_begin, seg_n, seg_k, out_base, nseg, sorted, drop_front, drop_back,
-                       add_begin, lcap, out_idx);
+    if (!sorted && max_k >= SEG_CUT_K)
+        launch_segments<true>(dtype, grid, stream, scores, seg_begin, seg_n, seg_k, out_base, nseg,
+                              sorted, drop_front, drop_back, add_begin, out_idx);
+    else
+        launch_segments<false>(dtype, grid, stream, scores, seg_begin, seg_n, seg_k, out_base, nseg,
+                               sorted, drop_front, drop_back, add_begin, out_idx);
     return check_launch("topk_segments");
 }
