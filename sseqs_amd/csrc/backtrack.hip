@@ -163,8 +163,10 @@ __device__ inline bt_i16x2 bt_v(uint32_t u) { return __builtin_bit_cast(bt_i16x2
 __device__ inline uint32_t bt_u(bt_i16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ inline bt_i16x2 bt_max(bt_i16x2 a, bt_i16x2 b) { return __builtin_elementwise_max(a, b); }
 
-// Longest target of k_backtrack (16-bit cells and, past it, LDS); longer ones take
-// the 32-bit k_backtrack_global.
+// Longest target of k_backtrack (its boundary row and target codes in LDS);
+// longer ones take k_backtrack_global.  Cells are 16 bits as in the definition:
+// scores wrap past 32767 (11 a residue: from 2979 residues on), as the
+// reference's int16 matrices do; k_backtrack_global's 32-bit cells do not.
 constexpr int BT_MAX_T = 5416;
 constexpr uint32_t BT_NEG2 = 0xC000C000u;  // BT_NEG in both halves
 constexpr int BT_LETTERS = 22;             // 20 residues, 20 any other letter, 21 outside the target
