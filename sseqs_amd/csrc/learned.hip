@@ -488,6 +488,12 @@ __device__ inline bf16x8 tr_frag(const uint8_t* p) {  // rows 0..3 and 4..7 of 1
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+// TAIL: M is not a multiple of WP.  dU's rows past M - 1 are zeros in LDS, but
+// the rows of X that they would meet belong to earlier rows of dU or follow
+// the sequence, and 0 times an infinity or NaN is NaN: they are cleared in the
+// fragments, by an instance of its own (312 001 rows, 128 -> 256 channels: 228
+// us, 312 000 rows 204; the encoder itself always has whole stages).
+template <bool TAIL>
 __global__ __launch_bounds__(256, 2) void k_conv_wgrad(const __bf16* __restrict__ X, int Cin,
                                                        const __bf16* __restrict__ dU, int Cout,
                                                        int64_t M, int64_t per, float* __restrict__ dW) {
@@ -545,9 +551,19 @@ __global__ __launch_bounds__(256, 2) void k_conv_wgrad(const __bf16* __restrict_
 #pragma unroll
         for (int k = 0; k < WP / 16; ++k) {
             const bf16x8 fb = tr_frag(sD[buf] + ad + 16 * k * WSTRIDE);
+            u32x4 keep;
+            if constexpr (TAIL) {
+                // of the lane's rows, eight from 8 (lane / 32) on, the ones below M
+                const int nv = (int)min((int64_t)8, M - (st * WP + 16 * k + 8 * (g >> 1)));
+#pragma unroll
+                for (int y = 0; y < 4; ++y)
+                    keep[y] = nv > 2 * y + 1 ? 0xffffffffu : nv > 2 * y ? 0xffffu : 0u;
+            }
 #pragma unroll
             for (int t = 0; t < 9; ++t) {
-                const bf16x8 fa = tr_frag(sX[buf] + ax + (16 * k + t) * WSTRIDE);
+                bf16x8 fa = tr_frag(sX[buf] + ax + (16 * k + t) * WSTRIDE);
+                if constexpr (TAIL)
+                    fa = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, fa) & keep);
                 acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb, acc[t], 0, 0, 0);
             }
         }
@@ -1207,8 +1223,8 @@ extern "C" int sseqs_enc_wgrad(const void* X, int Cin, const void* dU, int Cout,
     if (tiles == 0) return 0;
     const int64_t per = std::max(ceil_div(stages, std::max<int64_t>(1, WG_FILL / tiles)), ceil_div(stages, 65535));
     const dim3 grid((unsigned)(Cin / 64), (unsigned)(Cout / 64), (unsigned)ceil_div(stages, per));
-    hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(256), 0, stream, static_cast<const __bf16*>(X),
-                       Cin, static_cast<const __bf16*>(dU), Cout, M, per, dW);
+    hipLaunchKernelGGL(M % WP ? k_conv_wgrad<true> : k_conv_wgrad<false>, grid, dim3(256), 0, stream,
+                       static_cast<const __bf16*>(X), Cin, static_cast<const __bf16*>(dU), Cout, M, per, dW);
     return check_launch("enc_wgrad");
 }
 
