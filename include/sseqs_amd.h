@@ -122,8 +122,10 @@ int sseqs_db_index_write(const uint8_t* packed, int64_t n_syms, int64_t* seq_off
  * 0..20), lutA and lutB (k rows of vocab_size floats, flat indexing as in
  * launch_warp_corr) are device arrays.  Sequences longer than
  * min(maxlen, N) are truncated to it, as in sseqs/fft.cu:124-126.
- * N: power of two, 16..2048; k: 1..20.  Fused unpack + prefilter of the
- * resident database. */
+ * N: power of two, 16..2048; k: 1..20.  `packed` may lie at any address (the
+ * fastest rank-4 kernel for queries of up to 515 residues needs 16-byte
+ * alignment, others take its place).  Fused unpack + prefilter of the resident
+ * database. */
 int sseqs_db_prefilter(const uint8_t* packed, const int64_t* seq_off, const int32_t* seq_len,
                        int64_t s_begin, int64_t s_end, const uint8_t* qrev, int query_len,
                        const float* lutA, const float* lutB, int vocab_size, int k, int N,

@@ -565,7 +565,7 @@ __global__ __launch_bounds__(64) void k_corr_db4(const uint8_t* __restrict__ pac
 // nonzero (R == ND, d0 == 0); all m-tiles stay live and are folded at the end.
 //
 // Staging is asynchronous: while a tile is computed, the next tile's packed
-// bytes are copied global -> LDS (global_load_lds_dwordx4) into the second
+// bytes (a 16-byte aligned stream) are copied global -> LDS (global_load_lds_dwordx4) into the second
 // stage buffer (DBL) and the index entries of the one after are loaded.
 //
 // Dynamic LDS: btab4 40 x 8 B | qtab4 (N+8) x 8 B during set-up, then
@@ -1025,31 +1025,35 @@ __global__ __launch_bounds__(64, (G == 1 && R <= 8 ? 2 : 1)) void k_corr_band(
 // positions, so an '@' inside a span has its own value) or an ASCII batch
 // (bytes, masked index 256).  A tile is staged like the band kernel's: as one
 // byte range, as one slot per sequence, or not at all (symbols are then read
-// from global memory).  Only 16-byte granules that hold a symbol in use are
-// copied: whatever the address and size of the buffer, a copy stays within
-// the granules of its own bytes.
+// from global memory).  The copies take 16-byte granules at 16-byte aligned
+// addresses: `base` is the buffer's address rounded down, bit0 the bits from
+// there to symbol 0.  Only granules that hold a symbol in use are copied:
+// whatever the address and size of the buffer, a copy stays within the
+// granules of its own bytes.
 //
 // What bounds it and what it measured: see plan_prefilter.
 // ---------------------------------------------------------------------------
 struct RingPacked {
     static constexpr int BITS = 5, TAB = 33, MASKED = 32;
-    const uint8_t* base;  // 16-byte aligned
-    int64_t shift;        // symbols from base to symbol 0
+    const uint8_t* base;
+    int bit0;
     const int64_t* off;
     const int32_t* len;
     __device__ int64_t offset(int64_t s) const { return off[s]; }
     __device__ static int code(int c) { return corr_code((uint32_t)c + 64u); }
-    __device__ uint32_t sym(int64_t o, int p) const { return packed_sym(base, o + p) - 64u; }
+    __device__ uint32_t sym(int64_t o, int p) const {
+        return packed_sym(base + (bit0 >> 3), o + p) - 64u;
+    }
 };
 struct RingAscii {
     static constexpr int BITS = 8, TAB = 257, MASKED = 256;
     const uint8_t* base;
-    int64_t shift;
+    int bit0;
     const int32_t* off;
     const int32_t* len;
-    __device__ int64_t offset(int64_t s) const { return off[s] + shift; }
+    __device__ int64_t offset(int64_t s) const { return off[s]; }
     __device__ static int code(int c) { return corr_code((uint32_t)c); }
-    __device__ uint32_t sym(int64_t o, int p) const { return base[o + p]; }
+    __device__ uint32_t sym(int64_t o, int p) const { return base[(bit0 >> 3) + o + p]; }
 };
 
 template <int W, int R, bool FULL, bool DBL, class Src, class OutT>
@@ -1125,9 +1129,9 @@ __global__ __launch_bounds__(64 * W, 2) void k_corr_ring(
         *L = src.len[s_begin + sid];
     };
     // first byte of a symbol, and the 16-byte granules that hold symbols o .. o+n-1 (n > 0)
-    auto byte_of = [&](int64_t o) -> int64_t { return (S * o) >> 3; };
+    auto byte_of = [&](int64_t o) -> int64_t { return (S * o + src.bit0) >> 3; };
     auto granules = [&](int64_t b_lo, int64_t o, int64_t n) -> int64_t {
-        return (((S * (o + n) - 1) >> 3) - b_lo + 16) >> 4;
+        return (((S * (o + n) + src.bit0 - 1) >> 3) - b_lo + 16) >> 4;
     };
     struct Tile {
         int64_t o, b_lo;
@@ -1246,8 +1250,9 @@ __global__ __launch_bounds__(64 * W, 2) void k_corr_ring(
         const int C = cur.C;
         const int x = FULL ? 0 : max(0, C - ND + Rn - 1);
         // bit of this lane's sequence in the stage
-        const int relbit = cur.scb ? 128 * cur.scb * col + (int)(S * cur.o - 8 * (byte_of(cur.o) & ~(int64_t)15))
-                                   : (int)(S * cur.o - 8 * cur.b_lo);
+        const int relbit =
+            cur.scb ? 128 * cur.scb * col + (int)(S * cur.o + src.bit0 - 8 * (byte_of(cur.o) & ~(int64_t)15))
+                    : (int)(S * cur.o + src.bit0 - 8 * cur.b_lo);
         float best = -INFINITY;
         // Decode of sub-chunk q of chunk v (positions pb, pb + 1 of this lane's
         // sequence) in two steps: the stage words that hold its symbols, and
@@ -1549,6 +1554,11 @@ static RingPlan plan_ring(int N, int rn, int mlen, int bits, int tab) {
     return P;
 }
 
+static const uint8_t* ring_base(const uint8_t* p) {
+    return reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(p) & ~(uintptr_t)15);
+}
+static int ring_bit0(const uint8_t* p) { return 8 * (int)(reinterpret_cast<uintptr_t>(p) & 15); }
+
 static bool ring_fits(const RingPlan& P) { return P.W && P.lds <= 160 * 1024; }
 
 template <class Src, class OutT>
@@ -1603,9 +1613,7 @@ extern "C" int launch_warp_corr(uint16_t* corr, const uint8_t* qrev, const float
         band_diagonals(N_full, Lqe, &d0, &rn);
         const RingPlan P = plan_ring(N_full, rn, mlen, RingAscii::BITS, RingAscii::TAB);
         if (ring_fits(P)) {
-            const uintptr_t at = reinterpret_cast<uintptr_t>(flat);
-            const RingAscii src{reinterpret_cast<const uint8_t*>(at & ~(uintptr_t)15),
-                                (int64_t)(at & 15), offsets, lengths};
+            const RingAscii src{ring_base(flat), ring_bit0(flat), offsets, lengths};
             return launch_ring(P, src, 0, B, qrev, query_len, lutA, W_db, vocab_size, N_full,
                                mlen, d0, rn, reinterpret_cast<_Float16*>(corr), stream);
         }
@@ -1679,7 +1687,8 @@ static PrefilterPlan plan_prefilter(int query_len, int k, int N, int mlen, bool 
         }
     }
     // Past the band kernel's 18 diagonals (queries of about 515 residues and
-    // more), and for spans that may hold '@': the ring kernel.  4 M sequences
+    // more), for spans that may hold '@' and for a stream that is not 16-byte
+    // aligned: the ring kernel.  4 M sequences
     // (0.77 GB packed), this against the dense rank-4 kernel below: 560
     // residues 2.7 / 5.0 ms, 900 3.15 / 5.06 ms.  Bound by the matrix cores: a
     // chunk of 128 diagonal products runs at 1.6 PF/s (independent products
@@ -1755,7 +1764,9 @@ static int db_prefilter(const uint8_t* packed, const int64_t* seq_off, const int
     if (k < 1 || k > 20) return fail(-1, "db_prefilter: k must be 1..20");
     if (vocab_size < 1) return fail(-1, "db_prefilter: vocab_size must be >= 1");
     const int mlen = maxlen < 0 ? 0 : maxlen;
-    const PrefilterPlan P = plan_prefilter(query_len, k, N, mlen, allow_band);
+    // the band kernel copies 16-byte granules from `packed` on
+    const bool aligned = (reinterpret_cast<uintptr_t>(packed) & 15) == 0;
+    const PrefilterPlan P = plan_prefilter(query_len, k, N, mlen, allow_band && aligned);
     if (P.lds > 160 * 1024) return fail(-1, "db_prefilter: tables exceed LDS (reduce k or N)");
     const int64_t tiles = ceil_div(nseq, P.tile);
     const unsigned grid = (unsigned)(tiles < 8192 ? tiles : 8192);
@@ -1791,7 +1802,7 @@ static int db_prefilter(const uint8_t* packed, const int64_t* seq_off, const int
         return P.dbl ? pick(std::true_type{}) : pick(std::false_type{});
     }
     if (P.kind == PrefilterPlan::RING) {
-        const RingPacked src{packed, 0, seq_off, seq_len};
+        const RingPacked src{ring_base(packed), ring_bit0(packed), seq_off, seq_len};
         return launch_ring(P.ring, src, s_begin, nseq, qrev, query_len, lutA, lutB, vocab_size, N,
                            mlen, P.d0, P.rn, scores, stream);
     }

@@ -50,3 +50,45 @@ def test_wgrad_not_finite(dev, M):
         for t in range(9):
             want = (X[t:t + M, :, None].astype(np.float64) * dU[:, None, :]).sum(0)
             assert np.array_equal(dW[64 * t:64 * t + 64].double().cpu().numpy(), want, equal_nan=True), t
+
+
+@pytest.mark.parametrize("N,Lq", [(128, 60), (256, 200), (512, 400), (1024, 560), (1024, 1000), (2048, 1700)])
+def test_prefilter_packed_alignment(orc, dev, N, Lq):
+    """A packed stream at any address: the ring kernel's copies start at the
+    16-byte granule that holds its first byte, and the band kernel's sizes take
+    it too.  Sequences back to back and scattered, spans that hold '@', the
+    stream's last symbol in the last byte."""
+    from sseqs_amd import ops
+    from sseqs_amd._lib import call, ptr, stream_of
+    announce(f"prefilter alignment N={N} Lq={Lq}")
+    rng = np.random.default_rng(N + Lq)
+    query = rand_seq(rng, Lq)
+    A, B = orc.weighted_luts(query, 4)
+    qrev = orc.encode_query_rev(query)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)  # noqa: E731
+    lens = np.sort(np.array([0, 1, 31, 32, 33, N // 2, N - 31, N - 1, N] + list(rng.integers(1, N + 1, 40)), np.int32))
+    lutB = torch.cat([t(B).reshape(-1), torch.zeros(1, device=dev)])
+    for gap in (1, 40 * N):
+        off = np.concatenate([[0], np.cumsum(lens + gap)[:-1]]).astype(np.int32)
+        flat = np.full(int(off[-1] + lens[-1]), 64, np.uint8)
+        for o, n in zip(off, lens):
+            flat[o:o + n] = np.frombuffer((query * (N // Lq + 1)).encode(), np.uint8)[:n] if n % 3 else \
+                rng.choice(np.frombuffer((AA + "XB").encode(), np.uint8), n)
+        spans = flat.copy()
+        for o, n in zip(off, lens):
+            if n > 2:
+                spans[o + n // 2] = 64
+        for name, sym in (("sseqs_db_prefilter", flat), ("sseqs_db_prefilter_spans", spans)):
+            want = orc.corr(qrev, A, B, 4, sym.tobytes(), off, lens, N, N)
+            tol = orc.corr_tol(qrev, A, B, 4, sym.tobytes(), off, lens, N, N, want)
+            packed = ops.compress(t(sym))
+            keep = [t(off.astype(np.int64)), t(lens), t(qrev), t(A)]
+            for lead in (0, 1, 4, 8, 13):
+                buf = torch.zeros(16 + lead + packed.numel() + 64, dtype=torch.uint8, device=dev)
+                at = buf[16 + lead:]
+                at[:packed.numel()] = packed
+                assert at.data_ptr() % 16 == lead
+                out = torch.full((lens.size,), -7.0, dtype=torch.float32, device=dev)
+                call(name, ptr(at), ptr(keep[0]), ptr(keep[1]), 0, lens.size, ptr(keep[2]), Lq, ptr(keep[3]),
+                     ptr(lutB), 21, 4, N, N, ptr(out), stream_of(dev))
+                assert (np.abs(out.cpu().numpy() - want) <= tol).all(), (name, gap, lead)
