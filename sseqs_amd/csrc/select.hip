@@ -234,7 +234,7 @@ __global__ __launch_bounds__(1024) void k_sel_sample(const void* s, int64_t n, u
     const uint32_t P = lo + prefix;
     __syncthreads();
     if (t == 0) {
-        const uint32_t last = lh[(prefix >> shift) & (SEL_BINS - 1)];
+        const uint32_t last = lh[pick[0]];  // the last pass's bins, and its pick
         *st = SelState{0u, 0u, k, k, got + last <= SEL_SAMPLE / 8 ? P : 0u, 0u, 0u, 0u};
     }
 }

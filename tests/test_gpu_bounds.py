@@ -92,3 +92,30 @@ def test_prefilter_packed_alignment(orc, dev, N, Lq):
                 call(name, ptr(at), ptr(keep[0]), ptr(keep[1]), 0, lens.size, ptr(keep[2]), Lq, ptr(keep[3]),
                      ptr(lutB), 21, 4, N, N, ptr(out), stream_of(dev))
                 assert (np.abs(out.cpu().numpy() - want) <= tol).all(), (name, gap, lead)
+
+
+@pytest.mark.parametrize("bits", [5, 11, 12, 13, 17, 21, 22, 23, 28])
+def test_topk_sample_guard(dev, bits):
+    """The guess of the sampled select is dropped (P, the fifth word of the
+    state behind the histogram, is 0) when more than an eighth of the scores
+    reach it, whatever the digits of the sample's key range, and kept when
+    they do not; the indices are the same either way."""
+    from sseqs_amd import _lib
+    announce(f"topk sample guard bits={bits}")
+    n, k = 1 << 22, 10000
+    g = torch.Generator(device=dev).manual_seed(bits)
+    base = torch.randint(0, 1 << (bits - 1), (n,), generator=g, device=dev, dtype=torch.int32)
+    top = (1 << bits) - 1
+    few = torch.rand(n, generator=g, device=dev) < 0.01
+    for share, kept in ((0.01, True), (0.3, False)):
+        tied = torch.rand(n, generator=g, device=dev) < share
+        x = torch.where(tied, torch.full_like(base, top - 1), base)
+        x[few & tied] = top  # some above the tie, fewer than k
+        ws = torch.zeros(_lib.load().sseqs_topk_ws_bytes(n), dtype=torch.uint8, device=dev)
+        out = torch.empty(k, dtype=torch.int64, device=dev)
+        _lib.call("sseqs_topk", x.data_ptr(), _lib.I32, n, k, 0, out.data_ptr(), ws.data_ptr(), ws.numel(),
+                  _lib.stream_of(dev))
+        P = int(ws[2048 * 4:2048 * 4 + 32].view(torch.int32)[4].item())
+        assert (P != 0) == kept, (share, P)
+        want = torch.sort(torch.sort(x, descending=True, stable=True).indices[:k]).values
+        assert torch.equal(out, want)
