@@ -1222,13 +1222,19 @@ using namespace sseqs;
 // aligned to.  Top 100 000, sampled against all passes over the scores (us):
 // fp32 200 M 298 / 1153, 20 M 115 / 233, 8 M 102 / 137; fp16 200 M 209 / 489,
 // 8 M 89 / 109; int32 200 M 274 / 1956.  The marked scores' passes grow with
-// k: at 8 M and k = n / 64 they still win (107 / 137), at 4 M and n / 32 they
-// do not (128 / 96).
+// k, the others' with n: from 6 M on k = n / 64 is no loss (fp32 6 M 116 / 117,
+// 8 M 124 / 131; fp16 6 M 94 / 94); below, at 4 M, fp32 gains up to n / 400 (81 /
+// 85; n / 200 90 / 86, n / 64 114 / 95), fp16 up to n / 128 (75 / 77; n / 64
+// 85 / 78), and int32 at n / 64 (80 / 111).
 constexpr int64_t SEL_SAMPLE_MIN_N = 1 << 22;
-constexpr int64_t SEL_SAMPLE_MIN_RATIO = 64;
+constexpr int64_t SEL_SAMPLE_ANY_N = 6000000;
+static int64_t sel_sample_ratio(int dtype, int64_t n) {
+    if (n >= SEL_SAMPLE_ANY_N || dtype == SSEQS_I32) return 64;
+    return dtype == SSEQS_F16 ? 128 : 400;
+}
 static bool sel_sampled(const void* scores, int dtype, int64_t n, int64_t k) {
     const uintptr_t al = dtype == SSEQS_F16 ? 8 : 16;
-    return n >= SEL_SAMPLE_MIN_N && k <= n / SEL_SAMPLE_MIN_RATIO && n <= 0xffffffffLL &&
+    return n >= SEL_SAMPLE_MIN_N && k <= n / sel_sample_ratio(dtype, n) && n <= 0xffffffffLL &&
            (reinterpret_cast<uintptr_t>(scores) & (al - 1)) == 0;
 }
 

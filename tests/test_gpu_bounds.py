@@ -119,3 +119,26 @@ def test_topk_sample_guard(dev, bits):
         assert (P != 0) == kept, (share, P)
         want = torch.sort(torch.sort(x, descending=True, stable=True).indices[:k]).values
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("dtype,n,ratio", [
+    ("f32", 1 << 22, 400), ("f32", 5999999, 400), ("f32", 6000000, 64), ("f16", 1 << 22, 128), ("f16", 5999996, 128),
+    ("f16", 6000004, 64), ("i32", 1 << 22, 64), ("i32", 6000000, 64)])
+def test_topk_sample_line(dev, dtype, n, ratio):
+    """The largest selection that takes a sample's guess (P, the fifth word of
+    the state, is not 0) and one more, for the types and lengths that choose it;
+    the same indices either way."""
+    from sseqs_amd import _lib, ops
+    announce(f"topk sample line {dtype} n={n}")
+    g = torch.Generator(device=dev).manual_seed(n)
+    x = torch.randn(n, generator=g, device=dev) * 8 + 21
+    x = x.half() if dtype == "f16" else (x * 1000).int() if dtype == "i32" else x
+    order = torch.sort(x, descending=True, stable=True).indices
+    for k, sampled in ((n // ratio, True), (n // ratio + 1, False)):
+        ws = torch.zeros(_lib.load().sseqs_topk_ws_bytes(n), dtype=torch.uint8, device=dev)
+        out = torch.empty(k, dtype=torch.int64, device=dev)
+        _lib.call("sseqs_topk", x.data_ptr(), ops._DT[x.dtype], n, k, 0, out.data_ptr(), ws.data_ptr(), ws.numel(),
+                  _lib.stream_of(dev))
+        P = int(ws[2048 * 4:2048 * 4 + 32].view(torch.int32)[4].item())
+        assert (P != 0) == sampled, (k, P)
+        assert torch.equal(out, torch.sort(order[:k]).values)
