@@ -894,20 +894,29 @@ __device__ inline uint32_t key_h16(uint16_t h) {
     return (h & 0x8000u) ? (~h & 0xffffu) : (h | 0x8000u);
 }
 
+// A score as loaded, and its key.
+template <int DT>
+__device__ inline uint32_t seg_raw(const void* s, int64_t i) {
+    if constexpr (DT == SSEQS_F16) return static_cast<const uint16_t*>(s)[i];
+    else return static_cast<const uint32_t*>(s)[i];
+}
+template <int DT>
+__device__ inline uint32_t seg_key_of(uint32_t w) {
+    if constexpr (DT == SSEQS_F16) return key_h16((uint16_t)w);
+    else return load_key<DT>(&w, 0);
+}
 template <int DT>
 __device__ inline uint32_t seg_key(const void* s, int64_t i) {
-    if constexpr (DT == SSEQS_F16)
-        return key_h16(static_cast<const uint16_t*>(s)[i]);
-    else
-        return load_key<DT>(s, i);
+    return seg_key_of<DT>(seg_raw<DT>(s, i));
 }
 
 constexpr int SEG_SAMPLE = SEG_THREADS * SEG_E;
 constexpr int SEG_LIST = 12288;     // keys and indices: 96 KiB of LDS
-// Selections in index order of at least so many are of long segments (a
-// cascade takes 1/200): the list pays (710 segments of 281 000, k = 1405: 711 ->
-// 372 us). Of short segments the LDS it takes costs more than it gives (1000 of
-// 5000, k = 25: 46 -> 54 us; sorted, 710 of 1400, k = 7: 57 -> 63 us).
+// Selections in index order of at least so many take the instance that can cut
+// (a cascade selects 1/200 of segments of some 10^5: 710 of 281 000 fp16 scores,
+// k = 1405, 713 us uncut, 371 cut).  Segments that it does not cut take the time
+// of the other instance (1000 of 5000 fp32, k = 200: 68 us; 600 of 281 000 fp16,
+// k = 20 000: 756 / 697), whose LDS holds the sort instead of the list.
 constexpr int SEG_CUT_K = 128;
 
 // The rank among SEG_SAMPLE of n keys to guess at, or 0 where the passes read
@@ -922,12 +931,11 @@ __device__ inline int seg_guess(int n, int k) {
 
 typedef uint32_t seg_u32x4_el __attribute__((ext_vector_type(4), aligned(2)));
 
-// A wave's step: 512 consecutive elements, eight to a lane; SEG_U steps' loads
-// are in flight together.
-constexpr int SEG_U = 4;
+// A wave's step: 512 consecutive elements, eight to a lane; U steps' loads are in
+// flight together.
 template <int DT>
 struct SegStep {
-    static constexpr int NV = DT == SSEQS_F16 ? 1 : 2;
+    static constexpr int NV = DT == SSEQS_F16 ? 1 : 2, U = 4 / NV;
     uint32_t w[4 * NV];
     __device__ void load(const void* s, int i0) {
         const int i = i0 + 8 * (threadIdx.x & 63);
@@ -970,12 +978,13 @@ struct SegStep {
 template <int DT, class F>
 __device__ inline void seg_steps(const void* s, int lo, int hi, int n, F f) {
     int i0 = lo;
-    for (; i0 + 512 * SEG_U <= hi; i0 += 512 * SEG_U) {
-        SegStep<DT> st[SEG_U];
+    constexpr int U = SegStep<DT>::U;
+    for (; i0 + 512 * U <= hi; i0 += 512 * U) {
+        SegStep<DT> st[U];
 #pragma unroll
-        for (int u = 0; u < SEG_U; ++u) st[u].load(s, i0 + 512 * u);
+        for (int u = 0; u < U; ++u) st[u].load(s, i0 + 512 * u);
 #pragma unroll
-        for (int u = 0; u < SEG_U; ++u) f(i0 + 512 * u, st[u]);
+        for (int u = 0; u < U; ++u) f(i0 + 512 * u, st[u]);
     }
     for (; i0 < hi; i0 += 512) {
         SegStep<DT> st;
@@ -992,7 +1001,7 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
     const int64_t* __restrict__ out_base, int64_t nseg, int sorted, int drop_front,
     int drop_back, int add_begin, int64_t* __restrict__ out) {
     __shared__ uint32_t hist[SEL_BINS];
-    __shared__ uint64_t comp[SEG_SORT_MAX];
+    __shared__ uint64_t comp[CUT ? 1 : SEG_SORT_MAX];  // sorted output
     __shared__ uint32_t wsum[SEG_WAVES];
     __shared__ uint32_t s_pick[2];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -1027,30 +1036,40 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
                 const uint32_t bm = (1u << bits) - 1u;
                 for (int i = tid; i < SEL_BINS; i += SEG_THREADS) hist[i] = 0;
                 __syncthreads();
-                // SEG_E independent loads in flight per thread
-                for (int i0 = 0; i0 < m; i0 += SEG_THREADS * SEG_E) {
-                    uint32_t key[SEG_E];
+                const auto count = [&](auto get, auto key_of) {
+                    for (int i0 = 0; i0 < m; i0 += SEG_THREADS * SEG_E) {
+                        uint32_t w[SEG_E];
+                        // SEG_E independent loads in flight per thread: the index is
+                        // clamped, so that they are unconditional, and none is moved
+                        // to its use
 #pragma unroll
-                    for (int e = 0; e < SEG_E; ++e) {
-                        // clamped index: the loads are unconditional and all in flight
-                        const int i = min(i0 + e * SEG_THREADS + tid, m - 1);
-                        key[e] = CUT && listed
-                                     ? l_key[i]
-                                     : seg_key<DT>(base, !CUT || round ? i : (int)((int64_t)i * n / SEG_SAMPLE));
-                    }
+                        for (int e = 0; e < SEG_E; ++e) w[e] = get(min(i0 + e * SEG_THREADS + tid, m - 1));
+                        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int e = 0; e < SEG_E; ++e) {
-                        const int i = i0 + e * SEG_THREADS + tid;
-                        if (i < m && (key[e] & mask) == prefix)
-                            atomicAdd(&hist[(key[e] >> shift) & bm], 1u);
+                        for (int e = 0; e < SEG_E; ++e) {
+                            const uint32_t key = key_of(w[e]);
+                            if ((i0 + e * SEG_THREADS + tid < m) & ((key & mask) == prefix))
+                                atomicAdd(&hist[(key >> shift) & bm], 1u);
+                        }
                     }
-                }
+                };
+                // a loop of its own for each source of keys: one loop that asked
+                // for every key made a pass over a segment half as fast
+                const auto key_of = [](uint32_t w) { return seg_key_of<DT>(w); };
+                if (CUT && listed)
+                    count([&](int i) { return l_key[i]; }, [](uint32_t w) { return w; });
+                else if (CUT && round == 0)
+                    count([&](int i) { return seg_raw<DT>(base, (int)((int64_t)i * n / SEG_SAMPLE)); }, key_of);
+                else
+                    count([&](int i) { return seg_raw<DT>(base, i); }, key_of);
                 __syncthreads();
                 if (wid == 0) {
                     // lane L holds bins 32L..32L+31; the lane whose bins contain
                     // the krem-th largest key walks them from the top
                     uint32_t sum = 0;
-                    for (int t = 0; t < 32; ++t) sum += hist[lane * 32 + ((t + lane) & 31)];
+                    // (16-byte reads; single words from rotated places, which meet
+                    // in no bank, made a launch of short segments 4-8 us longer)
+                    for (int t = 0; t < 32; ++t) sum += hist[lane * 32 + t];
                     uint32_t incl = sum;  // keys in bins of lanes >= this one
                     for (int off = 1; off < 64; off <<= 1) {
                         const uint32_t t = __shfl_down(incl, off, 64);
@@ -1125,57 +1144,63 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_topk(
         const int64_t ob = out_base[j] - drop_front;
         const int64_t add = add_begin ? beg : 0;
         int gt_run = 0, eq_run = 0;
-        for (int i0 = 0; i0 < n; i0 += SEG_THREADS * SEG_E) {
-            const int ib = i0 + tid * SEG_E;
-            uint32_t key[SEG_E];
+        const auto write = [&](auto get, auto index) {
+            for (int i0 = 0; i0 < n; i0 += SEG_THREADS * SEG_E) {
+                const int ib = i0 + tid * SEG_E;
+                uint32_t key[SEG_E];
 #pragma unroll
-            for (int e = 0; e < SEG_E; ++e)
-                key[e] = CUT && listed ? l_key[min(ib + e, n - 1)] : seg_key<DT>(base, min(ib + e, n - 1));
-            uint32_t cnt = 0;
+                for (int e = 0; e < SEG_E; ++e)
+                    key[e] = get(min(ib + e, n - 1));
+                uint32_t cnt = 0;
 #pragma unroll
-            for (int e = 0; e < SEG_E; ++e) {
-                const bool in = ib + e < n;
-                cnt += (in && key[e] > T) ? 0x10000u : 0u;
-                cnt += (in && key[e] == T) ? 1u : 0u;
-            }
-            // inclusive scan over the wave, then over the waves
-            uint32_t inc = cnt;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const uint32_t t = __shfl_up(inc, o, 64);
-                if (lane >= o) inc += t;
-            }
-            if (lane == 63) wsum[wid] = inc;
-            __syncthreads();
-            uint32_t before = inc - cnt, total = 0;
-#pragma unroll
-            for (int w = 0; w < SEG_WAVES; ++w) {
-                const uint32_t t = wsum[w];
-                before += w < wid ? t : 0u;
-                total += t;
-            }
-            int gb = gt_run + (int)(before >> 16), eb = eq_run + (int)(before & 0xffffu);
-#pragma unroll
-            for (int e = 0; e < SEG_E; ++e) {
-                const bool in = ib + e < n;
-                const bool g = in && key[e] > T;
-                const bool q = in && key[e] == T;
-                const int slot = gb + min(eb, keq);
-                if ((g || (q && eb < keq)) && slot < k) {
-                    const uint32_t at = CUT && listed ? l_idx[ib + e] : (uint32_t)(ib + e);
-                    if (sorted)
-                        comp[slot] = ((uint64_t)(~key[e]) << 32) | (uint64_t)at;
-                    else if (slot >= drop_front && slot < hi)
-                        out[ob + slot] = add + at;
+                for (int e = 0; e < SEG_E; ++e) {
+                    const bool in = ib + e < n;
+                    cnt += (in && key[e] > T) ? 0x10000u : 0u;
+                    cnt += (in && key[e] == T) ? 1u : 0u;
                 }
-                gb += g;
-                eb += q;
+                // inclusive scan over the wave, then over the waves
+                uint32_t inc = cnt;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t t = __shfl_up(inc, o, 64);
+                    if (lane >= o) inc += t;
+                }
+                if (lane == 63) wsum[wid] = inc;
+                __syncthreads();
+                uint32_t before = inc - cnt, total = 0;
+#pragma unroll
+                for (int w = 0; w < SEG_WAVES; ++w) {
+                    const uint32_t t = wsum[w];
+                    before += w < wid ? t : 0u;
+                    total += t;
+                }
+                int gb = gt_run + (int)(before >> 16), eb = eq_run + (int)(before & 0xffffu);
+#pragma unroll
+                for (int e = 0; e < SEG_E; ++e) {
+                    const bool in = ib + e < n;
+                    const bool g = in && key[e] > T;
+                    const bool q = in && key[e] == T;
+                    const int slot = gb + min(eb, keq);
+                    if ((g || (q && eb < keq)) && slot < k) {
+                        const uint32_t at = index(ib + e);
+                        if (!CUT && sorted)
+                            comp[slot] = ((uint64_t)(~key[e]) << 32) | (uint64_t)at;
+                        else if (slot >= drop_front && slot < hi)
+                            out[ob + slot] = add + at;
+                    }
+                    gb += g;
+                    eb += q;
+                }
+                gt_run += (int)(total >> 16);
+                eq_run += (int)(total & 0xffffu);
+                __syncthreads();
             }
-            gt_run += (int)(total >> 16);
-            eq_run += (int)(total & 0xffffu);
-            __syncthreads();
-        }
-        if (sorted) {
+        };
+        if (CUT && listed)
+            write([&](int i) { return l_key[i]; }, [&](int i) { return l_idx[i]; });
+        else
+            write([&](int i) { return seg_key<DT>(base, i); }, [](int i) { return (uint32_t)i; });
+        if (!CUT && sorted) {
             int P = 1;
             while (P < k) P <<= 1;
             for (int i = k + tid; i < P; i += SEG_THREADS) comp[i] = ~0ull;
@@ -1414,14 +1439,18 @@ extern "C" int sseqs_topk_noalloc(const void* scores, int dtype, int64_t n, int6
 }
 
 template <bool CUT, class... Args>
-static void launch_segments(int dtype, unsigned grid, hipStream_t stream, Args... args) {
-    const size_t lds = CUT ? (size_t)8 * SEG_LIST : 0;
-    if (dtype == SSEQS_F32)
-        hipLaunchKernelGGL((k_seg_topk<SSEQS_F32, CUT>), dim3(grid), dim3(SEG_THREADS), lds, stream, args...);
-    else if (dtype == SSEQS_F16)
-        hipLaunchKernelGGL((k_seg_topk<SSEQS_F16, CUT>), dim3(grid), dim3(SEG_THREADS), lds, stream, args...);
-    else
-        hipLaunchKernelGGL((k_seg_topk<SSEQS_I32, CUT>), dim3(grid), dim3(SEG_THREADS), lds, stream, args...);
+static int launch_segments(int dtype, unsigned grid, hipStream_t stream, Args... args) {
+    const auto go = [&](auto kern) -> int {
+        const size_t lds = CUT ? (size_t)8 * SEG_LIST : 0;
+        if (CUT && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return fail(-3, "topk_segments: cannot enable large LDS");
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(SEG_THREADS), lds, stream, args...);
+        return check_launch("topk_segments");
+    };
+    if (dtype == SSEQS_F32) return go(&k_seg_topk<SSEQS_F32, CUT>);
+    if (dtype == SSEQS_F16) return go(&k_seg_topk<SSEQS_F16, CUT>);
+    return go(&k_seg_topk<SSEQS_I32, CUT>);
 }
 
 extern "C" int sseqs_topk_segments(const void* scores, int dtype, const int64_t* seg_begin,
@@ -1440,10 +1469,8 @@ extern "C" int sseqs_topk_segments(const void* scores, int dtype, const int64_t*
         return fail(-1, "topk_segments: null pointer");
     const unsigned grid = (unsigned)(nseg < 8192 ? nseg : 8192);
     if (!sorted && max_k >= SEG_CUT_K)
-        launch_segments<true>(dtype, grid, stream, scores, seg_begin, seg_n, seg_k, out_base, nseg,
-                              sorted, drop_front, drop_back, add_begin, out_idx);
-    else
-        launch_segments<false>(dtype, grid, stream, scores, seg_begin, seg_n, seg_k, out_base, nseg,
-                               sorted, drop_front, drop_back, add_begin, out_idx);
-    return check_launch("topk_segments");
+        return launch_segments<true>(dtype, grid, stream, scores, seg_begin, seg_n, seg_k, out_base, nseg,
+                                     sorted, drop_front, drop_back, add_begin, out_idx);
+    return launch_segments<false>(dtype, grid, stream, scores, seg_begin, seg_n, seg_k, out_base, nseg,
+                                  sorted, drop_front, drop_back, add_begin, out_idx);
 }

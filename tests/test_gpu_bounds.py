@@ -142,3 +142,28 @@ def test_topk_sample_line(dev, dtype, n, ratio):
         P = int(ws[2048 * 4:2048 * 4 + 32].view(torch.int32)[4].item())
         assert (P != 0) == sampled, (k, P)
         assert torch.equal(out, torch.sort(order[:k]).values)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32", "i32"])
+def test_topk_segments_uncut(dev, dtype):
+    """Segments that the instance with a list does not cut, next to ones that
+    it does: short ones, selections too large for the list, an empty one, all of
+    a segment, begins of any alignment."""
+    from sseqs_amd import ops
+    announce(f"topk_segments uncut {dtype}")
+    rng = np.random.default_rng(4)
+    segs = [(1, 1), (127, 127), (128, 128), (129, 128), (5000, 200), (8191, 8191), (8192, 4000), (8193, 150),
+            (32767, 160), (32768, 160), (0, 0), (100003, 30000), (300007, 20000), (281000, 1405), (70001, 70001)]
+    n = np.array([s[0] for s in segs])
+    k = np.array([s[1] for s in segs])
+    begin = np.concatenate([[1], 1 + np.cumsum(n + 1)[:-1]])
+    flat = np.round(rng.normal(21.0, 4.0, int(n.sum() + n.size + 1)) * 8) / 8  # ties
+    flat = flat.astype({"f16": np.float16, "f32": np.float32, "i32": np.int32}[dtype])
+    for drop in ((0, 0), (1, 2)):
+        got, base = ops.topk_segments(torch.from_numpy(flat).to(dev), begin, n, k, drop_front=drop[0],
+                                      drop_back=drop[1])
+        got = got.cpu().numpy()
+        for j, (nj, kj) in enumerate(segs):
+            x = flat[begin[j]: begin[j] + nj].astype(np.float64)
+            want = np.sort(np.argsort(-x, kind="stable")[:kj])[drop[0]: max(drop[0], kj - drop[1])]
+            assert np.array_equal(got[base[j]: base[j] + want.size], want), (segs[j], drop)
