@@ -360,6 +360,7 @@ __global__ __launch_bounds__(256) void k_sel_hist(const void* s, int64_t n,
         uint32_t key[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) key[e] = load_key<DT>(s, min(i0 + e * 256 + threadIdx.x, n - 1));
+        __builtin_amdgcn_sched_barrier(0);  // the loads first: the compiler waited for one of them
         // one LDS atomic per run of equal bins: tied scores and constant top
         // digits (int32 scores) would otherwise queue at one address
         uint32_t run_bin = 0, run = 0;
@@ -507,10 +508,11 @@ __global__ __launch_bounds__(256) void k_sel_count(const void* s, int64_t n,
     __shared__ int rg[256], re[256];
     for (int64_t tile = blockIdx.x; tile < nb; tile += gridDim.x) {
     const int64_t base = tile * SEL_TILE;
+    const int m = (int)min((int64_t)SEL_TILE, n - base);  // the last tile ends early
     int gt = 0, eq = 0;
 #pragma unroll 4
-    for (int j = threadIdx.x; j < SEL_TILE; j += 256) {
-        const int64_t i = base + j;
+    for (int j0 = 0; j0 < m; j0 += 256) {
+        const int64_t i = base + j0 + threadIdx.x;
         const uint32_t key = load_key<DT>(s, min(i, n - 1));
         if (i < n) {
             gt += key > T;
@@ -624,8 +626,9 @@ __global__ __launch_bounds__(256) void k_sel_write(const void* s, int64_t n,
     for (int64_t tile = blockIdx.x; tile < nb; tile += gridDim.x) {
         int64_t gt_run = bgt[tile], eq_run = beq[tile];
         const int64_t base = tile * SEL_TILE;
+        const int m = (int)min((int64_t)SEL_TILE, n - base);
         // four steps of 256 elements per barrier pair; loads first, in flight together
-        for (int j0 = 0; j0 < SEL_TILE; j0 += 1024) {
+        for (int j0 = 0; j0 < m; j0 += 1024) {
             uint32_t key[4];
             uint64_t mg[4], me[4];
 #pragma unroll

@@ -167,3 +167,21 @@ def test_topk_segments_uncut(dev, dtype):
             x = flat[begin[j]: begin[j] + nj].astype(np.float64)
             want = np.sort(np.argsort(-x, kind="stable")[:kj])[drop[0]: max(drop[0], kj - drop[1])]
             assert np.array_equal(got[base[j]: base[j] + want.size], want), (segs[j], drop)
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1023, 1025, 16383, 16384, 16385, 16384 + 1024, 3 * 16384 + 257])
+@pytest.mark.parametrize("dtype", ["f16", "f32", "i32"])
+def test_topk_last_tile(dev, dtype, n):
+    """The count and write passes end with the scores: lengths around their
+    steps of 256 and 1024 in the last tile of 16384, aligned and one score past
+    an aligned address, few and all of them selected, with ties."""
+    from sseqs_amd import ops
+    announce(f"topk last tile {dtype} n={n}")
+    g = torch.Generator(device=dev).manual_seed(n)
+    full = torch.round(torch.randn(n + 1, generator=g, device=dev) * 40)
+    full = full.half() if dtype == "f16" else full.int() if dtype == "i32" else full
+    for lead in (0, 1):
+        x = full[lead:lead + n]
+        order = torch.sort(x, descending=True, stable=True).indices
+        for k in sorted({1, (n + 3) // 4, n}):
+            assert torch.equal(ops.topk_indices(x, k, sorted=False), torch.sort(order[:k]).values), (lead, k)
