@@ -29,6 +29,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace sseqs {
 
@@ -469,15 +470,15 @@ __global__ __launch_bounds__(256) void k_conv_any(ConvArgs a) {
 // LDS through transposing reads, for which a tap is a row offset.  The next
 // stage's global loads are issued before the current stage's products.  The
 // block's sums are added to dW (fp32) atomically at the end.  Bound by the
-// products and those additions: WG_FILL blocks a layer, two to a CU (one to a
-// CU: 520 us).  312 k rows, three layers: 1000 -> 445 us against 64 x 64 tiles
-// of one tap whose operands were gathered from LDS two bytes at a time.
+// products and those additions (wg_slices).  312 k rows, three layers: 1000 -> 445
+// us against 64 x 64 tiles of one tap whose operands were gathered from LDS two
+// bytes at a time.
 //
 // ds_read_b64_tr_b16: of 16 lanes, lane 4 j + q reads the four elements q of
 // row j of a 4 x 16 tile, and lane l receives column l: its four rows.
 constexpr int WP = 64;           // rows per stage
 constexpr int WSTRIDE = 192;     // bytes of a row of 64 channels: rows j .. j + 3 meet in no bank
-constexpr int64_t WG_FILL = 512;
+constexpr int64_t WG_FILL = 512;  // blocks that are resident at once, two to a CU
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -1215,13 +1216,24 @@ extern "C" int sseqs_enc_conv(const void* A, int lda, const void* Bt, int64_t M,
     return check_launch("enc_conv");
 }
 
+// Blocks along the rows.  A stage takes a block 1.26 us, the blocks' additions
+// 0.13 us for each 64 x 64 tile of dW and slice, one slice after the other on the
+// same addresses: 1.26 stages / slices + 0.13 tiles slices is least at 3.1
+// sqrt(stages / tiles).  128 -> 256 channels, against filling all WG_FILL places for
+// any number of rows: 2048 rows 34 -> 14 us, 20 000 rows 70 -> 41, 100 000 rows 104 -> 97;
+// from about 220 000 rows on the places are the bound.
+static int64_t wg_slices(int64_t stages, int64_t tiles) {
+    const int64_t s = (int64_t)(3.1 * sqrt((double)stages / (double)tiles) + 0.5);
+    return std::max<int64_t>(1, std::min(s, WG_FILL / tiles));
+}
+
 extern "C" int sseqs_enc_wgrad(const void* X, int Cin, const void* dU, int Cout, int64_t M,
                                float* dW, hipStream_t stream) {
     if (M <= 0 || Cin % 64 || Cout % 64) return fail(-1, "enc_wgrad: bad sizes");
     if (ceil_div(M, 2048) > 65535) return fail(-1, "enc_wgrad: at most 65535 * 2048 rows");
     const int64_t tiles = (int64_t)(Cin / 64) * (Cout / 64), stages = ceil_div(M, WP);
     if (tiles == 0) return 0;
-    const int64_t per = std::max(ceil_div(stages, std::max<int64_t>(1, WG_FILL / tiles)), ceil_div(stages, 65535));
+    const int64_t per = std::max(ceil_div(stages, wg_slices(stages, tiles)), ceil_div(stages, 65535));
     const dim3 grid((unsigned)(Cin / 64), (unsigned)(Cout / 64), (unsigned)ceil_div(stages, per));
     hipLaunchKernelGGL(M % WP ? k_conv_wgrad<true> : k_conv_wgrad<false>, grid, dim3(256), 0, stream,
                        static_cast<const __bf16*>(X), Cin, static_cast<const __bf16*>(dU), Cout, M, per, dW);

@@ -185,3 +185,35 @@ def test_topk_last_tile(dev, dtype, n):
         order = torch.sort(x, descending=True, stable=True).indices
         for k in sorted({1, (n + 3) // 4, n}):
             assert torch.equal(ops.topk_indices(x, k, sorted=False), torch.sort(order[:k]).values), (lead, k)
+
+
+@pytest.mark.parametrize("M,cin,cout", [(64, 64, 64), (128, 128, 256), (64 * 9 + 1, 64, 64), (64 * 64, 64, 128),
+                                        (64 * 333, 128, 256), (64 * 1400, 64, 64)])
+def test_gradient_sums_exact(dev, M, cin, cout):
+    """Weight, bias and embedding gradients of small whole numbers, whose fp32
+    sums are exact in any order: one lost or doubled row or stage shows.  Row
+    counts of one slice, of a few stages each and of many blocks."""
+    from sseqs_amd._lib import call, stream_of
+    announce(f"exact gradient sums M={M} cin={cin} cout={cout}")
+    g = torch.Generator(device=dev).manual_seed(M + cin + cout)
+    small = lambda *s: torch.randint(-3, 4, s, generator=g, device=dev)  # noqa: E731
+    X = torch.zeros(M + 8, cin, device=dev)
+    X[4:-4] = small(M, cin)
+    dU = small(M, cout).float()
+    tX, tU, st = X.to(torch.bfloat16), dU.to(torch.bfloat16), stream_of(X.device)
+    assert 9 * M < 2 ** 23  # the largest sum there can be, and the start of 3
+    dW = torch.full((9 * cin, cout), 3.0, device=dev)
+    call("sseqs_enc_wgrad", tX.data_ptr() + 8 * cin, cin, tU.data_ptr(), cout, M, dW.data_ptr(), st)
+    for t in range(9):
+        want = X[t:t + M].double().T @ dU.double() + 3
+        assert torch.equal(dW[t * cin:(t + 1) * cin].double(), want), t
+    db = torch.full((cout,), 3.0, device=dev)
+    call("sseqs_enc_bias_grad", tU.data_ptr(), cout, M, db.data_ptr(), st)
+    assert torch.equal(db.double(), dU.double().sum(0) + 3)
+    code = torch.randint(0, 22, (M,), generator=g, device=dev).to(torch.uint8)
+    dx = small(M, 64).float()
+    dE = torch.full((22, 64), 3.0, device=dev)
+    call("sseqs_enc_embed_grad", code.data_ptr(), M, dx.data_ptr(), dE.data_ptr(), st)
+    want = torch.zeros(22, 64, dtype=torch.float64, device=dev).index_add_(0, code.long(), dx.double())
+    want[20:] = 0
+    assert torch.equal(dE.double(), want + 3)
