@@ -737,7 +737,11 @@ __global__ __launch_bounds__(256) void k_pool(const __bf16* __restrict__ h3,
 // gridDim.y-th group of eight rows, a thread eight channels of one row from
 // one 16-byte load.  Bound by gelu' (tanh).  1056 sequences, 312 k rows:
 // 553 -> 100 us against one block and one row at a time per sequence.
+// A split costs dz once more: at most PG_SPLIT blocks a sequence, and no more than
+// make PG_BLOCKS in all (64 sequences of 1000 rows: 1 block 142 us, 8 27; 1056 of
+// 300: 102, 4 or 8 81; 5000 of 10: 19, 8 34; 100 000 of 3: 184, 8 588).
 constexpr int PG_SPLIT = 8;
+constexpr int64_t PG_BLOCKS = 4096;
 __global__ __launch_bounds__(256) void k_pool_grad(const float* __restrict__ de,
                                                    const float* __restrict__ e,
                                                    const float* __restrict__ znorm,
@@ -1277,7 +1281,8 @@ extern "C" int sseqs_enc_pool_grad(const float* de, const float* e, const float*
                                    const void* U3, const int64_t* row0, const int32_t* len,
                                    int64_t nseq, void* dU3, hipStream_t stream) {
     if (nseq <= 0) return 0;
-    hipLaunchKernelGGL(k_pool_grad, dim3(grid_cap(nseq, 1), PG_SPLIT), dim3(256), 0, stream, de, e, znorm,
+    const unsigned split = (unsigned)std::min<int64_t>(PG_SPLIT, ceil_div(PG_BLOCKS, nseq));
+    hipLaunchKernelGGL(k_pool_grad, dim3(grid_cap(nseq, 1), split), dim3(256), 0, stream, de, e, znorm,
                        static_cast<const __bf16*>(U3), row0, len, nseq, static_cast<__bf16*>(dU3));
     return check_launch("enc_pool_grad");
 }

@@ -217,3 +217,31 @@ def test_gradient_sums_exact(dev, M, cin, cout):
     want = torch.zeros(22, 64, dtype=torch.float64, device=dev).index_add_(0, code.long(), dx.double())
     want[20:] = 0
     assert torch.equal(dE.double(), want + 3)
+
+
+@pytest.mark.parametrize("nseq,most", [(1, 70), (511, 40), (512, 17), (513, 17), (1056, 40), (2048, 9), (4095, 20),
+                                       (4096, 20), (70000, 3)])
+def test_pool_gradient_split(dev, nseq, most):
+    """The pool's gradient for the numbers of sequences that choose its blocks
+    per sequence, past the grid's 65536 blocks too, equals that of 256 sequences
+    at a time bit for bit: every row of every sequence, no row between them."""
+    from sseqs_amd._lib import call, stream_of
+    announce(f"pool gradient nseq={nseq}")
+    g = torch.Generator(device=dev).manual_seed(nseq)
+    lens = torch.randint(0, most + 1, (nseq,), generator=g, device=dev)
+    lens[-1] = most
+    row0 = 4 + torch.cumsum(lens + 2, 0) - (lens + 2)
+    M = int((row0[-1] + lens[-1] + 4).item())
+    e = torch.nn.functional.normalize(torch.randn(nseq, 256, generator=g, device=dev), dim=1)
+    de = torch.randn(nseq, 256, generator=g, device=dev)
+    zn = torch.rand(nseq, generator=g, device=dev) + 0.5
+    U = torch.randn(M, 256, generator=g, device=dev).to(torch.bfloat16)
+    tl = lens.to(torch.int32)
+    out, want = (torch.full((M, 256), 7.0, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    grad = lambda a, b, t: call("sseqs_enc_pool_grad", de[a:].data_ptr(), e[a:].data_ptr(), zn[a:].data_ptr(),  # noqa: E731
+                                U.data_ptr(), row0[a:].data_ptr(), tl[a:].data_ptr(), b - a, t.data_ptr(),
+                                stream_of(e.device))
+    grad(0, nseq, out)
+    for a in range(0, nseq, 256):  # the most blocks a sequence, against 64 bits in test_encoder_pool_gradient_rows
+        grad(a, min(a + 256, nseq), want)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
