@@ -392,11 +392,25 @@ __device__ __forceinline__ void sw16_quad(const Src& src, int64_t quad, int64_t 
     if (l == 0 && g < n) out[g] = valid ? bv : -1;
 }
 
+// Waves per SIMD that the compiler may aim at (8: all that the LDS admits).  The
+// affine cells of 21-24 and 29-32 columns a lane want 170 and 180-200 registers,
+// more than the 128 and 168 of the four and three waves that their LDS admits:
+// held to those, the rows were full of waits, and a launch that gives each wave a
+// SIMD of its own was slower than k_sw (ASCII targets, 2048 of 400: 700 residues
+// 235 us, k_sw 218, with this 179; 928: 300, 274, 229; 1024: 314, 292, 270).  Launches
+// that fill the chip take the same time (40 000 at 700 residues 1440 and 1434 us),
+// with packed targets 5 % more, and those keep the default.
 template <int TPT, bool AFFINE, class Src>
-__global__ __launch_bounds__(64 * SW16_WAVES) void k_sw16(Src src,
-                                                         const uint8_t* __restrict__ query,
-                                                         int Lq, int64_t n, int p1, int p2,
-                                                         int32_t* __restrict__ out, Blosum bl) {
+constexpr int sw16_waves() {
+    constexpr int NW = (TPT + 3) / 4;
+    return AFFINE && std::is_same<Src, SrcAscii>::value && (NW == 6 || NW == 8) ? 2 : 8;
+}
+
+template <int TPT, bool AFFINE, class Src>
+__global__ __launch_bounds__(64 * SW16_WAVES)
+    __attribute__((amdgpu_waves_per_eu(1, sw16_waves<TPT, AFFINE, Src>()))) void k_sw16(
+        Src src, const uint8_t* __restrict__ query, int Lq, int64_t n, int p1, int p2,
+        int32_t* __restrict__ out, Blosum bl) {
     constexpr int NW = (TPT + 3) / 4;
     __shared__ int8_t s_bl[400];
     __shared__ uint4 s_prof[21 * NW * 16];
@@ -510,8 +524,9 @@ static int launch_sw(const Src& src, const uint8_t* q, int Lq, int64_t n, int p1
     // Both sources take the packed kernel wherever it is exact (sw16_ok): VALU
     // issue bounds both kernels, and it advances two cells per instruction.
     // ASCII targets, affine, 40 000 of mean length 284 at 350 residues: 636 us
-    // (6.3 T cells/s) against 1183 us on k_sw; 32 targets at 120 residues, a
-    // latency chain of rows: 129 against 154 us for the whole call.
+    // (6.3 T cells/s) against 1183 us on k_sw; 32 targets of 300 at 120 residues, a
+    // latency chain of rows: 33 against 47 us (the whole `sw` call, with its host
+    // work, 0.13 ms either way within the spread of its timings).
     if (sw16_ok(Lq, AFFINE, p1, p2)) {
         const int64_t quads = ceil_div(n, 4 * SW16_WAVES);
         const unsigned grid16 = (unsigned)(quads < 8192 ? quads : 8192);

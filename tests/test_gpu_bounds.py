@@ -245,3 +245,22 @@ def test_pool_gradient_split(dev, nseq, most):
     for a in range(0, nseq, 256):  # the most blocks a sequence, against 64 bits in test_encoder_pool_gradient_rows
         grad(a, min(a + 256, nseq), want)
     assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("Lq", [640, 641, 672, 673, 768, 769, 896, 897, 928, 929, 1023, 1024])
+def test_ascii_affine_stripes(orc, dev, Lq):
+    """Affine SW of ASCII targets at the stripe widths around which the packed
+    kernel's registers change."""
+    from sseqs_amd import ops
+    announce(f"ascii affine stripes Lq={Lq}")
+    rng = np.random.default_rng(Lq)
+    query = rand_seq(rng, Lq, AA + "X")
+    tg = [query, query[Lq // 3:] + rand_seq(rng, 40), "", rand_seq(rng, 300, AA + "XB*"), query[:200][::-1], "W" * 700,
+          query[: Lq // 2] + rand_seq(rng, 31) + query[Lq // 2 + 7:]] * 3
+    a = np.frombuffer(("@".join(tg) + "@").encode(), np.uint8).copy()
+    P = np.nonzero(a == 64)[0].astype(np.int32)
+    gi = np.arange(P.size, dtype=np.int32)
+    qc = orc.encode_query_sw(query)
+    t = [torch.from_numpy(x).to(dev) for x in (qc, gi, a, P)]
+    for o, e in ((11, 1), (0, 0), (3, 7)):
+        assert np.array_equal(ops.sw_cuda_affine(*t, o, e).cpu().numpy(), orc.sw_affine(qc, gi, a, P, o, e)), (o, e)
