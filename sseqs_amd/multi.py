@@ -53,6 +53,11 @@ SW_CLASSES = ((1, 8), (9, 16), (17, 32))
 # 5.8 ms at 16 (7.6 T cells/s), 8.0 at 32, 12.5 at 64 and 37.5 at 256;
 # 8 x 100 000 take 15.2, 15.9, 17.6 and 42 ms.
 DEFAULT_SW = {"item": 16, "blocks_per_cu": 4}
+# A queue of many more items gains nothing and its table (8 bytes an item, made
+# on the host) only grows: past this many, items are doubled.  One query x 1 M
+# candidates takes 18.02 ms in 62 500 items, 18.10 in 15 600, 18.6 in 3900; the
+# tables of 64 queries x 4 M take 128 MB and 17.6 ms in items of 16.
+SW_QUEUE_ITEMS = 32768
 N_CU = 256
 
 
@@ -71,6 +76,15 @@ def sw_params(tuning: dict, tpt: int) -> dict:
         if lo <= tpt <= hi:
             return dict(DEFAULT_SW, **tuning.get("sw", {}).get(f"{lo}-{hi}", {}))
     return dict(DEFAULT_SW)
+
+
+def sw_item(item: int, counts) -> int:
+    """Candidates per work item of one SW queue: ``item``, doubled while the
+    queries' ``counts`` of candidates make more than SW_QUEUE_ITEMS items."""
+    item = int(item)
+    while sum(-(-int(c) // item) for c in counts) > SW_QUEUE_ITEMS and item < max(counts):
+        item *= 2
+    return item
 
 
 @contextmanager
@@ -199,7 +213,7 @@ class MultiSearch:
 
     def set_sw_tuning(self, tuning: dict) -> None:
         """Plan the SW queues: one per stripe width (widest first), items
-        (query, chunk of ``item`` candidates) in query order, a query's
+        (query, chunk of ``sw_item`` candidates) in query order, a query's
         chunks from its last to its first: candidate ids ascend with the
         sequence length, so the longest targets start first and the queue's
         tail is made of short ones (5.8 against 6.5 ms in the first order)."""
@@ -209,7 +223,7 @@ class MultiSearch:
         for tpt in sorted({int((L + 31) // 32) for L in lens if L <= 1024}, reverse=True):
             qi = [i for i in range(self.nq) if lens[i] <= 1024 and (lens[i] + 31) // 32 == tpt]
             prm = sw_params(self.tuning, tpt)
-            item = int(prm["item"])
+            item = sw_item(prm["item"], [self.kc_q[i] for i in qi])
             per = [-(-int(self.kc_q[i]) // item) for i in qi]
             iq = np.repeat(np.array(qi, np.int32), per)
             ij = np.concatenate([np.arange(p, dtype=np.int32)[::-1] for p in per])

@@ -39,7 +39,7 @@ import torch
 
 from . import _lib
 from .db import SeqDB
-from .multi import BT_STREAMS, MultiSearch
+from .multi import BT_STREAMS, DEFAULT_SW, SW_QUEUE_ITEMS, MultiSearch
 
 
 @dataclass
@@ -60,13 +60,14 @@ class EngineStats:
 
 def query_bytes(db: SeqDB, q_len: int, top_prefilter: int, top_hits: int,
                 hit_width: int = 500) -> int:
-    """Device bytes one query holds in a sweep: candidate ids and scores,
-    hit ids/scores/positions, and its backtrack rows (aligned query and
-    target, right-aligned, and the alignment info)."""
+    """Device bytes one query holds in a sweep: candidate ids and scores, its
+    SW work items, hit ids/scores/positions, and its backtrack rows (aligned
+    query and target, right-aligned, and the alignment info)."""
     kc = min(top_prefilter, db.n)
     kh = min(top_hits, kc)
     A = q_len + hit_width + 1
-    return kc * 12 + kh * 20 + kh * A * 2 + kh * 24
+    items = min(-(-kc // DEFAULT_SW["item"]), SW_QUEUE_ITEMS)
+    return kc * 12 + items * 8 + kh * 20 + kh * A * 2 + kh * 24
 
 
 def sweep_bytes(db: SeqDB, lq_max: int, top_hits: int, hit_width: int = 500) -> int:
