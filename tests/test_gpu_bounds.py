@@ -264,3 +264,37 @@ def test_ascii_affine_stripes(orc, dev, Lq):
     t = [torch.from_numpy(x).to(dev) for x in (qc, gi, a, P)]
     for o, e in ((11, 1), (0, 0), (3, 7)):
         assert np.array_equal(ops.sw_cuda_affine(*t, o, e).cpu().numpy(), orc.sw_affine(qc, gi, a, P, o, e)), (o, e)
+
+
+@pytest.mark.parametrize("sign", [1, -1])
+def test_encoder_gelu_every_float(dev, sign):
+    """The tiled kernels' GELU equals the general kernel's for every normal fp32
+    number: the upper seven bits of the mantissa come as a product with 1, the
+    lower sixteen as a bias, and the sum is exact.  (Subnormal numbers and
+    infinities: test_encoder_gelu_rounding.)"""
+    from sseqs_amd._lib import call, stream_of
+    announce(f"gelu of every float, sign {sign}")
+    M, N = 128, 1 << 16
+    A = torch.zeros(M + 8, 64, dtype=torch.bfloat16, device=dev)
+    Bt = torch.zeros(N, 576, dtype=torch.bfloat16, device=dev)
+    Bt[:, 4 * 64] = 1  # the row itself, channel 0
+    mask = torch.ones(M, dtype=torch.uint8, device=dev)
+    U, Y, Z = (torch.empty(M * N + 8, dtype=torch.bfloat16, device=dev) for _ in range(3))
+    hi = torch.arange(128, device=dev, dtype=torch.int64) << 16
+    low = torch.arange(N, device=dev, dtype=torch.int64)
+    neg = -2 ** 31 if sign < 0 else 0
+    st = stream_of(A.device)
+    bad = torch.zeros((), dtype=torch.int64, device=dev)
+    for e in range(1, 255):  # the exponent's field
+        head = ((e << 23) | hi) + neg
+        A[4:-4, 0] = head.to(torch.int32).view(torch.float32).to(torch.bfloat16)
+        one = torch.tensor([(e << 23) + neg], device=dev).to(torch.int32).view(torch.float32)
+        bias = (((e << 23) | low) + neg).to(torch.int32).view(torch.float32) - one
+        for out, shift in ((Y, 0), (Z, 2)):  # 2: not 16-byte aligned, the general kernel
+            call("sseqs_enc_conv", A.data_ptr() + 8 * 64, 64, Bt.data_ptr(), M, N, 576, bias.data_ptr(), mask.data_ptr(),
+                 U.data_ptr() if shift == 0 else None, out.data_ptr() + 2 * shift, None, None, 0, st)
+        bad += (Y[:M * N].view(torch.int16) != Z[2:M * N + 2].view(torch.int16)).sum()
+        x = (head[:, None] + low[None, :]).to(torch.int32).view(torch.float32)
+        if e in (1, 100, 127, 254):  # the numbers are the ones meant
+            assert torch.equal(U[:M * N].view(M, N).view(torch.int16), x.to(torch.bfloat16).view(torch.int16)), e
+    assert int(bad) == 0
