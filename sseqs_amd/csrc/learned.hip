@@ -68,11 +68,11 @@ __device__ inline float gelu_grad(float x) {
 // instructions, twice the products' own time in the narrow layers.  Here
 // tanh u = 2 g - 1 with g = 1 / (1 + exp(-2u)) comes from the hardware's
 // exponential and reciprocal, once with g a little too small and once a little
-// too large (GELU_EPS: for every float the tanhf of gelu() lies between, and
-// the rounding to 24 bits that makes 1 + tanh u coarse for negative u is the
-// same).  Each further step is monotonic, so where both ends round to one
-// bf16 that is gelu's; where they differ (about 1 in 2000), gelu() itself is
-// evaluated.
+// too large (GELU_EPS).  Each further step is monotonic, so where both ends round
+// to one bf16 that is gelu's; where they differ (about 1 in 2000), gelu() itself
+// is evaluated.  That the tanhf of gelu() lies between them, its rounding of
+// 1 + tanh u for negative u included, is a fact about the installed tanhf: a test
+// compares all normal floats.
 constexpr float GELU_EPS = 3e-6f;
 __device__ inline uint32_t gelu_bf16x2(float x0, float x1, float m0, float m1) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
