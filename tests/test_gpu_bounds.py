@@ -298,3 +298,44 @@ def test_encoder_gelu_every_float(dev, sign):
         if e in (1, 100, 127, 254):  # the numbers are the ones meant
             assert torch.equal(U[:M * N].view(M, N).view(torch.int16), x.to(torch.bfloat16).view(torch.int16)), e
     assert int(bad) == 0
+
+
+@pytest.mark.parametrize("N,Lq", [(64, 50), (128, 100), (256, 200), (512, 400), (1024, 700), (2048, 1500)])
+@pytest.mark.parametrize("mt", [None, "1"])
+def test_prefilter_without_band(orc, dev, monkeypatch, N, Lq, mt):
+    """SSEQS_CORR_NO_BAND takes every rank-4 size to the dense kernels (m-tiles
+    per pass capped by SSEQS_CORR_MT) and the ASCII operator to the general one:
+    scores within the tolerance, and the kernels' names say so."""
+    from sseqs_amd import ops
+    from sseqs_amd._lib import call, ptr, stream_of
+    from sseqs_amd.search import prefilter_kernel_name
+    announce(f"prefilter without band N={N} Lq={Lq} mt={mt}")
+    monkeypatch.setenv("SSEQS_CORR_NO_BAND", "1")
+    if mt:
+        monkeypatch.setenv("SSEQS_CORR_MT", mt)
+    passes = min(N // 64, 4 if N <= 512 else 8)
+    assert prefilter_kernel_name(Lq, 4, N) == f"k_corr_db4<{1 if mt else passes}>"
+    rng = np.random.default_rng(N + Lq)
+    query = rand_seq(rng, Lq)
+    A, B = orc.weighted_luts(query, 4)
+    qrev = orc.encode_query_rev(query)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)  # noqa: E731
+    lens = np.sort(np.array([1, 15, 16, 17, N // 2, N - 1, N] + list(rng.integers(1, N + 1, 70)), np.int32))
+    off = np.concatenate([[0], np.cumsum(lens + 1)[:-1]]).astype(np.int32)
+    flat = np.full(int(off[-1] + lens[-1] + 1), 64, np.uint8)
+    for o, n in zip(off, lens):
+        flat[o:o + n] = np.frombuffer((query * (N // Lq + 1)).encode(), np.uint8)[:n] if n % 3 else \
+            rng.choice(np.frombuffer((AA + "XB").encode(), np.uint8), n)
+    want = orc.corr(qrev, A, B, 4, flat.tobytes(), off, lens, N, N)
+    tol = orc.corr_tol(qrev, A, B, 4, flat.tobytes(), off, lens, N, N, want)
+    packed = torch.cat([ops.compress(t(flat)), torch.zeros(64, dtype=torch.uint8, device=dev)])
+    keep = [t(off.astype(np.int64)), t(lens), t(qrev), t(A), torch.cat([t(B).reshape(-1), torch.zeros(1, device=dev)])]
+    for name in ("sseqs_db_prefilter", "sseqs_db_prefilter_spans"):
+        out = torch.empty(lens.size, dtype=torch.float32, device=dev)
+        call(name, ptr(packed), ptr(keep[0]), ptr(keep[1]), 0, lens.size, ptr(keep[2]), Lq, ptr(keep[3]), ptr(keep[4]),
+             21, 4, N, N, ptr(out), stream_of(dev))
+        assert (np.abs(out.cpu().numpy() - want) <= tol).all(), name
+    scores = torch.zeros(lens.size, dtype=torch.float16, device=dev)
+    ops.warp_corr(scores, keep[2], keep[3], t(B), t(flat), t(off), keep[1], 4, Lq, N, N,
+                  torch.zeros(1, dtype=torch.float16, device=dev))
+    assert (np.abs(scores.float().cpu().numpy() - want) <= tol).all()
