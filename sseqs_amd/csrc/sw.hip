@@ -525,8 +525,7 @@ static int launch_sw(const Src& src, const uint8_t* q, int Lq, int64_t n, int p1
     // issue bounds both kernels, and it advances two cells per instruction.
     // ASCII targets, affine, 40 000 of mean length 284 at 350 residues: 636 us
     // (6.3 T cells/s) against 1183 us on k_sw; 32 targets of 300 at 120 residues, a
-    // latency chain of rows: 33 against 47 us (the whole `sw` call, with its host
-    // work, 0.13 ms either way within the spread of its timings).
+    // latency chain of rows: 33 against 47 us.
     if (sw16_ok(Lq, AFFINE, p1, p2)) {
         const int64_t quads = ceil_div(n, 4 * SW16_WAVES);
         const unsigned grid16 = (unsigned)(quads < 8192 ? quads : 8192);

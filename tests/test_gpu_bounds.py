@@ -339,3 +339,30 @@ def test_prefilter_without_band(orc, dev, monkeypatch, N, Lq, mt):
     ops.warp_corr(scores, keep[2], keep[3], t(B), t(flat), t(off), keep[1], 4, Lq, N, N,
                   torch.zeros(1, dtype=torch.float16, device=dev))
     assert (np.abs(scores.float().cpu().numpy() - want) <= tol).all()
+
+
+def test_topk_segments_captured(dev):
+    """The segmented select that cuts long segments, captured in a graph: the
+    same indices on every replay, with eager work between the replays."""
+    from sseqs_amd import _lib
+    announce("topk_segments captured")
+    g = torch.Generator(device=dev).manual_seed(9)
+    n, k, nseg = 50000, 300, 6
+    x = torch.randn(nseg * n, generator=g, device=dev).half()
+    begin = torch.arange(nseg, device=dev) * n
+    base = torch.arange(nseg, device=dev) * k
+    nn, kk = (torch.full((nseg,), v, dtype=torch.int32, device=dev) for v in (n, k))
+    out = torch.zeros(nseg * k, dtype=torch.int64, device=dev)
+    call = lambda: _lib.call("sseqs_topk_segments", x.data_ptr(), _lib.F16, begin.data_ptr(), nn.data_ptr(),  # noqa: E731
+                             kk.data_ptr(), base.data_ptr(), nseg, k, 0, 0, 0, 0, out.data_ptr(), _lib.stream_of(dev))
+    want = lambda: torch.cat([torch.sort(torch.sort(s, descending=True, stable=True).indices[:k]).values  # noqa: E731
+                              for s in x.view(nseg, n)])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for i in range(3):
+        x.copy_(torch.randn(nseg * n, generator=g, device=dev).half())
+        out.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want()), i
