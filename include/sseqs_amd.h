@@ -135,8 +135,8 @@ int sseqs_db_prefilter(const uint8_t* packed, const int64_t* seq_off, const int3
  * the per-batch cascade's segments of a batch whose `lengths != 0` filter
  * shifted its offsets (sseqs/msa.py:253,266-267), where the reference's
  * ASCII prefilter scores an in-span '@' through LUT code 21
- * (sseqs/fft.cu:5-15,91-93).  Always uses the generic kernels, which do the
- * same; arguments as sseqs_db_prefilter. */
+ * (sseqs/fft.cu:5-15,91-93).  Never uses the band kernel, which masks it;
+ * arguments as sseqs_db_prefilter. */
 int sseqs_db_prefilter_spans(const uint8_t* packed, const int64_t* seq_off,
                              const int32_t* seq_len, int64_t s_begin, int64_t s_end,
                              const uint8_t* qrev, int query_len, const float* lutA,

@@ -1714,9 +1714,10 @@ static PrefilterPlan plan_prefilter(int query_len, int k, int N, int mlen, bool 
     P.lds = ((size_t)k * (N + 8) * 2 + (size_t)k * CORR_NB * 2 + (size_t)P.capb + 64 + 15) &
             ~(size_t)15;
     P.nmt = N >= 64 ? N / 64 : 1;
-    // m-tiles per pass: more reuse of each decoded B fragment against more
-    // registers (8 -> 1 wave per SIMD, 4 -> 2).  Measured on gfx950 with
-    // rank 4: N = 512 runs fastest at 4, N = 1024 and 2048 at 8.
+    // The dense kernels: other ranks, N < 128 and, under SSEQS_CORR_NO_BAND, any
+    // rank-4 size.  m-tiles per pass: more reuse of each decoded B fragment
+    // against more registers (8 -> 1 wave per SIMD, 4 -> 2).  Measured with rank
+    // 4: N = 512 runs fastest at 4, N = 1024 and 2048 at 8.
     if (P.nmt > 4 && N <= 512) P.nmt = 4;
     if (P.nmt > 8) P.nmt = 8;
     // SSEQS_CORR_MT caps it further (tuning knob; results do not depend on it)
@@ -1848,8 +1849,8 @@ extern "C" int sseqs_db_prefilter(const uint8_t* packed, const int64_t* seq_off,
 }
 
 // Spans that may hold '@' inside them (the shifted segments of the per-batch
-// cascade): the generic kernels only, whose table gives '@' the value of
-// code 21 like the ASCII operator, while the band kernel's symbol 0 masks.
+// cascade): the ring and dense kernels only, whose tables give '@' the value
+// of code 21 like the ASCII operator, while the band kernel's symbol 0 masks.
 extern "C" int sseqs_db_prefilter_spans(const uint8_t* packed, const int64_t* seq_off,
                                         const int32_t* seq_len, int64_t s_begin, int64_t s_end,
                                         const uint8_t* qrev, int query_len, const float* lutA,

@@ -298,8 +298,8 @@ class MultiSearch:
         """Gather + backtrack of every query's hits.  With several queries
         the queries alternate over BT_STREAMS streams forked from and joined
         back to the current stream, each with its own workspace: one
-        query's launch holds four waves per SIMD, and its longest hits are
-        its tail, so two queries in flight fill the GPU better."""
+        query's launch of 4096 hits is sixteen waves per CU, and its longest
+        hits are its tail, so two queries in flight fill the GPU better."""
         if not self.backtrack:
             return
         from .search import backtrack_hits

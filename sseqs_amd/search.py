@@ -369,8 +369,8 @@ def _resident_batches(db: SeqDB, query: str, q: PreparedQuery, plan, top_fft: in
     fb = np.nonzero(fast)[0]
 
     # prefilter: one launch per run of consecutive batches with one N and one
-    # kind; a shifted batch's spans may hold '@', which the generic kernels
-    # score like the reference's ASCII operator
+    # kind; a shifted batch's spans may hold '@', which the ring and dense
+    # kernels score like the reference's ASCII operator
     t0 = time.time()
     sc32 = torch.empty(plan.seg_off.numel(), dtype=torch.float32, device=dev)
     # each batch's segments in length order when the plan has one (same
